@@ -230,9 +230,8 @@ void og_launch_zero_acc(long long* facc, long long* iacc, int n_atoms, hipStream
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) og_k_back(og_back_args a) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= a.n_atoms) return;
     if (i == 0 && a.do_kick && a.step_dev) *a.step_dev += 1u;
-    back_atom(a, i);
+    back_wave(a, i, a.n_atoms);
 }
 
 __global__ void __launch_bounds__(256) og_k_zero_i64(long long* p, long long n) {

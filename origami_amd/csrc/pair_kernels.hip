@@ -955,7 +955,7 @@ __global__ void __launch_bounds__(OG_PERSIST_THREADS) og_k_replica_steps(og_pair
         __syncthreads();
         og_back_args b = bk;
         b.ke_acc = pp.ke_acc ? pp.ke_acc + (size_t)k * pp.n_sys : nullptr;
-        for (int i = a0 + tid; i < a1; i += NT) back_atom(b, i);
+        for (int i0 = a0; i0 < a1; i0 += NT) back_wave(b, i0 + tid, a1);
         __syncthreads();
     }
 }
