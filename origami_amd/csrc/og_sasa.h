@@ -15,7 +15,7 @@ struct og_sasa_data {
     int n_work = 0;               // atoms with gamma != 0
     int n_cu = 0;
     int blocks = 0;               // launch width of the arrangement kernel
-    bool one_pass = false;        // arrangement in one pass of MAXC caps (no second pass)
+    bool blocks_set = false;      // blocks chosen by the caller or the autotuner
     int passes = 0;               // 0: one pass when the blocks fit its LDS; 1 or 2: forced
     long long lds_cu = 0;         // LDS bytes per CU
     int stride = 0;               // waves launched (= per-wave staging slots)

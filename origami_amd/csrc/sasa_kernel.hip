@@ -56,6 +56,8 @@
 #define SA_COV_CAPS (SA_TMAX / 6)     // union cover test: circles per batch (bases in ta)
 #define SA_COV_PAIRS (3 * SA_TMAX)    // union cover test: arcs per batch (in tx..tz)
 #define SA_COV_EPS 1e-5f              // cover margin on angles (rad)
+#define SA_FORCE_BLOCKS_CU 3          // default arrangement blocks per CU beside the pair kernels
+#define SA_ONE_EACH_CU 4              // up to so many where every atom then has its own wave
 #define SA_QUEUES 8                   // arrangement work queues (one per XCD)
 #define SA_QSTRIDE 64                 // ints between queue counters (256 bytes)
 #define SA_NCOUNTERS (SA_QSTRIDE * (SA_QUEUES + 1))
@@ -1412,7 +1414,6 @@ int og_sasa_build(og_sasa_data* d, int n_atoms, const std::vector<int>& atom_sys
     blocks = std::min(blocks, d->n_cu * 8);   // staging for up to 8 blocks per CU (autotuner range)
     d->blocks = std::max(blocks, 1);
     d->stride = d->blocks * SA_WAVES;
-    og_sasa_set_blocks(d, d->blocks);
     // pool capacity: OG_SASA_POOL_ARCS arcs and vertices per SASA atom on average
     const long long per = OG_SASA_POOL_ARCS;
     d->arc_cap = (int)std::min<long long>(per * std::max(d->n_work, 1), 1ll << 30);
@@ -1609,19 +1610,35 @@ int og_sasa_launch(og_sasa_data* d, const double* pos, long long* facc, double g
     d->sflag = sflag;
     hipLaunchKernelGGL(og_k_tile_bounds, dim3(d->n_tiles > 0 ? d->n_tiles : 1), dim3(64), 0, s, pos,
                        d->tile_atom0, d->tile_cnt, d->n_tiles, d->tile_bound, d->counters);
+    // Until a width is chosen, a force evaluation takes at most
+    // SA_FORCE_BLOCKS_CU blocks per CU, so that the pair kernels beside it
+    // find room: a grid that fills the CUs (8 blocks) keeps them waiting until
+    // the arrangement ends.  Measured per step on 64 chains with 51 918 SASA
+    // atoms: 4.2, 2.35, 1.84, 1.99, 2.3 and 2.24 ms at 1 to 5 and 8 blocks per
+    // CU; on 4 chains with 3 493 atoms 0.27 ms at 3 against 0.30 at 8.  Up to
+    // SA_ONE_EACH_CU blocks per CU are launched where that gives every atom a
+    // wave of its own (one chain with 1 666 atoms: 0.383 ms per force call at
+    // 4, 0.397 at 3, where some waves take a second atom).  Areas (energies) have little beside them and take the full width (16 chains,
+    // 12 011 atoms: 1.01 ms at 6 to 8 blocks, 1.23 at 3).
+    const int own_wave = (d->n_work + SA_WAVES - 1) / SA_WAVES;
+    const int width = own_wave <= SA_ONE_EACH_CU * d->n_cu ? own_wave : SA_FORCE_BLOCKS_CU * d->n_cu;
+    const int blocks = d->blocks_set || area ? d->blocks : std::min(d->blocks, width);
     // One pass with MAXC caps when the grid fits its LDS; otherwise the
     // SA_NC_MAIN pass and the second pass over the atoms it deferred (usually
     // few or none), one block per CU.
-    const int blocks2 = d->blocks < d->n_cu ? d->blocks : d->n_cu;
+    const long long per_block = (long long)SA_WAVES * sizeof(ArrLds<MAXC>);
+    const bool one_pass = d->passes == 1 ||
+                          (d->passes == 0 && (long long)blocks <= (long long)d->n_cu * (d->lds_cu / per_block));
+    const int blocks2 = blocks < d->n_cu ? blocks : d->n_cu;
     const dim3 blk(64 * SA_WAVES);
-    if (d->one_pass) {
-        if (area) hipLaunchKernelGGL((og_k_sasa_arrange<true, MAXC, false>), dim3(d->blocks), blk, 0, s, *d, pos);
-        else hipLaunchKernelGGL((og_k_sasa_arrange<false, MAXC, false>), dim3(d->blocks), blk, 0, s, *d, pos);
+    if (one_pass) {
+        if (area) hipLaunchKernelGGL((og_k_sasa_arrange<true, MAXC, false>), dim3(blocks), blk, 0, s, *d, pos);
+        else hipLaunchKernelGGL((og_k_sasa_arrange<false, MAXC, false>), dim3(blocks), blk, 0, s, *d, pos);
     } else if (area) {
-        hipLaunchKernelGGL((og_k_sasa_arrange<true, SA_NC_MAIN, false>), dim3(d->blocks), blk, 0, s, *d, pos);
+        hipLaunchKernelGGL((og_k_sasa_arrange<true, SA_NC_MAIN, false>), dim3(blocks), blk, 0, s, *d, pos);
         hipLaunchKernelGGL((og_k_sasa_arrange<true, MAXC, true>), dim3(blocks2), blk, 0, s, *d, pos);
     } else {
-        hipLaunchKernelGGL((og_k_sasa_arrange<false, SA_NC_MAIN, false>), dim3(d->blocks), blk, 0, s, *d, pos);
+        hipLaunchKernelGGL((og_k_sasa_arrange<false, SA_NC_MAIN, false>), dim3(blocks), blk, 0, s, *d, pos);
         hipLaunchKernelGGL((og_k_sasa_arrange<false, MAXC, true>), dim3(blocks2), blk, 0, s, *d, pos);
     }
     if (gamma_scale != 0.0) {                 // forces (not only areas)
@@ -1641,15 +1658,10 @@ int og_sasa_max_blocks(const og_sasa_data* d) { return d->stride / SA_WAVES; }
 void og_sasa_set_blocks(og_sasa_data* d, int blocks) {
     const int mx = d->stride / SA_WAVES;
     d->blocks = blocks < 1 ? 1 : (blocks > mx ? mx : blocks);
-    const long long per_block = (long long)SA_WAVES * sizeof(ArrLds<MAXC>);
-    d->one_pass = d->passes == 1 ||
-                  (d->passes == 0 && (long long)d->blocks <= (long long)d->n_cu * (d->lds_cu / per_block));
+    d->blocks_set = true;
 }
 
-void og_sasa_set_passes(og_sasa_data* d, int passes) {
-    d->passes = passes;
-    og_sasa_set_blocks(d, d->blocks);
-}
+void og_sasa_set_passes(og_sasa_data* d, int passes) { d->passes = passes; }
 
 int og_sasa_overflow(og_sasa_data* d, int* count) {
     if (hipMemcpy(count, d->overflow, sizeof(int), hipMemcpyDeviceToHost) != hipSuccess) return -2;
