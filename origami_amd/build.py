@@ -15,7 +15,7 @@ CSRC = os.path.join(HERE, "csrc")
 OUT_DIR = os.path.join(HERE, "_lib")
 LIB = os.path.join(OUT_DIR, "liborigami_gpu.so")
 
-SOURCES = ["engine.cpp", "pair_kernels.hip", "md_kernels.hip", "sasa_kernel.hip", "sasa_terms.hip",
+SOURCES = ["engine.cpp", "pair_kernels.hip", "pair_wide.hip", "md_kernels.hip", "sasa_kernel.hip", "sasa_terms.hip",
            "surrogate.hip", "lbfgs.hip"]
 
 # Per-file additions.  The SASA JVP terms take one-hot tangents whose zero

@@ -882,8 +882,12 @@ static int launch_forces(og_engine* e, uint32_t flags, double cutoff_a, double s
     og_sur* sur = (flags & OG_SURROGATE) ? e->sur : nullptr;
     // Small batches (the LDS gather's range): the bonded terms share one
     // launch with the descreening pass, the bonded gather one with the Born
-    // radii after it.
-    const bool fuse = !energy && !sur && !e->prof && e->n_atoms < OG_GATHER_LDS_MAX_ATOMS;
+    // radii after it, or, on short work lists (a block per work item,
+    // pair_wide.hip), with the force pass, which forms the radii itself.
+    const bool lean = !energy && !sur && !e->prof;
+    const bool wide = lean && forces && e->n_tile_pairs <= OG_WIDE_FORCE_MAX;
+    const bool wide_d = wide && e->n_work <= OG_WIDE_DESCREEN_MAX;
+    const bool fuse = wide || (lean && e->n_atoms < OG_GATHER_LDS_MAX_ATOMS);
     og_bonded_args b{};
     {
         ProfScope p(e, OG_K_BONDED);
@@ -920,7 +924,8 @@ static int launch_forces(og_engine* e, uint32_t flags, double cutoff_a, double s
         ProfScope p(e, OG_K_DESCREEN);
         og_pair_args ad = a;
         ad.skip_sys = (sur && !check) ? sur->mode : (!forces ? e->eval_skip : nullptr);
-        if (fuse) og_launch_descreen_bonded(ad, b, mode_a, e->stream);
+        if (wide_d) og_launch_wide_descreen(ad, b, mode_a, e->stream);
+        else if (fuse) og_launch_descreen_bonded(ad, b, mode_a, e->stream);
         else og_launch_pair_descreen(ad, mode_a, e->stream);
     }
     {
@@ -931,14 +936,15 @@ static int launch_forces(og_engine* e, uint32_t flags, double cutoff_a, double s
         r.eacc = e->eacc; r.n_atoms = e->n_atoms;
         r.sflag = e->sflag;
         if (sur) { r.sur_mode = sur->mode; r.r_sur = sur->r_sur; r.dev = sur->dev; r.check = check ? 1 : 0; }
-        if (fuse) og_launch_radii_gather(r, b, e->stream);
+        if (wide) og_launch_wide_force(a, r, b, mode_a, e->stream);
+        else if (fuse) og_launch_radii_gather(r, b, e->stream);
         else og_launch_radii(r, energy, e->stream);
         if (sur && check && og_sur_check_apply(sur)) {
             if (fork) (void)hipStreamWaitEvent(e->stream, e->join_ev, 0);
             return fail(OG_ERR_HIP, "surrogate launch failed: %s", og_sur_error());
         }
     }
-    if (forces) {
+    if (forces && !wide) {
         ProfScope p(e, OG_K_FORCE);
         og_launch_pair_force(a, mode_a, e->stream);
     }

@@ -86,6 +86,21 @@ __device__ __forceinline__ void noise_atom_at(const og_noise_args& a, int i, uin
 // ---------------------------------------------------------------------------
 // Born radii from the descreening integral (gb.rs:327-341), GB self energy.
 // ---------------------------------------------------------------------------
+// Effective radius of an atom from its descreening integral; clamped: the
+// transform left the valid range and the floor stands in.
+__device__ __forceinline__ double born_radius(double integral, double rho, bool& clamped) {
+    const double rt = rho - OG_OBC_OFFSET;
+    const double psi = integral * rt;
+    const double arg = 1.0 * psi - 0.8 * psi * psi + 4.85 * psi * psi * psi;
+    const double inv = 1.0 / rt - tanh(arg) / rho;
+    const double floor_r = rt > 0.5 ? rt : 0.5;
+    clamped = inv <= 0.0 || !isfinite(inv);
+    if (clamped) return floor_r;
+    const double R = 1.0 / inv;
+    return R > floor_r ? R : floor_r;
+}
+constexpr double kGbWidth = 0.60056120439322491;   // sqrt(log2(e) / 4): gw = kGbWidth / R
+
 template <bool ENERGY>
 __device__ __forceinline__ void radii_body(const og_radii_args& a, int i) {
     int sys = 0;
@@ -97,20 +112,11 @@ __device__ __forceinline__ void radii_body(const og_radii_args& a, int i) {
         double R = 0.0;
         if (!sur || a.check) {
             const double rho = a.rho[i];
-            const double rt = rho - OG_OBC_OFFSET;
             const double integral =
                 (double)__hip_atomic_load(a.iacc + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) * OG_FIX_INV;
-            const double psi = integral * rt;
-            const double arg = 1.0 * psi - 0.8 * psi * psi + 4.85 * psi * psi * psi;
-            const double inv = 1.0 / rt - tanh(arg) / rho;
-            const double floor_r = rt > 0.5 ? rt : 0.5;
-            if (inv <= 0.0 || !isfinite(inv)) {
-                if (!sur) atomicAdd(a.clamped + sys, 1);
-                R = floor_r;
-            } else {
-                R = 1.0 / inv;
-                R = R > floor_r ? R : floor_r;
-            }
+            bool clamped;
+            R = born_radius(integral, rho, clamped);
+            if (clamped && !sur) atomicAdd(a.clamped + sys, 1);
         }
         if (sur) {
             const double Rs = a.r_sur[i];
@@ -123,7 +129,7 @@ __device__ __forceinline__ void radii_body(const og_radii_args& a, int i) {
         a.radii[i] = R;
         float4 g = a.gb[a.atom_slot[i]];
         g.z = (float)R;
-        g.w = (float)(0.60056120439322491 / R);  // sqrt(log2(e)/4) / R
+        g.w = (float)(kGbWidth / R);
         a.gb[a.atom_slot[i]] = g;
         if (ENERGY) {
             const double q = a.charge[i];
@@ -307,6 +313,77 @@ __device__ __forceinline__ void gather_atom(const og_bonded_args& a, int i) {
     og_atomic_add_fix(a.facc + 3 * (size_t)i + 0, og_to_fix_chk(fx, fl));
     og_atomic_add_fix(a.facc + 3 * (size_t)i + 1, og_to_fix_chk(fy, fl));
     og_atomic_add_fix(a.facc + 3 * (size_t)i + 2, og_to_fix_chk(fz, fl));
+}
+
+// Per atom: sum its (term, atom) force slots in slot order (bonds, angles,
+// dihedrals, impropers, each in list order, as origami's term loops add
+// them) in FP64, then one fixed-point add per component.  A block takes 64
+// consecutive atoms, whose slots are one contiguous CSR range: all its
+// threads first copy the slot forces of that range into LDS (independent
+// loads, all in flight together, where a thread walking its own atom's
+// slots would wait on each one), then wave 0 sums each atom's slots from
+// LDS in slot order.  Ranges longer than the LDS copy go in chunks.
+// NOISE: wave 1 meanwhile forms the block's atoms' O-step normals for the
+// next step.
+#define OG_GATHER_ATOMS 64
+#define OG_GATHER_CHUNK 2048
+// NT: threads of the block; s_t: its LDS, 3 OG_GATHER_CHUNK doubles.
+template <bool NOISE, int NT>
+__device__ __forceinline__ void gather_lds_body(const og_bonded_args& a, int blk, double* s_t) {
+    constexpr int U = OG_GATHER_CHUNK / NT;
+    const int a0 = blk * OG_GATHER_ATOMS;
+    const int a1 = min(a0 + OG_GATHER_ATOMS, a.n_atoms);
+    const int t = threadIdx.x;
+    const int i = a0 + t;
+    const bool own = t < OG_GATHER_ATOMS && i < a1;
+    const int q_begin = a.csr_start[a0], q_end = a.csr_start[a1];
+    int q = own ? a.csr_start[i] : 0;
+    const int qe = own ? a.csr_start[i + 1] : 0;
+    double fx = 0.0, fy = 0.0, fz = 0.0;
+    for (int c0 = q_begin; c0 < q_end; c0 += OG_GATHER_CHUNK) {
+        const int c1 = min(c0 + OG_GATHER_CHUNK, q_end);
+        __syncthreads();                                  // the previous chunk is summed
+        // U entries per thread, every load issued before the first LDS store
+        size_t sl[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = c0 + t + NT * u;
+            sl[u] = k < c1 ? 3 * (size_t)a.csr_slot[k] : 0;
+        }
+        double v[3 * U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (c0 + t + NT * u < c1) {
+                v[3 * u] = a.tf[sl[u]];
+                v[3 * u + 1] = a.tf[sl[u] + 1];
+                v[3 * u + 2] = a.tf[sl[u] + 2];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int e = t + NT * u;
+            if (c0 + e < c1) {
+                s_t[3 * e] = v[3 * u];
+                s_t[3 * e + 1] = v[3 * u + 1];
+                s_t[3 * e + 2] = v[3 * u + 2];
+            }
+        }
+        __syncthreads();
+        for (; q < qe && q < c1; ++q) {
+            const double* d = s_t + 3 * (q - c0);
+            fx += d[0];
+            fy += d[1];
+            fz += d[2];
+        }
+    }
+    if (NOISE && t >= OG_GATHER_ATOMS && t < 2 * OG_GATHER_ATOMS && a0 + t - OG_GATHER_ATOMS < a1)
+        noise_atom(a.noise, a0 + t - OG_GATHER_ATOMS);
+    if (own) {
+        int* fl = a.sflag ? a.sflag + a.atom_sys[i] : nullptr;
+        og_atomic_add_fix(a.facc + 3 * (size_t)i + 0, og_to_fix_chk(fx, fl));
+        og_atomic_add_fix(a.facc + 3 * (size_t)i + 1, og_to_fix_chk(fy, fl));
+        og_atomic_add_fix(a.facc + 3 * (size_t)i + 2, og_to_fix_chk(fz, fl));
+    }
 }
 
 // Atom i: fixed point -> FP64 force; with do_kick the closing half-kick,

@@ -170,6 +170,21 @@ void og_launch_bonded(const og_bonded_args& a, bool energy, hipStream_t s);
 void og_launch_descreen_bonded(const og_pair_args& a, const og_bonded_args& b, bool mode_a, hipStream_t s);
 // the bonded terms alone (forces), the gather left to og_launch_radii_gather
 void og_launch_bonded_terms(const og_bonded_args& a, hipStream_t s);
+// Short work lists (pair_wide.hip): a block per work item.  The wide force
+// launch takes the place of the radii + gather and force launches of a force
+// evaluation (forces only, no surrogate), the wide descreening launch that of
+// the descreening + bonded launch.  Where the lines lie (us per step, one wave
+// per item -> a block per item):
+//   force, up to 19 tile pairs per CU: 33 -> 25 at 6 tile pairs, 82 -> 54 at
+//   210, 83 -> 55 at 861, 100 -> 91 at 4 274; 103 -> 108 at 6 007, where the
+//   one-wave items fill the chip and the block form's LDS traffic costs more
+//   descreening, up to 2 items per CU: 69 -> 63 at 21 items, 82 -> 78 at 210,
+//   83 -> 81 at 496; 83 -> 86 at 861
+#define OG_WIDE_FORCE_MAX 4864
+#define OG_WIDE_DESCREEN_MAX 512
+void og_launch_wide_descreen(const og_pair_args& a, const og_bonded_args& b, bool mode_a, hipStream_t s);
+void og_launch_wide_force(const og_pair_args& a, const og_radii_args& r, const og_bonded_args& b, bool mode_a,
+                          hipStream_t s);
 // Born radii (forces only, no surrogate) and the bonded gather's LDS form
 // in one launch; batches below 20 000 atoms
 void og_launch_radii_gather(const og_radii_args& r, const og_bonded_args& b, hipStream_t s);

@@ -1,0 +1,268 @@
+// Per-pair arithmetic and tile loads of the all-pairs kernels, shared by the
+// wave-per-item kernels (pair_kernels.hip) and the block-per-item kernels for
+// small work lists (pair_wide.hip).  Both forms evaluate a pair with the same
+// products in the same order, so their results agree bit for bit.
+//
+//   descreening   energy/src/gb.rs:271-283 (pair), :347-369 (h)
+//   LJ + Coulomb  energy/src/forces_nonbonded.rs:196-232
+//   GB pair force energy/src/forces_gb.rs:72-112
+#pragma once
+#include "og_device.h"
+#include "og_kernels.h"
+
+namespace {
+
+constexpr float kGbK = (float)(1.0 - 1.0 / OG_EPS_WATER);
+constexpr float kHalfLn2 = 0.34657359027997264f;
+
+struct LaneData {
+    float x, y, z, q;
+    float4 par;   // se, rm, se14, rm14
+    float4 gb;    // rho~, S, R, invRq
+};
+
+__device__ __forceinline__ LaneData load_lane(const og_pair_args& a, int tile, int atom0, int cnt,
+                                              int lane, double ox, double oy, double oz) {
+    LaneData d;
+    const int slot = tile * OG_TILE + lane;
+    if (lane < cnt) {
+        const double* p = a.pos + 3 * (size_t)(atom0 + lane);
+        d.x = (float)(p[0] - ox);
+        d.y = (float)(p[1] - oy);
+        d.z = (float)(p[2] - oz);
+    } else {
+        // Padding slot: far away and (via zero parameters) inert.
+        d.x = 1.0e6f + 97.0f * (float)lane;
+        d.y = 1.0e6f;
+        d.z = 1.0e6f;
+    }
+    d.q = a.qs[slot];
+    d.par = a.par[slot];
+    d.gb = a.gb[slot];
+    return d;
+}
+
+__device__ __forceinline__ float rl(float v, int j) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j));
+}
+
+// one-lane rotation of a value around the wave (DPP wave_rol:1)
+// (mov_dpp: every lane is written, so no "old" value has to be materialised)
+__device__ __forceinline__ float rot(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x134, 0xF, 0xF, false));
+}
+__device__ __forceinline__ int roti(int v) { return __builtin_amdgcn_mov_dpp(v, 0x134, 0xF, 0xF, false); }
+// exchange with the lane 32 away (halves of the wave)
+__device__ __forceinline__ float swap32(float v) { return __shfl_xor(v, 32, 64); }
+
+// Descreening integral term h(r, rho~_i, S_j) of energy/src/gb.rs:347-369,
+// written with one reciprocal and one log:  1/L - 1/U = (U-L)/(LU),
+// 1/U^2 - 1/L^2 = -(1/L - 1/U)(U+L)/(LU),  ln(L/U) = ln(L^2/(LU)), with
+// L = max(r - S, rho~) covering both the overlapping and the separate case.
+__device__ __forceinline__ float descreen_h(float r2, float inv_r, float rt, float S, float S2) {
+    // r = r2 * inv_r is not rounded on its own (left to the compiler, some
+    // loops did and some did not)
+    const float U = fmaf(r2, inv_r, S);
+    const float L = fmaxf(fmaf(r2, inv_r, -S), rt);
+    const float UmL = U - L;
+    const float UpL = U + L;
+    const float w = __builtin_amdgcn_rcpf(L * U);
+    const float t = UmL * w;
+    const float s2q = S2 * (0.25f * inv_r);
+    const float lg = __builtin_amdgcn_logf(L * L * w);   // log2
+    float h = fmaf(0.5f, t, -(t * UpL * w) * s2q);
+    h = fmaf(lg, kHalfLn2 * inv_r, h);
+    return (U <= rt) ? 0.0f : h;
+}
+
+// Orders a wave's own LDS accesses across lanes for the compiler; a wave's
+// LDS operations are performed in program order, so no wait is needed.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Far-field form of descreen_tile_lds for tile pairs whose atoms are all at
+// least og_pair_args::ds_far apart: there S / r <= 0.1 and L = r - S, and
+// the HCT term (1/r)[x/(1-x^2) - x^3/(1-x^2)^2 - atanh x], x = S/r, is the
+// series (1/r) sum_n c_n x^(2n+1), c_n = 1 - n - 1/(2n+1):
+//   h = -(S^3 / (3 r^4)) (1 + 3.6 y + (45/7) y^2 + (28/3) y^3),  y = x^2,
+// whose next term, (135/11) y^4 relative, is below 1.3e-7 at x = 0.1 (FP32
+// rounding is 6e-8); the closed form evaluated in FP32 there loses about
+// 6e-8 / x^2 to cancellation.  Every term is negative, as h is.  Q[e].z holds
+// -S^3/3 of j atom e.
+template <bool MODEA, int PART>
+__device__ __forceinline__ void descreen_tile_far(const og_pair_args& a, const LaneData& di,
+                                                  const float4* P, const float4* Q, int lane,
+                                                  float& acc_i, float& acc_j) {
+    float gj = 0.0f;
+    const float Si2 = di.gb.y * di.gb.y;
+    const float ci3 = (-1.0f / 3.0f) * Si2 * di.gb.y;
+    auto series = [](float y) { return fmaf(y, fmaf(y, fmaf(y, 28.0f / 3.0f, 45.0f / 7.0f), 3.6f), 1.0f); };
+    auto step = [&](float4 pj, float4 qj) {
+        const float dx = pj.x - di.x, dy = pj.y - di.y, dz = pj.z - di.z;
+        const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+        const float inv_r = __builtin_amdgcn_rsqf(r2);
+        const float inv_r2 = inv_r * inv_r;
+        const float inv_r4 = inv_r2 * inv_r2;
+        const float hij = (qj.z * inv_r4) * series(qj.y * inv_r2);
+        const float hji = (ci3 * inv_r4) * series(Si2 * inv_r2);
+        if (MODEA) {
+            const bool ok = r2 <= a.rc2_ds;
+            acc_i += ok ? hij : 0.0f;
+            gj += ok ? hji : 0.0f;
+        } else {
+            acc_i += hij;
+            gj += hji;
+        }
+        gj = rot(gj);                  // after step 63 this is the way home
+    };
+    constexpr int kb = PART == 1 ? 32 : 0, ke = PART == 0 ? 32 : 64;
+    for (int k = kb; k < ke; k += 2) {
+        const int idx = (lane + k) & 63;
+        const float4 p0 = P[idx], p1 = P[idx + 1];
+        const float4 q0 = Q[idx], q1 = Q[idx + 1];
+        step(p0, q0);
+        step(p1, q1);
+    }
+    if (PART == 0) gj = swap32(gj);
+    acc_j += gj;
+}
+
+__device__ __forceinline__ float wave_max_f(float v) {
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+    return v;
+}
+
+// Far tile pair of the descreening pass: the distance of the two first atoms
+// less the radii of both tiles about them (positions are relative to the i
+// tile's first atom, so lane 0's i position is the origin) bounds every pair's
+// distance from below; 1e-3 A covers the FP32 rounding.
+__device__ __forceinline__ bool descreen_far(const og_pair_args& a, const LaneData& di, const LaneData& dj, int ci,
+                                             int cj, int lane) {
+    const float jx0 = rl(dj.x, 0), jy0 = rl(dj.y, 0), jz0 = rl(dj.z, 0);
+    const float ri = lane < ci ? sqrtf(fmaf(di.x, di.x, fmaf(di.y, di.y, di.z * di.z))) : 0.0f;
+    const float ex = dj.x - jx0, ey = dj.y - jy0, ez = dj.z - jz0;
+    const float rj = lane < cj ? sqrtf(fmaf(ex, ex, fmaf(ey, ey, ez * ez))) : 0.0f;
+    const float d0 = sqrtf(fmaf(jx0, jx0, fmaf(jy0, jy0, jz0 * jz0)));
+    return a.ds_far > 0.0f && d0 - wave_max_f(ri) - wave_max_f(rj) - 1e-3f >= a.ds_far;
+}
+
+// Pair coefficient c (force on i = c * d, d = x_j - x_i) of a tile pair's
+// fused LJ + Coulomb + GB-pair force.  MASKED: excl drops the LJ and Coulomb
+// terms, one4 selects the 1-4 parameters.
+template <bool MODEA, bool MASKED>
+__device__ __forceinline__ float tile_coef(const og_pair_args& a, const LaneData& di, float qki, float qj, float sej,
+                                           float rmj, float se14j, float rm14j, float Rj, float iRj, bool excl,
+                                           bool one4, float dx, float dy, float dz) {
+    const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+    const float inv_r = __builtin_amdgcn_rsqf(r2);
+    const float inv_r2 = inv_r * inv_r;
+    float rmin, eij;
+    if (MASKED) {
+        rmin = one4 ? di.par.w + rm14j : di.par.y + rmj;
+        eij = one4 ? di.par.z * se14j : di.par.x * sej;
+    } else {
+        rmin = di.par.y + rmj;
+        eij = di.par.x * sej;
+    }
+    const float t2 = rmin * rmin * inv_r2;
+    const float t6 = t2 * t2 * t2;
+    const float lj = eij * inv_r2 * (t6 - t6 * t6);
+    const float qq = di.q * qj;
+    float coul;
+    if (MODEA) coul = -qq * (inv_r2 * inv_r - a.inv_rc3);
+    else coul = -qq * inv_r2 * inv_r;
+    float cnb = lj + coul;
+    if (MODEA) cnb = (r2 <= a.rc2_nb) ? cnb : 0.0f;
+    if (MASKED) cnb = excl ? 0.0f : cnb;
+    // GB pair (frozen radii): f^2 = r^2 + R_i R_j exp(-r^2 / (4 R_i R_j))
+    const float Rp = di.gb.z * Rj;
+    const float e = __builtin_amdgcn_exp2f(-r2 * (di.gb.w * iRj));
+    const float f2 = fmaf(Rp, e, r2);
+    const float inv_f = __builtin_amdgcn_rsqf(f2);
+    const float qgb = qki * qj;
+    float gbc = qgb * fmaf(-0.25f, e, 1.0f) * (inv_f * inv_f * inv_f);
+    if (MODEA) gbc = (r2 <= a.rc2_gb) ? gbc : 0.0f;
+    const float c = cnb + gbc;
+    return r2 >= 1e-18f ? c : 0.0f;
+}
+
+// One i atom of a strip: position relative to the strip's origin, charge,
+// LJ and GB parameters, and its force sum over the strip.
+struct StripAtom {
+    float x, y, z, q;
+    float se, rm, R, gw;
+    float fx, fy, fz;
+};
+
+__device__ __forceinline__ StripAtom strip_atom(const LaneData& d) {
+    return {d.x, d.y, d.z, d.q, d.par.x, d.par.y, d.gb.z, d.gb.w, 0.0f, 0.0f, 0.0f};
+}
+
+// Pair coefficient c (force on i = c * d, d = x_j - x_i) of the fused
+// LJ + Coulomb + GB-pair force for an unmasked pair; j data as in the LDS
+// layout of force_tile_lds (P = x, y, z, q; Q = se, rm, R, 1/R scaled).
+// Mode B groups the two charge terms: q_i q_j (k_GB (1 - e/4) / f^3 - 1/r^3).
+// FAR: every pair of the j tile has r^2 gw_i gw_j >= 32 (gw = sqrt(log2 e / 4)
+// / R), so e = exp2(-r^2 gw_i gw_j) <= 2^-32.  Then R_i R_j e is below 1e-11
+// r^2 (r^2 = 4 R_i R_j x, x = r^2 gw_i gw_j / log2 e >= 22), far under half an
+// FP32 ulp of r^2, so f^2 = fma(R_i R_j, e, r^2) rounds to r^2 and 1/f is the
+// 1/r above; likewise k (1 - e/4) rounds to k.  The exponential and the
+// second square root are left out, with the same products in the same order:
+// the coefficient is bit-identical.
+template <bool MODEA, bool FAR = false>
+__device__ __forceinline__ float strip_coef(const og_pair_args& a, const StripAtom& I, float4 pj, float4 qj,
+                                            float dx, float dy, float dz) {
+    const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+    const float inv_r = __builtin_amdgcn_rsqf(r2);
+    const float inv_r2 = inv_r * inv_r;
+    const float rmin = I.rm + qj.y;
+    const float t2 = rmin * rmin * inv_r2;
+    const float t6 = t2 * t2 * t2;
+    const float lj = (I.se * qj.x) * inv_r2 * fmaf(-t6, t6, t6);
+    const float qq = I.q * pj.w;
+    float gb;
+    if (FAR) {
+        gb = kGbK * (inv_r * inv_r * inv_r);
+    } else {
+        const float e = __builtin_amdgcn_exp2f(-r2 * (I.gw * qj.w));
+        const float f2 = fmaf(I.R * qj.z, e, r2);
+        const float inv_f = __builtin_amdgcn_rsqf(f2);
+        gb = fmaf(-0.25f * kGbK, e, kGbK) * (inv_f * inv_f * inv_f);
+    }
+    if (MODEA) {
+        float cnb = fmaf(-qq, inv_r2 * inv_r - a.inv_rc3, lj);
+        cnb = (r2 <= a.rc2_nb) ? cnb : 0.0f;
+        const float gbc = (r2 <= a.rc2_gb) ? qq * gb : 0.0f;
+        return cnb + gbc;
+    }
+    return fmaf(qq, gb - inv_r2 * inv_r, lj);
+}
+
+// Bounds of a strip's two i tiles about the origin (the first one's first
+// atom; both tiles are full) and their smallest gw, for the far test.
+struct StripBound {
+    float rad, gw;
+};
+
+__device__ __forceinline__ StripBound strip_bound(const StripAtom& A, const StripAtom& B) {
+    return {wave_max_f(fmaxf(sqrtf(fmaf(A.x, A.x, fmaf(A.y, A.y, A.z * A.z))),
+                             sqrtf(fmaf(B.x, B.x, fmaf(B.y, B.y, B.z * B.z))))),
+            -wave_max_f(-fminf(A.gw, B.gw))};
+}
+
+// Far j tile: the smallest pair distance (distance of the first atoms less
+// both tiles' radii, 1e-3 A for FP32 rounding) gives r^2 gw_i gw_j >= 33 for
+// every pair (padding slots excluded).
+__device__ __forceinline__ bool strip_far(const StripBound& b, const LaneData& dj, int cj, int lane) {
+    const float jx0 = rl(dj.x, 0), jy0 = rl(dj.y, 0), jz0 = rl(dj.z, 0);
+    const float ex = dj.x - jx0, ey = dj.y - jy0, ez = dj.z - jz0;
+    const float rad_j = wave_max_f(lane < cj ? sqrtf(fmaf(ex, ex, fmaf(ey, ey, ez * ez))) : 0.0f);
+    const float gw_j = -wave_max_f(lane < cj ? -dj.gb.w : -1.0e30f);
+    const float rmn = sqrtf(fmaf(jx0, jx0, fmaf(jy0, jy0, jz0 * jz0))) - b.rad - rad_j - 1e-3f;
+    return rmn > 0.0f && rmn * rmn * (b.gw * gw_j) >= 33.0f;
+}
+
+}  // namespace

@@ -34,3 +34,44 @@ def test_recorded_kinetic_energy_of_systems_sharing_waves(E, lengths):
     again.dynamics_setup([300.0] * len(systems), dt_fs=0.01, friction_ps_inv=1.0, seed=3)
     again.run(3)
     assert np.array_equal(again.velocities(), eng.velocities())
+
+
+# (seed, residues) of chains whose atom counts end a tile: 63, 64, 65 (one
+# tile and a bit), 256 / 257 (the last split system, the first with strips),
+# 319, 320, 321, 512, 577 and, with strips of more than one group of j tiles,
+# 1 201 atoms
+EDGE_CHAINS = [(16, 4), (21, 4), (3, 3), (9, 15), (13, 16), (14, 19), (22, 18), (28, 19), (14, 30), (26, 33), (2, 70)]
+
+
+@pytest.mark.parametrize("mode_a", [False, True])
+@pytest.mark.parametrize("chains, strip", [([c], 4) for c in EDGE_CHAINS] + [(EDGE_CHAINS, 4), ([(2, 70)], 8),
+                                                                             ([(2, 70)], 5), ([(2, 70)], 1)])
+def test_block_per_item_equals_wave_per_item(E, chains, strip, mode_a):
+    """The block-per-item pair kernels add the same pair terms in the same
+    order as the one-wave kernels (which the profiled path runs): forces,
+    radii and integrals agree bit for bit, and so does a trajectory."""
+    systems = [S.seeded_chain(*c) for c in chains]
+    rng = np.random.default_rng(5)
+    x = np.concatenate([s.pos + rng.normal(scale=0.02, size=s.pos.shape) for s in systems])
+    out = []
+    for profiled in (False, True):
+        eng = E.Engine(systems)
+        eng.strip_tiles(strip)
+        eng.profile(profiled)
+        f = eng.total_force(x, mode_a=mode_a)
+        r, h = eng.born_radii()
+        eng.set_velocities(np.zeros_like(x))
+        eng.dynamics_setup([300.0] * len(systems), dt_fs=0.01, seed=9, mode_a=mode_a)
+        eng.run(3)
+        out.append((f, r, h, eng.positions(), eng.velocities(), eng.status()["clamped"]))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
+def test_block_per_item_forces_against_oracle(E):
+    """Against the FP64 oracle within the engine's force bar (1e-5)."""
+    s = S.seeded_chain(2, 70)
+    x = s.pos + np.random.default_rng(6).normal(scale=0.02, size=s.pos.shape)
+    ref = O.Oracle(s).total_force(x)
+    got = E.Engine([s]).total_force(x)
+    assert np.sqrt(((got - ref) ** 2).sum() / (ref ** 2).sum()) < 1e-5
