@@ -812,7 +812,7 @@ static og_pair_args pair_args(og_engine* e, double cutoff_a) {
     a.pos = e->pos; a.par = e->par; a.gb = e->gb; a.qs = e->qs;
     a.tile_atom0 = e->tile_atom0; a.tile_cnt = e->tile_cnt;
     a.work = e->work; a.n_work = e->n_work; a.masks = e->masks;
-    a.strips = e->strips; a.n_strip = e->n_strip; a.fwork = e->fwork; a.n_fwork = e->n_fwork;
+    a.strips = e->strips; a.n_strip = e->n_strip; a.strip_j = e->strip_j; a.fwork = e->fwork; a.n_fwork = e->n_fwork;
     a.ds_far = e->ds_far;
     a.facc = e->facc; a.iacc = e->iacc; a.eacc = e->eacc;
     a.grid = e->pair_grid;

@@ -30,6 +30,7 @@ struct og_pair_args {
     // tile pairs, and every tile pair of small systems)
     const og_strip* strips;
     int n_strip;
+    int strip_j;                     // j tiles per strip (at most)
     const og_work* fwork;
     int n_fwork;
     // descreening: tile pairs whose atoms are all at least ds_far apart take
@@ -180,6 +181,10 @@ void og_launch_bonded_terms(const og_bonded_args& a, hipStream_t s);
 //   one-wave items fill the chip and the block form's LDS traffic costs more
 //   descreening, up to 2 items per CU: 69 -> 63 at 21 items, 82 -> 78 at 210,
 //   83 -> 81 at 496; 83 -> 86 at 861
+//   strips split into their i sides and j sides (pairs evaluated twice), up
+//   to 4 tile pairs per CU in strips: 41 -> 29 at 21 tile pairs, 49 -> 33 at
+//   210, 54 -> 48 at 861; even at 1 326, 72 -> 90 at 2 850
+#define OG_WIDE_SPLIT_MAX 1024
 #define OG_WIDE_FORCE_MAX 4864
 #define OG_WIDE_DESCREEN_MAX 512
 void og_launch_wide_descreen(const og_pair_args& a, const og_bonded_args& b, bool mode_a, hipStream_t s);

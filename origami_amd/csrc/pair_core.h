@@ -135,6 +135,28 @@ __device__ __forceinline__ float wave_max_f(float v) {
     return v;
 }
 
+// Radius of a tile's atoms (lanes below cnt) about the point (x0, y0, z0).
+__device__ __forceinline__ float tile_radius(const LaneData& d, int cnt, int lane, float x0, float y0, float z0) {
+    const float ex = d.x - x0, ey = d.y - y0, ez = d.z - z0;
+    return wave_max_f(lane < cnt ? sqrtf(fmaf(ex, ex, fmaf(ey, ey, ez * ez))) : 0.0f);
+}
+
+// Every pair of a tile pair lies beyond a cutoff (rc2 its square): the
+// distance of the two first atoms (positions are relative to the i side's
+// origin) less both tiles' radii about them bounds every pair's distance from
+// below; the margin covers the FP32 rounding at any size.  Such a tile pair
+// adds exact zeros under a cutoff and is left out.  A bound that is not finite
+// leaves nothing out.
+__device__ __forceinline__ bool tiles_beyond(float rad_i, const LaneData& dj, int cj, int lane, float rc2) {
+    const float jx0 = rl(dj.x, 0), jy0 = rl(dj.y, 0), jz0 = rl(dj.z, 0);
+    const float rad_j = tile_radius(dj, cj, lane, jx0, jy0, jz0);
+    const float d0 = sqrtf(fmaf(jx0, jx0, fmaf(jy0, jy0, jz0 * jz0)));
+    const float far = d0 - rad_i - rad_j - (1e-3f + 1e-6f * (d0 + rad_i + rad_j));
+    return far > 0.0f && far < 1e15f && far * far > rc2;
+}
+
+__device__ __forceinline__ float force_cutoff2(const og_pair_args& a) { return fmaxf(a.rc2_nb, a.rc2_gb); }
+
 // Far tile pair of the descreening pass: the distance of the two first atoms
 // less the radii of both tiles about them (positions are relative to the i
 // tile's first atom, so lane 0's i position is the origin) bounds every pair's

@@ -115,6 +115,7 @@ __device__ __forceinline__ void descreen_item(const og_pair_args& a, const og_wo
             descreen_tile<MODEA, true>(a, di, di, lane, acc_i, acc_j);
         } else {
             const LaneData dj = load_lane(a, it.tj, a0j, cj, lane, ox, oy, oz);
+            if (MODEA && tiles_beyond(tile_radius(di, ci, lane, 0.0f, 0.0f, 0.0f), dj, cj, lane, a.rc2_ds)) return;
             const float4 pj = make_float4(dj.x, dj.y, dj.z, dj.gb.x);
             const float4 qj = make_float4(dj.gb.y, dj.gb.y * dj.gb.y, (-1.0f / 3.0f) * (dj.gb.y * dj.gb.y) * dj.gb.y,
                                           0.0f);
@@ -309,9 +310,14 @@ __device__ __forceinline__ void force_strip(const og_pair_args& a, const og_stri
         if (lane == 0) { P[OG_TILE] = pjl; Q[OG_TILE] = qjl; }
         wave_lds_order();
         const bool far = strip_far(bi, dj, cj, lane);
+        const bool none = MODEA && tiles_beyond(bi.rad, dj, cj, lane, force_cutoff2(a));
         // the next j tile's data load while this one is evaluated
         const int tn = __builtin_amdgcn_readfirstlane(sp->tj[q + 1 < nj ? q + 1 : q]);
         dj = load_lane(a, tn, a.tile_atom0[tn], a.tile_cnt[tn], lane, ox, oy, oz);
+        if (none) {
+            tj = tn;
+            continue;
+        }
         float gx = 0.0f, gy = 0.0f, gz = 0.0f;
         auto step = [&](float4 pj, float4 qj, auto far_tag) {
             constexpr bool F = decltype(far_tag)::value;
@@ -389,6 +395,8 @@ __device__ __forceinline__ void force_item(const og_pair_args& a, const og_work&
             force_tile<MODEA, true, true, -1>(a, di, di, lane, xm, m14, acc);
         } else {
             const LaneData dj = load_lane(a, it.tj, a0j, cj, lane, ox, oy, oz);
+            if (MODEA && tiles_beyond(tile_radius(di, ci, lane, 0.0f, 0.0f, 0.0f), dj, cj, lane, force_cutoff2(a)))
+                return;
             if (it.mask >= 0) {
                 if (it.part < 0) force_tile<MODEA, true, false, -1>(a, di, dj, lane, xm, m14, acc);
                 else if (it.part == 0) force_tile<MODEA, true, false, 0>(a, di, dj, lane, xm, m14, acc);

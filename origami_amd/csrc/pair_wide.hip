@@ -29,10 +29,12 @@ namespace {
 // ---------------------------------------------------------------------------
 // Descreening
 // ---------------------------------------------------------------------------
+// a tile pair's form: as it stands, the far-field one, beyond the cutoff
+enum { WK_NEAR = 0, WK_FAR, WK_NONE };
 struct WideDescreen {
     float4 pq[2 * (OG_TILE + 1)];      // j atoms as in descreen_tile_lds: P, then Q
     float h[2][OG_TILE][OG_TILE];      // [i side, j side][step][lane]
-    int far_pair;
+    int kind;                          // WK_*
 };
 
 // Steps [KB, KE) of the tile pair in the wave's lanes: step k pairs lane l with
@@ -89,11 +91,14 @@ __device__ __forceinline__ void wide_descreen_item(WideDescreen& L, const og_pai
         Q[lane] = qj;
         if (lane == 0) { P[OG_TILE] = pj; Q[OG_TILE] = qj; }
         const bool far = it.ti != it.tj && descreen_far(a, di, dj, ci, cj, lane);
-        if (lane == 0) L.far_pair = far;
+        const bool none = MODEA && it.ti != it.tj && it.part < 0 &&
+                          tiles_beyond(tile_radius(di, ci, lane, 0.0f, 0.0f, 0.0f), dj, cj, lane, a.rc2_ds);
+        if (lane == 0) L.kind = none ? WK_NONE : far ? WK_FAR : WK_NEAR;
     }
     __syncthreads();
     int* fl = a.sflag ? a.sflag + it.sys : nullptr;
-    if (L.far_pair) {                  // the series is short: one wave runs it whole
+    if (MODEA && L.kind == WK_NONE) return;
+    if (L.kind == WK_FAR) {                  // the series is short: one wave runs it whole
         if (wave != 0) return;
         float acc_i = 0.0f, acc_j = 0.0f;
         if (it.part < 0) descreen_tile_far<MODEA, -1>(a, di, P, Q, lane, acc_i, acc_j);
@@ -121,35 +126,47 @@ struct WideForce {
     float j[OG_WIDE_GROUP][WJ_N][OG_TILE];
     float i[2][3][OG_TILE];            // positions of the (two) i tiles
     float j14[2][OG_TILE];             // 1-4 parameters (items)
-    int kind[OG_WIDE_GROUP];           // per j tile: WK_*
+    int kind[OG_STRIP_J];              // per j tile: WK_*
     float c[2][2][OG_TILE][OG_TILE];   // [buffer][i tile][step][lane] pair coefficients
 };
-enum { WK_NEAR = 0, WK_FAR, WK_NONE };
 
-// load_lane with the Born radius formed from the descreening integral
-// (padding slots keep R = gw = 1, as the engine lays them out).
-__device__ __forceinline__ LaneData wide_lane(const og_pair_args& a, const double* rho, int tile, int atom0, int cnt,
-                                              int lane, double ox, double oy, double oz) {
-    LaneData d;
-    const int slot = tile * OG_TILE + lane;
-    float R = 1.0f, gw = 1.0f;
+// The position of a tile's atom relative to the origin (as load_lane).
+__device__ __forceinline__ void wide_pos(LaneData& d, const og_pair_args& a, int atom0, int cnt, int lane, double ox,
+                                         double oy, double oz) {
     if (lane < cnt) {
         const double* p = a.pos + 3 * (size_t)(atom0 + lane);
         d.x = (float)(p[0] - ox);
         d.y = (float)(p[1] - oy);
         d.z = (float)(p[2] - oz);
-        bool clamped;
-        const double Rd = born_radius((double)a.iacc[atom0 + lane] * OG_FIX_INV, rho[atom0 + lane], clamped);
-        R = (float)Rd;
-        gw = (float)(kGbWidth / Rd);
     } else {
         d.x = 1.0e6f + 97.0f * (float)lane;
         d.y = 1.0e6f;
         d.z = 1.0e6f;
     }
+}
+
+// The rest of load_lane, the Born radius formed from the descreening integral
+// (padding slots keep R = gw = 1, as the engine lays them out).
+__device__ __forceinline__ void wide_fill(LaneData& d, const og_pair_args& a, const double* rho, int tile, int atom0,
+                                          int cnt, int lane) {
+    const int slot = tile * OG_TILE + lane;
+    float R = 1.0f, gw = 1.0f;
+    if (lane < cnt) {
+        bool clamped;
+        const double Rd = born_radius((double)a.iacc[atom0 + lane] * OG_FIX_INV, rho[atom0 + lane], clamped);
+        R = (float)Rd;
+        gw = (float)(kGbWidth / Rd);
+    }
     d.q = a.qs[slot];
     d.par = a.par[slot];
     d.gb = make_float4(0.0f, 0.0f, R, gw);
+}
+
+__device__ __forceinline__ LaneData wide_lane(const og_pair_args& a, const double* rho, int tile, int atom0, int cnt,
+                                              int lane, double ox, double oy, double oz) {
+    LaneData d;
+    wide_pos(d, a, atom0, cnt, lane, ox, oy, oz);
+    wide_fill(d, a, rho, tile, atom0, cnt, lane);
     return d;
 }
 
@@ -210,15 +227,24 @@ __device__ __forceinline__ void wide_force_item(WideForce& L, const og_pair_args
     const int a0i = a.tile_atom0[it.ti], ci = a.tile_cnt[it.ti];
     const int a0j = a.tile_atom0[it.tj], cj = a.tile_cnt[it.tj];
     const double ox = a.pos[3 * (size_t)a0i], oy = a.pos[3 * (size_t)a0i + 1], oz = a.pos[3 * (size_t)a0i + 2];
-    const LaneData di = wide_lane(a, rho, it.ti, a0i, ci, lane, ox, oy, oz);
+    LaneData di, dj;
+    wide_pos(di, a, a0i, ci, lane, ox, oy, oz);
     const bool diag = it.ti == it.tj;
+    // half tile pairs (systems of up to four tiles) are short and mostly within
+    // the cutoff: the test would cost them more than it saves
+    if (MODEA && !diag && it.part < 0) {
+        // every wave decides for itself, so that they agree without a barrier
+        wide_pos(dj, a, a0j, cj, lane, ox, oy, oz);
+        if (tiles_beyond(tile_radius(di, ci, lane, 0.0f, 0.0f, 0.0f), dj, cj, lane, force_cutoff2(a))) return;
+    }
+    wide_fill(di, a, rho, it.ti, a0i, ci, lane);
     unsigned long long xm = 0, m14 = 0;
     if (it.mask >= 0) {
         xm = a.masks[(size_t)it.mask * 128 + lane];
         m14 = a.masks[(size_t)it.mask * 128 + 64 + lane];
     }
     if (wave == 0) {
-        const LaneData dj = diag ? di : wide_lane(a, rho, it.tj, a0j, cj, lane, ox, oy, oz);
+        dj = diag ? di : wide_lane(a, rho, it.tj, a0j, cj, lane, ox, oy, oz);
         wide_store_j(L, 0, dj, lane);
         L.j14[0][lane] = dj.par.z;
         L.j14[1][lane] = dj.par.w;
@@ -255,82 +281,160 @@ __device__ __forceinline__ void wide_force_item(WideForce& L, const og_pair_args
     }
 }
 
-// A strip (force_strip of pair_kernels.hip).  Two coefficient buffers: the
-// waves that sum tile q's coefficients do so while the others form tile
-// q + 1's, one barrier per j tile.
+// What a block does with a strip (force_strip of pair_kernels.hip).
+//   WS_BOTH   everything; two coefficient buffers, one barrier per j tile: the
+//             waves that sum tile q's coefficients do so while the others form
+//             tile q + 1's
+//   WS_I + h  i tile h's sums only: its coefficients with every j tile of a
+//             group, then 64 steps per j tile in a row on one wave a component
+//   WS_J + q  j tile q's sums only
+// The split forms evaluate each pair twice but take a strip over 2 + nj CUs.
+enum { WS_BOTH = 0, WS_I = 1, WS_J = 3 };
+
+// i-side sum of component `wave`, continued over 64 steps; the j position
+// comes around the wave by rotation as in force_tile.
+__device__ __forceinline__ void wide_sum_i(const float (*c)[OG_TILE], const float* xj, float xi, int lane, float& f) {
+    float x = xj[lane];
+#pragma unroll 16
+    for (int k = 0; k < OG_TILE; ++k) {
+        f = fmaf(c[k][lane], x - xi, f);
+        x = rot(x);
+    }
+}
+
+// j-side sum of one component: lane = j atom, whose partners at step k are
+// lane - k of both i tiles, the first tile's added first.
+__device__ __forceinline__ float wide_sum_j(const float (*ca)[OG_TILE], const float (*cb)[OG_TILE], float x,
+                                            const float* xa, const float* xb, int lane) {
+    float g = 0.0f;
+#pragma unroll 16
+    for (int k = 0; k < OG_TILE; ++k) {
+        const int l = (lane - k) & 63;
+        g = fmaf(-cb[k][l], x - xb[l], fmaf(-ca[k][l], x - xa[l], g));
+    }
+    return g;
+}
+
 template <bool MODEA>
 __device__ __forceinline__ void wide_force_strip(WideForce& L, const og_pair_args& a, const double* rho,
-                                                 const og_strip* sp, int lane, int wave) {
+                                                 const og_strip* sp, int role, int lane, int wave) {
     const int ta = __builtin_amdgcn_readfirstlane(sp->ti), tb = ta + 1;
-    const int nj = __builtin_amdgcn_readfirstlane(sp->nj);
+    int nj = __builtin_amdgcn_readfirstlane(sp->nj), j0 = 0;
+    if (role >= WS_J) {
+        j0 = role - WS_J;
+        if (j0 >= nj) return;
+        nj = j0 + 1;
+    }
     const int a0 = a.tile_atom0[ta], b0 = a.tile_atom0[tb];
     const int ca = a.tile_cnt[ta], cb = a.tile_cnt[tb];
     const double ox = a.pos[3 * (size_t)a0], oy = a.pos[3 * (size_t)a0 + 1], oz = a.pos[3 * (size_t)a0 + 2];
-    const LaneData da = wide_lane(a, rho, ta, a0, ca, lane, ox, oy, oz);
-    const LaneData db = wide_lane(a, rho, tb, b0, cb, lane, ox, oy, oz);
+    LaneData da, db;
+    wide_pos(da, a, a0, ca, lane, ox, oy, oz);
+    wide_pos(db, a, b0, cb, lane, ox, oy, oz);
+    if (MODEA) {
+        // the j tiles beyond the cutoff, before anything else is formed
+        const float rad = fmaxf(tile_radius(da, ca, lane, 0.0f, 0.0f, 0.0f), tile_radius(db, cb, lane, 0.0f, 0.0f, 0.0f));
+        const int q = j0 + wave;
+        if (q < nj) {
+            const int tj = __builtin_amdgcn_readfirstlane(sp->tj[q]);
+            const int cj = a.tile_cnt[tj];
+            LaneData dj;
+            wide_pos(dj, a, a.tile_atom0[tj], cj, lane, ox, oy, oz);
+            const bool none = tiles_beyond(rad, dj, cj, lane, force_cutoff2(a));
+            if (lane == 0) L.kind[q] = none ? WK_NONE : WK_NEAR;
+        }
+        __syncthreads();
+        bool any = false;
+        for (int k = j0; k < nj; ++k) any = any || L.kind[k] != WK_NONE;
+        if (!any) return;
+    }
+    wide_fill(da, a, rho, ta, a0, ca, lane);
+    wide_fill(db, a, rho, tb, b0, cb, lane);
     const StripAtom A = strip_atom(da), B = strip_atom(db);
     const StripBound bi = strip_bound(A, B);
     if (wave == 4) wide_store_i(L, 0, da, lane);
     if (wave == 5) wide_store_i(L, 1, db, lane);
     int* fl = a.sflag ? a.sflag + sp->sys : nullptr;
     float fa = 0.0f, fb = 0.0f;        // waves 0-2: this component's i-side sums
+    // coefficients of i atom I and j tile q into c, 1/8 of the steps per wave
+    auto coefs = [&](const StripAtom& I, int q, float (*c)[OG_TILE], auto far_tag) {
+        constexpr bool F = decltype(far_tag)::value;
+        constexpr int N = OG_TILE / OG_WIDE_WAVES;
+        const float(*J)[OG_TILE] = L.j[q];
+#pragma unroll 4
+        for (int u = 0; u < N; ++u) {
+            const int k = wave * N + u, e = (lane + k) & 63;
+            const float4 pj = make_float4(J[WJ_X][e], J[WJ_Y][e], J[WJ_Z][e], J[WJ_Q][e]);
+            const float4 qj = make_float4(J[WJ_SE][e], J[WJ_RM][e], J[WJ_R][e], J[WJ_GW][e]);
+            c[k][lane] = strip_coef<MODEA, F>(a, I, pj, qj, pj.x - I.x, pj.y - I.y, pj.z - I.z);
+        }
+    };
+    auto flush_j = [&](int tj, int d, float g) {
+        if (lane < a.tile_cnt[tj])
+            og_atomic_add_fix(a.facc + 3 * (size_t)(a.tile_atom0[tj] + lane) + d, og_to_fix_chk((double)g, fl));
+    };
     int buf = 0;
-    for (int g0 = 0; g0 < nj; g0 += OG_WIDE_GROUP) {
-        if (wave < OG_WIDE_GROUP && g0 + wave < nj) {
+    for (int g0 = j0; g0 < nj; g0 += OG_WIDE_GROUP) {
+        if (wave < OG_WIDE_GROUP && g0 + wave < nj && !(MODEA && L.kind[g0 + wave] == WK_NONE)) {
             const int tj = __builtin_amdgcn_readfirstlane(sp->tj[g0 + wave]);
             const int cj = a.tile_cnt[tj];
             const LaneData dj = wide_lane(a, rho, tj, a.tile_atom0[tj], cj, lane, ox, oy, oz);
             wide_store_j(L, wave, dj, lane);
             const bool far = strip_far(bi, dj, cj, lane);
-            if (lane == 0) L.kind[wave] = far ? WK_FAR : WK_NEAR;
+            if (lane == 0) L.kind[g0 + wave] = far ? WK_FAR : WK_NEAR;
         }
         __syncthreads();
         const int ng = nj - g0 < OG_WIDE_GROUP ? nj - g0 : OG_WIDE_GROUP;
-        for (int q = 0; q < ng; ++q, buf ^= 1) {
-            const float(*J)[OG_TILE] = L.j[q];
-            auto coefs = [&](auto far_tag) {
-                constexpr bool F = decltype(far_tag)::value;
-                constexpr int N = OG_TILE / OG_WIDE_WAVES;
-#pragma unroll 4
-                for (int u = 0; u < N; ++u) {
-                    const int k = wave * N + u, e = (lane + k) & 63;
-                    const float4 pj = make_float4(J[WJ_X][e], J[WJ_Y][e], J[WJ_Z][e], J[WJ_Q][e]);
-                    const float4 qj = make_float4(J[WJ_SE][e], J[WJ_RM][e], J[WJ_R][e], J[WJ_GW][e]);
-                    L.c[buf][0][k][lane] = strip_coef<MODEA, F>(a, A, pj, qj, pj.x - A.x, pj.y - A.y, pj.z - A.z);
-                    L.c[buf][1][k][lane] = strip_coef<MODEA, F>(a, B, pj, qj, pj.x - B.x, pj.y - B.y, pj.z - B.z);
-                }
-            };
-            if (L.kind[q] == WK_FAR) coefs(std::true_type{});
-            else coefs(std::false_type{});
+        if (role == WS_I || role == WS_I + 1) {
+            const StripAtom& I = role == WS_I ? A : B;
+            float(*c)[OG_TILE] = &L.c[0][0][0];
+            for (int q = 0; q < ng; ++q) {
+                if (MODEA && L.kind[g0 + q] == WK_NONE) continue;
+                if (L.kind[g0 + q] == WK_FAR) coefs(I, q, c + q * OG_TILE, std::true_type{});
+                else coefs(I, q, c + q * OG_TILE, std::false_type{});
+            }
             __syncthreads();
             if (wave < 3) {
-                const float* xj = J[wave];
-                const float xa = L.i[0][wave][lane], xb = L.i[1][wave][lane];
-#pragma unroll 8
-                for (int k = 0; k < OG_TILE; ++k) {
-                    const float x = xj[(lane + k) & 63];
-                    fa = fmaf(L.c[buf][0][k][lane], x - xa, fa);
-                    fb = fmaf(L.c[buf][1][k][lane], x - xb, fb);
+                const float xi = L.i[role - WS_I][wave][lane];
+                for (int q = 0; q < ng; ++q) {
+                    if (MODEA && L.kind[g0 + q] == WK_NONE) continue;
+                    wide_sum_i(c + q * OG_TILE, L.j[q][wave], xi, lane, fa);
                 }
-            } else if (wave < 6) {
-                const int d = wave - 3;
-                const float x = J[d][lane];
-                float g = 0.0f;
-#pragma unroll 8
-                for (int k = 0; k < OG_TILE; ++k) {
-                    const int l = (lane - k) & 63;
-                    g = fmaf(-L.c[buf][1][k][l], x - L.i[1][d][l], fmaf(-L.c[buf][0][k][l], x - L.i[0][d][l], g));
+            }
+        } else {
+            for (int q = 0; q < ng; ++q) {
+                if (MODEA && L.kind[g0 + q] == WK_NONE) continue;
+                buf ^= 1;
+                if (L.kind[g0 + q] == WK_FAR) {
+                    coefs(A, q, L.c[buf][0], std::true_type{});
+                    coefs(B, q, L.c[buf][1], std::true_type{});
+                } else {
+                    coefs(A, q, L.c[buf][0], std::false_type{});
+                    coefs(B, q, L.c[buf][1], std::false_type{});
                 }
-                const int tj = __builtin_amdgcn_readfirstlane(sp->tj[g0 + q]);
-                if (lane < a.tile_cnt[tj])
-                    og_atomic_add_fix(a.facc + 3 * (size_t)(a.tile_atom0[tj] + lane) + d, og_to_fix_chk((double)g, fl));
+                __syncthreads();
+                if (wave < 3) {
+                    if (role == WS_BOTH) {
+                        wide_sum_i(L.c[buf][0], L.j[q][wave], L.i[0][wave][lane], lane, fa);
+                        wide_sum_i(L.c[buf][1], L.j[q][wave], L.i[1][wave][lane], lane, fb);
+                    }
+                } else if (wave < 6) {
+                    const int d = wave - 3;
+                    const float g = wide_sum_j(L.c[buf][0], L.c[buf][1], L.j[q][d][lane], L.i[0][d], L.i[1][d], lane);
+                    flush_j(__builtin_amdgcn_readfirstlane(sp->tj[g0 + q]), d, g);
+                }
             }
         }
         if (g0 + OG_WIDE_GROUP < nj) __syncthreads();      // the group's sums are done with its j atoms
     }
-    if (wave < 3) {
+    if (wave < 3 && role < WS_J) {
+        if (role == WS_I + 1) {
+            if (lane < cb) og_atomic_add_fix(a.facc + 3 * (size_t)(b0 + lane) + wave, og_to_fix_chk((double)fa, fl));
+            return;
+        }
         if (lane < ca) og_atomic_add_fix(a.facc + 3 * (size_t)(a0 + lane) + wave, og_to_fix_chk((double)fa, fl));
-        if (lane < cb) og_atomic_add_fix(a.facc + 3 * (size_t)(b0 + lane) + wave, og_to_fix_chk((double)fb, fl));
+        if (role == WS_BOTH && lane < cb)
+            og_atomic_add_fix(a.facc + 3 * (size_t)(b0 + lane) + wave, og_to_fix_chk((double)fb, fl));
     }
 }
 
@@ -348,21 +452,25 @@ __global__ void __launch_bounds__(OG_WIDE_THREADS) og_k_wide_descreen(og_pair_ar
     }
 }
 
-// blocks: strips, force items, then nr blocks of radii, the rest the gather
+// blocks: strips (ns blocks each), force items, then nr blocks of radii, the
+// rest the gather
 template <bool MODEA, bool NOISE>
 __global__ void __launch_bounds__(OG_WIDE_THREADS) og_k_wide_force(og_pair_args a, og_radii_args r, og_bonded_args b,
-                                                                   int nr) {
+                                                                   int ns, int nr) {
     __shared__ union {
         WideForce f;
         double t[3 * OG_GATHER_CHUNK];
     } L;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int k = blockIdx.x;
-    if (k < a.n_strip) {
-        wide_force_strip<MODEA>(L.f, a, r.rho, a.strips + k, lane, wave);
+    if (k < a.n_strip * ns) {
+        // the i-side blocks, the longer ones, come first
+        const int sub = k / a.n_strip;
+        wide_force_strip<MODEA>(L.f, a, r.rho, a.strips + (k - sub * a.n_strip), ns == 1 ? (int)WS_BOTH : WS_I + sub, lane,
+                                wave);
         return;
     }
-    k -= a.n_strip;
+    k -= a.n_strip * ns;
     if (k < a.n_fwork) {
         const og_work it = a.fwork[k];
         wide_force_item<MODEA>(L.f, a, r.rho, it, lane, wave);
@@ -384,10 +492,11 @@ void og_launch_wide_force(const og_pair_args& a, const og_radii_args& r, const o
                           hipStream_t s) {
     const int nr = (r.n_atoms + OG_WIDE_THREADS - 1) / OG_WIDE_THREADS;
     const int ng = (b.n_atoms + OG_GATHER_ATOMS - 1) / OG_GATHER_ATOMS;
-    const dim3 g(a.n_strip + a.n_fwork + nr + ng), t(OG_WIDE_THREADS);
+    const int ns = 2 * a.strip_j * a.n_strip <= OG_WIDE_SPLIT_MAX ? 2 + a.strip_j : 1;
+    const dim3 g(a.n_strip * ns + a.n_fwork + nr + ng), t(OG_WIDE_THREADS);
     const bool noise = b.noise.noise != nullptr;
-    if (mode_a && noise) hipLaunchKernelGGL((og_k_wide_force<true, true>), g, t, 0, s, a, r, b, nr);
-    else if (mode_a) hipLaunchKernelGGL((og_k_wide_force<true, false>), g, t, 0, s, a, r, b, nr);
-    else if (noise) hipLaunchKernelGGL((og_k_wide_force<false, true>), g, t, 0, s, a, r, b, nr);
-    else hipLaunchKernelGGL((og_k_wide_force<false, false>), g, t, 0, s, a, r, b, nr);
+    if (mode_a && noise) hipLaunchKernelGGL((og_k_wide_force<true, true>), g, t, 0, s, a, r, b, ns, nr);
+    else if (mode_a) hipLaunchKernelGGL((og_k_wide_force<true, false>), g, t, 0, s, a, r, b, ns, nr);
+    else if (noise) hipLaunchKernelGGL((og_k_wide_force<false, true>), g, t, 0, s, a, r, b, ns, nr);
+    else hipLaunchKernelGGL((og_k_wide_force<false, false>), g, t, 0, s, a, r, b, ns, nr);
 }

@@ -68,10 +68,20 @@ def test_block_per_item_equals_wave_per_item(E, chains, strip, mode_a):
         assert np.array_equal(a, b)
 
 
-def test_block_per_item_forces_against_oracle(E):
-    """Against the FP64 oracle within the engine's force bar (1e-5)."""
+@pytest.mark.parametrize("stretch", [1.0, 1.7, 1.0e4])
+@pytest.mark.parametrize("profiled", [False, True])
+@pytest.mark.parametrize("mode_a", [False, True])
+def test_pair_forces_against_oracle(E, mode_a, profiled, stretch):
+    """Both pair-kernel forms against the FP64 oracle within the engine's force
+    bar (1e-5): under the cutoffs, tile pairs on either side of them (stretched
+    coordinates move more of them past it, up to all) are left out only where
+    every pair is beyond."""
     s = S.seeded_chain(2, 70)
-    x = s.pos + np.random.default_rng(6).normal(scale=0.02, size=s.pos.shape)
-    ref = O.Oracle(s).total_force(x)
-    got = E.Engine([s]).total_force(x)
+    x = stretch * (s.pos + np.random.default_rng(6).normal(scale=0.02, size=s.pos.shape))
+    cut = (10.0, 10.0, 20.0) if mode_a else ()
+    orc = O.Oracle(s)
+    ref = orc.total_force(x, *cut)
+    eng = E.Engine([s])
+    eng.profile(profiled)
+    got = eng.total_force(x, mode_a=mode_a)
     assert np.sqrt(((got - ref) ** 2).sum() / (ref ** 2).sum()) < 1e-5
