@@ -55,6 +55,23 @@ OG_HD inline int pair_q(const PairDiv& d, int p) {
     return (int)(((unsigned long long)(unsigned)p * d.inv) >> 24);
 }
 
+// Division by a value that many quotients share: y = 1 / b once, then each
+// quotient from a product and two exact-remainder corrections (Markstein, IBM
+// J. Res. Dev. 34, 1990): q0 = RN(a y) is within two units in the last place,
+// q1 = RN(q0 + (a - b q0) y) within one, and for such a q1 and a correctly
+// rounded y, RN(q1 + (a - b q1) y) is a / b correctly rounded, barring
+// overflow and underflow (the values here lie between 1e-24 and 1e6, or are
+// zero).  Five operations instead of a division's eleven, one of them a
+// quarter-rate reciprocal; same bits.
+struct Rcp { double b, y; };
+OG_HD inline Rcp rcp_of(double b) { return {b, 1.0 / b}; }
+OG_HD inline double operator/(double a, Rcp r) {
+    double q = a * r.y;
+    q = fma(fma(-r.b, q, a), r.y, q);
+    return fma(fma(-r.b, q, a), r.y, q);
+}
+OG_HD inline v3 operator/(v3 a, Rcp r) { return {a.x / r, a.y / r, a.z / r}; }
+
 OG_HD inline Cap small_circle_new(v3 axis, double ca) { return {normalize(axis), ca}; }
 OG_HD inline bool contains_strict(const Cap& c, v3 p) { return dot(p, c.axis) > c.ca + 1e-12; }
 
@@ -410,7 +427,8 @@ OG_HD inline double cos_alpha_tangent(const CosAlphaP& P, v3 dri, v3 drk) {
 
 struct VertexJvpP {
     v3 wk, wl, np;
-    double dik, dil, cak, cal, sigma, denom, denom2, a, b, c, mn, num_a, num_b, sign;
+    Rcp dik, dil, denom2, c2, mn;       // what the tangents divide by
+    double cak, cal, sigma, denom, a, b, c, num_a, num_b, sign;
     CosAlphaP ck, cl;
     bool ok;
 };
@@ -419,32 +437,37 @@ OG_HD inline VertexJvpP vertex_jvp_primal(v3 pi, v3 pk, v3 pl, double ri, double
     VertexJvpP P{};
     P.ok = false;
     const v3 rkv = pk - pi;
-    P.dik = norm(rkv);
-    if (P.dik < 1e-12) return P;
+    const double dik = norm(rkv);
+    if (dik < 1e-12) return P;
+    P.dik = rcp_of(dik);
     P.wk = rkv / P.dik;
     const v3 rlv = pl - pi;
-    P.dil = norm(rlv);
-    if (P.dil < 1e-12) return P;
+    const double dil = norm(rlv);
+    if (dil < 1e-12) return P;
+    P.dil = rcp_of(dil);
     P.wl = rlv / P.dil;
-    P.cak = (P.dik * P.dik + ri * ri - rk * rk) / (2.0 * P.dik * ri);
-    P.cal = (P.dil * P.dil + ri * ri - rl * rl) / (2.0 * P.dil * ri);
+    P.cak = (dik * dik + ri * ri - rk * rk) / (2.0 * dik * ri);
+    P.cal = (dil * dil + ri * ri - rl * rl) / (2.0 * dil * ri);
     P.sigma = dot(P.wk, P.wl);
     P.denom = 1.0 - P.sigma * P.sigma;
     if (fabs(P.denom) < 1e-12) return P;
-    P.a = (P.cak - P.sigma * P.cal) / P.denom;
-    P.b = (P.cal - P.sigma * P.cak) / P.denom;
+    const Rcp denom = rcp_of(P.denom);
+    P.a = (P.cak - P.sigma * P.cal) / denom;
+    P.b = (P.cal - P.sigma * P.cak) / denom;
     const double c_sq = 1.0 - P.a * P.a - P.b * P.b - 2.0 * P.a * P.b * P.sigma;
     if (c_sq <= 0.0) return P;
     P.c = sqrt(c_sq);
+    P.c2 = rcp_of(2.0 * P.c);
     const v3 m = cross(P.wk, P.wl);
-    P.mn = sqrt(norm2(m));
-    if (P.mn < 1e-12) return P;
+    const double mn = sqrt(norm2(m));
+    if (mn < 1e-12) return P;
+    P.mn = rcp_of(mn);
     P.np = m / P.mn;
     P.ck = cos_alpha_primal(pi, pk, ri, rk);
     P.cl = cos_alpha_primal(pi, pl, ri, rl);
     P.num_a = P.cak - P.sigma * P.cal;
     P.num_b = P.cal - P.sigma * P.cak;
-    P.denom2 = P.denom * P.denom;
+    P.denom2 = rcp_of(P.denom * P.denom);
     P.sign = sign;
     P.ok = true;
     return P;
@@ -465,7 +488,7 @@ OG_HD inline v3 vertex_jvp_tangent(const VertexJvpP& P, v3 dri, v3 drk, v3 drl) 
     const double db = (dnum_b * P.denom - P.num_b * dden) / P.denom2;
     const double dc_sq = -2.0 * P.a * da - 2.0 * P.b * db - 2.0 * (da * P.b + P.a * db) * P.sigma -
                          2.0 * P.a * P.b * dsig;
-    const double dc = dc_sq / (2.0 * P.c);
+    const double dc = dc_sq / P.c2;
     const v3 dbase = P.wk * da + dwk * P.a + P.wl * db + dwl * P.b;
     const v3 dm = cross(dwk, P.wl) + cross(P.wk, dwl);
     const v3 dnp = (dm - P.np * dot(P.np, dm)) / P.mn;
@@ -476,7 +499,8 @@ OG_HD inline v3 vertex_jvp_tangent(const VertexJvpP& P, v3 dri, v3 drk, v3 drl) 
 struct ArcThetaP {
     VertexJvpP vs_p, ve_p;
     v3 wk, vs, ve, us, ue, x;
-    double dik, vdo_s, vdo_e, nn_s, nn_e, cos_t, sin_t;
+    Rcp dik, nn_s, nn_e;
+    double vdo_s, vdo_e, cos_t, sin_t;
     bool ok;
 };
 
@@ -485,10 +509,11 @@ OG_HD inline ArcThetaP arc_theta_primal(v3 pi, v3 pk, v3 pl, v3 pm, double ri, d
     ArcThetaP P{};
     P.ok = false;
     const v3 rkv = pk - pi;
-    P.dik = norm(rkv);
-    if (P.dik < 1e-12) return P;
+    const double dik = norm(rkv);
+    if (dik < 1e-12) return P;
+    P.dik = rcp_of(dik);
     P.wk = rkv / P.dik;
-    const double cak = (P.dik * P.dik + ri * ri - rk * rk) / (2.0 * P.dik * ri);
+    const double cak = (dik * dik + ri * ri - rk * rk) / (2.0 * dik * ri);
     const Cap ck = small_circle_new(P.wk, cak);
     if (norm(pl - pi) < 1e-12) return P;
     const Cap cl = cap_from(pi, pl, ri, rl);
@@ -503,15 +528,17 @@ OG_HD inline ArcThetaP arc_theta_primal(v3 pi, v3 pk, v3 pl, v3 pm, double ri, d
     {
         P.vdo_s = dot(P.vs, P.wk);
         const v3 proj = P.vs - P.wk * P.vdo_s;
-        P.nn_s = norm(proj);
-        if (P.nn_s < 1e-12) return P;
+        const double nn = norm(proj);
+        if (nn < 1e-12) return P;
+        P.nn_s = rcp_of(nn);
         P.us = proj / P.nn_s;
     }
     {
         P.vdo_e = dot(P.ve, P.wk);
         const v3 proj = P.ve - P.wk * P.vdo_e;
-        P.nn_e = norm(proj);
-        if (P.nn_e < 1e-12) return P;
+        const double nn = norm(proj);
+        if (nn < 1e-12) return P;
+        P.nn_e = rcp_of(nn);
         P.ue = proj / P.nn_e;
     }
     P.cos_t = dot(P.us, P.ue);
@@ -547,7 +574,8 @@ OG_HD inline double arc_theta_tangent(const ArcThetaP& P, v3 dri, v3 drk, v3 drl
 struct VertexEpsP {
     VertexJvpP vp;
     v3 wk, wl, v, tin, tout, x;
-    double dik, dil, nn_in, nn_out, ce, se;
+    Rcp dik, dil, nn_in, nn_out;
+    double ce, se;
     bool ok;
 };
 
@@ -555,29 +583,33 @@ OG_HD inline VertexEpsP vertex_eps_primal(v3 pi, v3 pk, v3 pl, double ri, double
     VertexEpsP P{};
     P.ok = false;
     const v3 rkv = pk - pi;
-    P.dik = norm(rkv);
-    if (P.dik < 1e-12) return P;
+    const double dik = norm(rkv);
+    if (dik < 1e-12) return P;
+    P.dik = rcp_of(dik);
     P.wk = rkv / P.dik;
     const v3 rlv = pl - pi;
-    P.dil = norm(rlv);
-    if (P.dil < 1e-12) return P;
+    const double dil = norm(rlv);
+    if (dil < 1e-12) return P;
+    P.dil = rcp_of(dil);
     P.wl = rlv / P.dil;
-    const double cak = (P.dik * P.dik + ri * ri - rk * rk) / (2.0 * P.dik * ri);
-    const double cal = (P.dil * P.dil + ri * ri - rl * rl) / (2.0 * P.dil * ri);
+    const double cak = (dik * dik + ri * ri - rk * rk) / (2.0 * dik * ri);
+    const double cal = (dil * dil + ri * ri - rl * rl) / (2.0 * dil * ri);
     const Cap ck = small_circle_new(P.wk, cak), cl = small_circle_new(P.wl, cal);
     if (!vertex_point(ck, cl, sign, P.v)) return P;
     P.vp = vertex_jvp_primal(pi, pk, pl, ri, rk, rl, sign);
     if (!P.vp.ok) return P;
     {
         const v3 cr = cross(P.v, P.wk);
-        P.nn_in = norm(cr);
-        if (P.nn_in < 1e-12) return P;
+        const double nn = norm(cr);
+        if (nn < 1e-12) return P;
+        P.nn_in = rcp_of(nn);
         P.tin = cr / P.nn_in;
     }
     {
         const v3 cr = cross(P.v, P.wl);
-        P.nn_out = norm(cr);
-        if (P.nn_out < 1e-12) return P;
+        const double nn = norm(cr);
+        if (nn < 1e-12) return P;
+        P.nn_out = rcp_of(nn);
         P.tout = cr / P.nn_out;
     }
     P.ce = dot(P.tin, P.tout);

@@ -17,6 +17,13 @@ long long host_pair_div_mismatches(void) {
     return bad;
 }
 
+// Mismatches of the shared-divisor quotient against division.
+long long host_rcp_mismatches(long long n, const double* a, const double* b) {
+    long long bad = 0;
+    for (long long i = 0; i < n; ++i) bad += a[i] / rcp_of(b[i]) != a[i] / b[i];
+    return bad;
+}
+
 // counts[i] = intersect_count, fast[i] = intersect_count_fast for cap pairs
 // (axis1, ca1, axis2, ca2) packed as 8 doubles each.
 void host_intersect_counts(int n, const double* caps, int* counts, int* fast) {

@@ -85,3 +85,29 @@ def test_pair_forces_against_oracle(E, mode_a, profiled, stretch):
     eng.profile(profiled)
     got = eng.total_force(x, mode_a=mode_a)
     assert np.sqrt(((got - ref) ** 2).sum() / (ref ** 2).sum()) < 1e-5
+
+
+@pytest.mark.parametrize("chains", [[(3, 3)], [(21, 4), (16, 4)], [(2, 70)]])
+def test_sasa_terms_forms_agree(E, chains):
+    """The SASA terms with a direction per lane (short lists) equal those with
+    a thread per arc (batches above 4 096 SASA atoms) bit for bit: a system's
+    SASA forces alone and inside a large batch."""
+    systems = [S.seeded_chain(*c) for c in chains]
+    rng = np.random.default_rng(8)
+    x = [s.pos + rng.normal(scale=0.02, size=s.pos.shape) for s in systems]
+    filler = S.seeded_chain(5, 300)
+    fx = filler.pos + rng.normal(scale=0.02, size=filler.pos.shape)
+    alone = E.Engine(systems)
+    batch = E.Engine(systems + [filler] * 4)
+    assert alone.info()["sasa_work_atoms"] <= 4096 < batch.info()["sasa_work_atoms"]
+    n = alone.n_atoms
+
+    def sasa(eng, pos):
+        # the pair and bonded parts are the same integers in both calls
+        return eng.total_force(pos, include_sasa=True) - eng.total_force(pos)
+
+    xs = np.concatenate(x)
+    a, b = sasa(alone, xs), sasa(batch, np.concatenate([xs] + [fx] * 4))[:n]
+    assert np.array_equal(a, b)
+    ref = np.concatenate([O.Oracle(s).sasa_forces(p)[0] for s, p in zip(systems, x)])
+    assert np.abs(a - ref).max() < 1e-8

@@ -287,6 +287,30 @@ def test_cover_walk_on_chain_atoms(host):
     assert checked > 200
 
 
+@pytest.mark.parametrize("lo, hi", [(-80, 20), (-1, 1), (0, 0)])
+def test_shared_divisor_quotient_is_the_division(host, lo, hi):
+    # quotients by a shared divisor must have the bits of a division: random
+    # significands over the exponents the geometry meets, divisors next to
+    # powers of two on both sides, and quotients next to rounding boundaries
+    host.host_rcp_mismatches.restype = C.c_longlong
+    host.host_rcp_mismatches.argtypes = [C.c_longlong, C.POINTER(C.c_double), C.POINTER(C.c_double)]
+    rng = np.random.default_rng(lo + 100)
+    n = 2_000_000
+    one = 1.0 + rng.random(n)
+    b = np.ldexp(one, rng.integers(lo, hi + 1, n))
+    edge = rng.random(n) < 0.2
+    b[edge] = np.ldexp(1.0 + rng.integers(0, 64, n) * 2.0 ** -52, 0)[edge]
+    edge = rng.random(n) < 0.2
+    b[edge] = np.ldexp(2.0 - rng.integers(1, 64, n) * 2.0 ** -52, 0)[edge]
+    a = np.ldexp(1.0 + rng.random(n), rng.integers(lo, hi + 1, n)) * rng.choice([-1.0, 1.0], n)
+    near = rng.random(n) < 0.4          # a = b q rounded, a unit to either side: quotients near a tie
+    q = 1.0 + rng.integers(0, 1 << 52, n) * 2.0 ** -52 + 2.0 ** -53
+    a[near] = np.nextafter(b * q, rng.choice([-1.0, 1.0], n) * np.inf)[near]
+    a[:1000] = 0.0
+    a, b = np.ascontiguousarray(a), np.ascontiguousarray(b)
+    assert host.host_rcp_mismatches(n, _ptr(a, C.c_double), _ptr(b, C.c_double)) == 0
+
+
 def test_jvp_split_is_bit_identical(host):
     # the terms kernel forms each arc's / vertex's primal geometry once and
     # one tangent per direction; every term must equal the full JVP's bits
