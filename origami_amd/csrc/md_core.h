@@ -193,9 +193,9 @@ __device__ __forceinline__ bool shake_cluster(double (&xs)[3 * MC], const double
     return false;
 }
 
-// Cluster c (at most MC atoms) for step `step` (the Philox counter).  PRE:
-// the O step reads its normals from a.noise rather than forming them.
-template <int MC, bool PRE>
+// Cluster c (at most MC atoms) for step `step`; the O step reads its normals
+// from a.noise.
+template <int MC>
 __device__ __forceinline__ void cluster_body(const og_cluster_args& a, int c, uint32_t step) {
     const int s0 = a.cl_start[c], na = a.cl_start[c + 1] - s0;
     const int k0 = a.cn_start[c], nc = a.cn_start[c + 1] - k0;
@@ -243,13 +243,8 @@ __device__ __forceinline__ void cluster_body(const og_cluster_args& a, int c, ui
                 if (t < na) {
                     const int g = at[t];
                     const double sigma = sqrt(om * kbt * dofc * OG_ACCEL / a.mass[g]);
-                    double g0, g1, g2;
-                    if (PRE) {
-                        const double* nz = a.noise + (size_t)(step & 1u) * 3 * a.n_atoms + 3 * (size_t)g;
-                        g0 = nz[0]; g1 = nz[1]; g2 = nz[2];
-                    } else {
-                        noise3(a.key0, a.key1, (uint32_t)sys, (uint32_t)a.atom_local[g], step, g0, g1, g2);
-                    }
+                    const double* nz = a.noise + (size_t)(step & 1u) * 3 * a.n_atoms + 3 * (size_t)g;
+                    const double g0 = nz[0], g1 = nz[1], g2 = nz[2];
                     vs[3 * t] = a.alpha * vs[3 * t] + sigma * g0;
                     vs[3 * t + 1] = a.alpha * vs[3 * t + 1] + sigma * g1;
                     vs[3 * t + 2] = a.alpha * vs[3 * t + 2] + sigma * g2;

@@ -106,14 +106,11 @@ void og_launch_radii(const og_radii_args& a, bool energy, hipStream_t s) {
 }
 
 // One thread per cluster of at most MC atoms: clusters [c_begin, c_end).
-// PRE: the O step reads its normals from a.noise (formed by og_k_noise)
-// rather than forming them; a separate instance keeps the other one's
-// registers as they are.
-template <int MC, bool PRE>
+template <int MC>
 __global__ void __launch_bounds__(256) og_k_cluster_step(og_cluster_args a, int c_begin, int c_end) {
     const int c = c_begin + blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= c_end) return;
-    cluster_body<MC, PRE>(a, c, a.step_dev ? *a.step_dev : a.step);
+    cluster_body<MC>(a, c, *a.step_dev);
 }
 
 __global__ void __launch_bounds__(256) og_k_noise(og_noise_args a) {
@@ -129,19 +126,10 @@ void og_launch_noise(const og_noise_args& a, hipStream_t s) {
 void og_launch_cluster_step(const og_cluster_args& a, hipStream_t s) {
     if (a.n_clusters <= 0) return;
     const dim3 g_small((a.n_small + 255) / 256), g_large((a.n_clusters - a.n_small + 255) / 256);
-    if (a.noise) {
-        if (a.n_small > 0)
-            hipLaunchKernelGGL((og_k_cluster_step<OG_SMALL_CL, true>), g_small, dim3(256), 0, s, a, 0, a.n_small);
-        if (a.n_clusters > a.n_small)
-            hipLaunchKernelGGL((og_k_cluster_step<OG_MAX_CL, true>), g_large, dim3(256), 0, s, a, a.n_small,
-                               a.n_clusters);
-    } else {
-        if (a.n_small > 0)
-            hipLaunchKernelGGL((og_k_cluster_step<OG_SMALL_CL, false>), g_small, dim3(256), 0, s, a, 0, a.n_small);
-        if (a.n_clusters > a.n_small)
-            hipLaunchKernelGGL((og_k_cluster_step<OG_MAX_CL, false>), g_large, dim3(256), 0, s, a, a.n_small,
-                               a.n_clusters);
-    }
+    if (a.n_small > 0)
+        hipLaunchKernelGGL(og_k_cluster_step<OG_SMALL_CL>, g_small, dim3(256), 0, s, a, 0, a.n_small);
+    if (a.n_clusters > a.n_small)
+        hipLaunchKernelGGL(og_k_cluster_step<OG_MAX_CL>, g_large, dim3(256), 0, s, a, a.n_small, a.n_clusters);
 }
 
 __global__ void __launch_bounds__(256) og_k_zero_acc(long long* facc, long long* iacc, int n) {

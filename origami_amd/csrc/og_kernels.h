@@ -106,7 +106,6 @@ struct og_cluster_args {
     long long* facc; long long* iacc;
     const double* mass;
     const int* atom_sys;
-    const int* atom_local;           // index within its system (RNG counter)
     const int* cl_start;             // [C+1] atoms of cluster c: cl_atoms[cl_start[c]..],
     const int* cl_atoms;             //   heavy atom first, then the hydrogen of each constraint
     const int* cn_start;             // [C+1] constraints of cluster c (constraint m: atoms 0, m + 1)
@@ -119,10 +118,8 @@ struct og_cluster_args {
     const int* diverged;             // [S]
     double dt, alpha;
     int use_shake;
-    uint32_t key0, key1;
-    uint32_t step;
-    const uint32_t* step_dev;        // if set, the step counter is read from device memory
-    const double* noise;             // if set, the O step's normals: [2][3N], step s in half s & 1
+    const uint32_t* step_dev;        // step counter in device memory
+    const double* noise;             // the O step's normals: [2][3N], step s in half s & 1
     int n_atoms;
 };
 

@@ -655,7 +655,7 @@ void og_launch_pair_energy64(const og_pair_args& a, const og_energy64_args& e, b
 // threads per block of the persistent replica-step kernel: 8 waves, which
 // take the work items of each phase (tile pairs, strips) in turn
 #define OG_PERSIST_THREADS 512
-template <bool MODEA, bool PRE>
+template <bool MODEA>
 __global__ void __launch_bounds__(OG_PERSIST_THREADS) og_k_replica_steps(og_pair_args pa, og_bonded_args ba, og_radii_args ra,
                                                           og_cluster_args ca, og_back_args bk, og_noise_args nz,
                                                           og_persist_args pp) {
@@ -674,12 +674,10 @@ __global__ void __launch_bounds__(OG_PERSIST_THREADS) og_k_replica_steps(og_pair
         __syncthreads();
         if (s_stop) break;
         const uint32_t step = pp.step0 + (uint32_t)k;
-        if (PRE) {
-            for (int i = a0 + tid; i < a1; i += NT) noise_atom_at(nz, i, step);
-            __syncthreads();
-        }
+        for (int i = a0 + tid; i < a1; i += NT) noise_atom_at(nz, i, step);
+        __syncthreads();
         for (int q = pp.cl_small_off[s] + tid; q < pp.cl_small_off[s + 1]; q += NT)
-            cluster_body<OG_SMALL_CL, PRE>(ca, pp.cl_small[q], step);
+            cluster_body<OG_SMALL_CL>(ca, pp.cl_small[q], step);
         __syncthreads();
 #pragma unroll
         for (int kind = 0; kind < 4; ++kind) {
@@ -721,13 +719,7 @@ void og_launch_replica_steps(const og_pair_args& pa, const og_bonded_args& ba, c
                              const og_cluster_args& ca, const og_back_args& bk, const og_noise_args& nz,
                              const og_persist_args& pp, bool mode_a, hipStream_t s) {
     if (pp.n_sys <= 0 || pp.n_steps <= 0) return;
-    const bool pre = nz.noise != nullptr;
-    if (mode_a) {
-        if (pre) hipLaunchKernelGGL((og_k_replica_steps<true, true>), dim3(pp.n_sys), dim3(OG_PERSIST_THREADS), 0, s, pa, ba, ra, ca, bk, nz, pp);
-        else hipLaunchKernelGGL((og_k_replica_steps<true, false>), dim3(pp.n_sys), dim3(OG_PERSIST_THREADS), 0, s, pa, ba, ra, ca, bk, nz, pp);
-    } else {
-        if (pre) hipLaunchKernelGGL((og_k_replica_steps<false, true>), dim3(pp.n_sys), dim3(OG_PERSIST_THREADS), 0, s, pa, ba, ra, ca, bk, nz, pp);
-        else hipLaunchKernelGGL((og_k_replica_steps<false, false>), dim3(pp.n_sys), dim3(OG_PERSIST_THREADS), 0, s, pa, ba, ra, ca, bk, nz, pp);
-    }
+    const dim3 g(pp.n_sys), t(OG_PERSIST_THREADS);
+    if (mode_a) hipLaunchKernelGGL(og_k_replica_steps<true>, g, t, 0, s, pa, ba, ra, ca, bk, nz, pp);
+    else hipLaunchKernelGGL(og_k_replica_steps<false>, g, t, 0, s, pa, ba, ra, ca, bk, nz, pp);
 }
-
