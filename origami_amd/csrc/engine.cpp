@@ -25,6 +25,7 @@
 // og_run's default: captured steps below this many atoms
 #define OG_SPLIT_MAX_TILES 4           // systems up to 256 atoms: off-diagonal tile pairs in halves
 #define OG_STRIP_DEFAULT 4             // j tiles per force strip until the autotuner picks
+#define OG_STAGE_MAX_ATOMS 8192        // host copies of up to so many atoms go through pinned staging
 #define OG_SR_DOTS 960                 // Shrake-Rupley dots per atom (SHRAKE_RUPLEY_DOTS, sasa.rs:27)
 #define OG_PERSIST_MAX_TILES 8         // persistent replica steps: systems of up to 512 atoms
 #define OG_PERSIST_CHUNK 512           // steps per persistent launch
@@ -110,6 +111,15 @@ struct og_engine {
     hipGraphExec_t gexec[2] = {nullptr, nullptr};   // step; step with surrogate check
     long long* noalloc_ke = nullptr;       // this device's og_run_noalloc scratch array
     int* eval_skip = nullptr;              // [S] systems an energy-only evaluation leaves out (minimiser probes)
+    // Pinned host memory that kernels read and write directly: coordinates and
+    // forces of small batches (3 stage_atoms doubles), energies, status words.
+    // A copy of a few KB costs a launch and a wait of its own, as much as a
+    // kernel of the evaluation; this way a call is kernels and one wait.
+    void* stage = nullptr;
+    size_t stage_bytes = 0;                // of the coordinate part
+    double* stage_x = nullptr;
+    long long* stage_e = nullptr;          // [S*OG_NE]
+    int* stage_i = nullptr;                // [3 S + 1]
     double* sr_dots = nullptr;             // [OG_SR_DOTS][3] Shrake-Rupley unit-sphere dots
     // persistent replica steps: per-system index ranges (og_persist_args)
     int *p_atom_off = nullptr, *p_cl_small_off = nullptr, *p_cl_small = nullptr, *p_cl_big_off = nullptr,
@@ -205,6 +215,7 @@ static void free_all(og_engine* e) {
     if (e->step_dev) (void)hipFree(e->step_dev);
     if (e->frames) (void)hipFree(e->frames);
     if (e->sr_dots) (void)hipFree(e->sr_dots);
+    if (e->stage) (void)hipHostFree(e->stage);
     for (int* q : {e->p_atom_off, e->p_cl_small_off, e->p_cl_small, e->p_cl_big_off, e->p_cl_big, e->p_term_off,
                    e->p_work_off, e->p_fwork_off, e->p_strip_off})
         if (q) (void)hipFree(q);
@@ -759,6 +770,14 @@ static int engine_build(og_engine* e, const og_system_desc* sys, int n_sys) {
         }
         HIPCHK(upload(&e->sr_dots, dots));
     }
+    {
+        e->stage_bytes = 3 * (size_t)std::min(N, OG_STAGE_MAX_ATOMS) * sizeof(double);
+        const size_t eb = (size_t)n_sys * OG_NE * sizeof(long long);
+        HIPCHK(hipHostMalloc(&e->stage, e->stage_bytes + eb + (3 * (size_t)n_sys + 1) * sizeof(int), hipHostMallocDefault));
+        e->stage_x = (double*)e->stage;
+        e->stage_e = (long long*)((char*)e->stage + e->stage_bytes);
+        e->stage_i = (int*)((char*)e->stage_e + eb);
+    }
     HIPCHK(hipStreamSynchronize(e->stream));
     HIPCHK(hipDeviceSynchronize());
     return OG_OK;
@@ -777,15 +796,57 @@ extern "C" int og_engine_info(const og_engine* e, int64_t* info) {
     return OG_OK;
 }
 
+// Index of the first non-finite value, n if there is none.
+static size_t first_nonfinite(const double* x, size_t n) {
+    double z[4] = {0.0, 0.0, 0.0, 0.0};            // x * 0 is a zero or NaN
+    size_t k = 0;
+    for (; k + 4 <= n; k += 4)
+        for (int q = 0; q < 4; ++q) z[q] += x[k + q] * 0.0;
+    for (; k < n; ++k) z[0] += x[k] * 0.0;
+    if ((z[0] + z[1]) + (z[2] + z[3]) == 0.0) return n;
+    for (k = 0; k < n; ++k)
+        if (!std::isfinite(x[k])) return k;
+    return n;
+}
+
+// words: 32-bit words of src published to dst (pinned host memory, or device)
+static void publish_add(og_publish_args& p, int q, const void* src, void* dst, size_t bytes) {
+    p.src[q] = (const uint32_t*)src;
+    p.dst[q] = (uint32_t*)dst;
+    p.n[q] = (int)(bytes / 4);
+}
+
+// Device words to the caller's buffer, through the staging buffer where they
+// fit; returns with the stream idle.
+static int fetch(og_engine* e, void* host, const void* dev, size_t bytes) {
+    if (bytes > e->stage_bytes) {
+        HIPCHK(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, e->stream));
+        HIPCHK(hipStreamSynchronize(e->stream));
+        return OG_OK;
+    }
+    og_publish_args p{};
+    publish_add(p, 0, dev, e->stage_x, bytes);
+    og_launch_publish(p, e->stream);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(e->stream));
+    std::memcpy(host, e->stage_x, bytes);
+    return OG_OK;
+}
+
 static int copy_state(og_engine* e, double* dev, const double* host, bool to_dev) {
     if (!e || !host) return fail(OG_ERR_ARG, "NULL argument");
-    const size_t bytes = 3 * (size_t)e->n_atoms * sizeof(double);
-    if (to_dev) {
-        for (size_t k = 0; k < 3 * (size_t)e->n_atoms; ++k)
-            if (!std::isfinite(host[k])) return fail(OG_ERR_ARG, "non-finite input at %zu", k);
-        HIPCHK(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, e->stream));
+    const size_t n = 3 * (size_t)e->n_atoms, bytes = n * sizeof(double);
+    if (!to_dev) return fetch(e, (void*)host, dev, bytes);
+    const size_t bad = first_nonfinite(host, n);
+    if (bad < n) return fail(OG_ERR_ARG, "non-finite input at %zu", bad);
+    if (bytes <= e->stage_bytes) {
+        std::memcpy(e->stage_x, host, bytes);
+        og_publish_args p{};
+        publish_add(p, 0, e->stage_x, dev, bytes);
+        og_launch_publish(p, e->stream);
+        HIPCHK(hipGetLastError());
     } else {
-        HIPCHK(hipMemcpyAsync((void*)host, dev, bytes, hipMemcpyDeviceToHost, e->stream));
+        HIPCHK(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, e->stream));
     }
     HIPCHK(hipStreamSynchronize(e->stream));
     return OG_OK;
@@ -984,8 +1045,10 @@ static int launch_forces(og_engine* e, uint32_t flags, double cutoff_a, double s
     return OG_OK;
 }
 
-static int check_sasa_overflow(og_engine* e, uint32_t flags) {
-    if (!(flags & (OG_SASA | OG_SASA_SR))) return OG_OK;
+// seen: the count published with the evaluation; nonzero counts are read
+// again and cleared.
+static int check_sasa_overflow(og_engine* e, uint32_t flags, int seen) {
+    if (!(flags & (OG_SASA | OG_SASA_SR)) || seen == 0) return OG_OK;
     int ovf = 0;
     if (og_sasa_overflow(&e->sasa, &ovf) != 0) return fail(OG_ERR_HIP, "reading SASA status failed");
     if (ovf) return fail(OG_ERR_ARG, "%d SASA atom evaluations exceeded the per-atom capacity "
@@ -997,14 +1060,6 @@ static const char* status_reason(int bits) {
     if (bits & OG_ST_SASA) return "a SASA atom exceeded the arrangement's capacity (128 caps / 256 arcs / 256 vertices)";
     if (bits & OG_ST_RANGE) return "a force or energy contribution was NaN or beyond the fixed-point range (|x| >= 2^30)";
     return "non-finite velocities";
-}
-
-static int read_energies(og_engine* e, double* out) {
-    std::vector<long long> acc((size_t)e->n_sys * OG_NE);
-    HIPCHK(hipMemcpyAsync(acc.data(), e->eacc, acc.size() * sizeof(long long), hipMemcpyDeviceToHost, e->stream));
-    HIPCHK(hipStreamSynchronize(e->stream));
-    for (size_t k = 0; k < acc.size(); ++k) out[k] = (double)acc[k] * OG_FIX_INV;
-    return OG_OK;
 }
 
 // forces = false: energies only; the engine's force array keeps the forces of
@@ -1020,13 +1075,26 @@ static int evaluate(og_engine* e, const double* xyz, double* f_out, uint32_t fla
         if (forces) return fail(OG_ERR_ARG, "OG_SASA_SR is an energy term only (og_energies)");
         if (flags & OG_SASA) return fail(OG_ERR_ARG, "OG_SASA and OG_SASA_SR select two SASA energies; pass one");
     }
-    if (xyz && (rc = og_set_positions(e, xyz))) return rc;
+    const size_t n3 = 3 * (size_t)e->n_atoms, bytes = n3 * sizeof(double);
+    const bool staged = bytes <= e->stage_bytes;
+    if (xyz && staged) {
+        const size_t bad = first_nonfinite(xyz, n3);
+        if (bad < n3) return fail(OG_ERR_ARG, "non-finite input at %zu", bad);
+        std::memcpy(e->stage_x, xyz, bytes);       // the stream is idle between calls
+    } else if (xyz && (rc = og_set_positions(e, xyz))) {
+        return rc;
+    }
     const bool energy = (flags & OG_ENERGY) || energies;
-    if (energy) HIPCHK(hipMemsetAsync(e->eacc, 0, (size_t)e->n_sys * OG_NE * sizeof(long long), e->stream));
-    HIPCHK(hipMemsetAsync(e->clamped, 0, (size_t)e->n_sys * sizeof(int), e->stream));
-    HIPCHK(hipMemsetAsync(e->sflag, 0, (size_t)e->n_sys * sizeof(int), e->stream));
-    og_launch_zero_acc(e->facc, e->iacc, e->n_atoms, e->stream);
-    if ((rc = launch_forces(e, flags, cutoff_a, sasa_gamma_scale, energy, -1, forces))) return rc;
+    og_begin_args bg{};
+    bg.xyz = xyz && staged ? e->stage_x : nullptr;
+    bg.pos = e->pos; bg.facc = e->facc; bg.iacc = e->iacc; bg.n_atoms = e->n_atoms;
+    bg.eacc = energy ? e->eacc : nullptr;
+    bg.sflag = e->sflag; bg.clamped = e->clamped; bg.n_sys = e->n_sys;
+    og_launch_begin(bg, e->stream);
+    if ((rc = launch_forces(e, flags, cutoff_a, sasa_gamma_scale, energy, -1, forces))) {
+        (void)hipStreamSynchronize(e->stream);
+        return rc;
+    }
     if (forces) {
         ProfScope p(e, OG_K_BACK);
         og_back_args b{};
@@ -1034,28 +1102,35 @@ static int evaluate(og_engine* e, const double* xyz, double* f_out, uint32_t fla
         b.atom_sys = e->atom_sys; b.n_atoms = e->n_atoms; b.dt = 0.0; b.do_kick = 0;
         b.ke_acc = nullptr; b.diverged = e->diverged; b.sflag = e->sflag;
         if (external) b.tun = e->tun;
+        if (f_out && staged) b.force_out = e->stage_x;
         og_launch_back(b, e->stream);
     }
-    HIPCHK(hipGetLastError());
-    if (f_out) {
-        HIPCHK(hipMemcpyAsync(f_out, e->force, 3 * (size_t)e->n_atoms * sizeof(double), hipMemcpyDeviceToHost, e->stream));
+    int* st = e->stage_i;                          // [S] status bits, then the SASA overflow count
+    {
+        og_publish_args p{};
+        publish_add(p, 0, e->sflag, st, (size_t)e->n_sys * sizeof(int));
+        if (flags & (OG_SASA | OG_SASA_SR)) publish_add(p, 1, e->sasa.overflow, st + e->n_sys, sizeof(int));
+        else st[e->n_sys] = 0;
+        if (energies) publish_add(p, 2, e->eacc, e->stage_e, (size_t)e->n_sys * OG_NE * sizeof(long long));
+        og_launch_publish(p, e->stream);
     }
+    HIPCHK(hipGetLastError());
+    if (f_out && !staged) HIPCHK(hipMemcpyAsync(f_out, e->force, bytes, hipMemcpyDeviceToHost, e->stream));
     HIPCHK(hipStreamSynchronize(e->stream));
     if (e->prof) prof_collect(e);
-    std::vector<int> st(e->n_sys);
-    HIPCHK(hipMemcpy(st.data(), e->sflag, e->n_sys * sizeof(int), hipMemcpyDeviceToHost));
+    if (f_out && staged) std::memcpy(f_out, e->stage_x, bytes);
     if (energies) {
-        if ((rc = read_energies(e, energies))) return rc;
+        for (size_t k = 0; k < (size_t)e->n_sys * OG_NE; ++k) energies[k] = (double)e->stage_e[k] * OG_FIX_INV;
         for (int s = 0; s < e->n_sys; ++s)     // a flagged system's sums are not its energies
             if (st[s])
                 for (int k = 0; k < OG_NE; ++k) energies[(size_t)s * OG_NE + k] = NAN;
     }
-    if ((rc = check_sasa_overflow(e, flags))) return rc;
+    if ((rc = check_sasa_overflow(e, flags, st[e->n_sys]))) return rc;
     for (int s = 0; s < e->n_sys; ++s)
         if (st[s]) return fail(OG_ERR_NONFINITE, "system %d: %s", s, status_reason(st[s]));
     if (f_out) {
-        for (size_t k = 0; k < 3 * (size_t)e->n_atoms; ++k)
-            if (!std::isfinite(f_out[k])) return fail(OG_ERR_NONFINITE, "non-finite force at component %zu", k);
+        const size_t bad = first_nonfinite(f_out, n3);
+        if (bad < n3) return fail(OG_ERR_NONFINITE, "non-finite force at component %zu", bad);
     }
     return OG_OK;
 }
@@ -1362,24 +1437,26 @@ static int run_steps(og_engine* e, int32_t n_steps, long long* ke_dev, bool allo
 }
 
 // After a run: SASA status, then OG_ERR_NONFINITE naming the first stopped
-// system (the diverged flags are read in chunks on the stack).
+// system (the diverged flags come through the staging buffer).
 static int run_status(og_engine* e) {
+    int* st = e->stage_i;                          // [S] stop reasons, then the SASA overflow count
+    og_publish_args p{};
+    publish_add(p, 0, e->diverged, st, (size_t)e->n_sys * sizeof(int));
+    if (e->dyn.flags & OG_SASA) publish_add(p, 1, e->sasa.overflow, st + e->n_sys, sizeof(int));
+    else st[e->n_sys] = 0;
+    og_launch_publish(p, e->stream);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(e->stream));
     if (e->prof) prof_collect(e);
     int ovf = 0;
-    if ((e->dyn.flags & OG_SASA) && og_sasa_overflow(&e->sasa, &ovf) != 0)
+    if (st[e->n_sys] != 0 && og_sasa_overflow(&e->sasa, &ovf) != 0)
         return fail(OG_ERR_HIP, "reading SASA status failed");
     int n_div = 0, first = -1, first_bits = 0;
-    int chunk[256];
-    for (int s0 = 0; s0 < e->n_sys; s0 += 256) {
-        const int m = std::min(256, e->n_sys - s0);
-        HIPCHK(hipMemcpy(chunk, e->diverged + s0, (size_t)m * sizeof(int), hipMemcpyDeviceToHost));
-        for (int k = 0; k < m; ++k)
-            if (chunk[k]) {
-                n_div++;
-                if (first < 0) { first = s0 + k; first_bits = chunk[k]; }
-            }
-    }
+    for (int s = 0; s < e->n_sys; ++s)
+        if (st[s]) {
+            n_div++;
+            if (first < 0) { first = s; first_bits = st[s]; }
+        }
     if (n_div)
         return fail(OG_ERR_NONFINITE, "%d system(s) stopped; system %d: %s (the others ran all steps)", n_div,
                     first, status_reason(first_bits));
@@ -1412,9 +1489,9 @@ extern "C" int og_run(og_engine* e, int32_t n_steps, double* ke_per_step) {
         return rc;
     }
     if (ke_dev) {
-        HIPCHK(hipMemcpyAsync(ke_per_step, ke_dev, n_ke * sizeof(long long), hipMemcpyDeviceToHost, e->stream));
+        const int rc = fetch(e, ke_per_step, ke_dev, n_ke * sizeof(long long));
         HIPCHK(hipFreeAsync(ke_dev, e->stream));
-        HIPCHK(hipStreamSynchronize(e->stream));
+        if (rc) return rc;
         ke_to_double(ke_per_step, n_ke);
     }
     return run_status(e);
@@ -1467,8 +1544,7 @@ extern "C" int og_run_noalloc(og_engine* e, int32_t n_steps, double* ke_per_step
     }
     if (int rc = run_steps(e, n_steps, ke_dev, false)) return rc;
     if (ke_dev) {
-        HIPCHK(hipMemcpyAsync(ke_per_step, ke_dev, n_ke * sizeof(long long), hipMemcpyDeviceToHost, e->stream));
-        HIPCHK(hipStreamSynchronize(e->stream));
+        if (int rc = fetch(e, ke_per_step, ke_dev, n_ke * sizeof(long long))) return rc;
         ke_to_double(ke_per_step, n_ke);
     }
     return run_status(e);
@@ -1637,18 +1713,21 @@ extern "C" int og_minimize(og_engine* e, const og_minimize_params* prm, og_minim
     int rc = OG_OK;
     auto run = [&]() -> int {
         HIPCHK(hipMemcpy(ip, off.data(), (S + 1) * sizeof(int), hipMemcpyHostToDevice));
+        auto clear = [&](long long* eacc) {
+            og_begin_args bg{};
+            bg.facc = e->facc; bg.iacc = e->iacc; bg.n_atoms = e->n_atoms;
+            bg.eacc = eacc; bg.sflag = e->sflag; bg.n_sys = S;
+            og_launch_begin(bg, e->stream);
+        };
         auto energies = [&](bool probes) -> int {
-            HIPCHK(hipMemsetAsync(e->eacc, 0, (size_t)S * OG_NE * sizeof(long long), e->stream));
-            HIPCHK(hipMemsetAsync(e->sflag, 0, (size_t)S * sizeof(int), e->stream));
-            og_launch_zero_acc(e->facc, e->iacc, e->n_atoms, e->stream);
+            clear(e->eacc);
             e->eval_skip = probes ? a.skip : nullptr;
             const int r = launch_forces(e, P.flags | OG_ENERGY, P.cutoff_a, P.sasa_gamma_scale, true, -1, false);
             e->eval_skip = nullptr;
             return r;
         };
         auto forces = [&]() -> int {
-            HIPCHK(hipMemsetAsync(e->sflag, 0, (size_t)S * sizeof(int), e->stream));
-            og_launch_zero_acc(e->facc, e->iacc, e->n_atoms, e->stream);
+            clear(nullptr);
             if (int r = launch_forces(e, P.flags & ~OG_ENERGY, P.cutoff_a, P.sasa_gamma_scale, false, -1, true)) return r;
             og_back_args b{};
             b.pos = e->pos; b.vel = e->vel; b.force = e->force; b.facc = e->facc; b.mass = e->mass;
@@ -1810,9 +1889,17 @@ extern "C" int og_swap_systems(og_engine* e, int32_t a, int32_t b) {
 
 extern "C" int og_get_status(og_engine* e, int32_t* div, int32_t* fails, int32_t* clamped) {
     if (!e) return fail(OG_ERR_ARG, "engine is NULL");
-    if (div) HIPCHK(hipMemcpy(div, e->diverged, e->n_sys * sizeof(int), hipMemcpyDeviceToHost));
-    if (fails) HIPCHK(hipMemcpy(fails, e->shake_fail, e->n_sys * sizeof(int), hipMemcpyDeviceToHost));
-    if (clamped) HIPCHK(hipMemcpy(clamped, e->clamped, e->n_sys * sizeof(int), hipMemcpyDeviceToHost));
+    const size_t n = e->n_sys, bytes = n * sizeof(int);
+    og_publish_args p{};
+    if (div) publish_add(p, 0, e->diverged, e->stage_i, bytes);
+    if (fails) publish_add(p, 1, e->shake_fail, e->stage_i + n, bytes);
+    if (clamped) publish_add(p, 2, e->clamped, e->stage_i + 2 * n, bytes);
+    og_launch_publish(p, e->stream);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(e->stream));
+    if (div) std::memcpy(div, e->stage_i, bytes);
+    if (fails) std::memcpy(fails, e->stage_i + n, bytes);
+    if (clamped) std::memcpy(clamped, e->stage_i + 2 * n, bytes);
     return OG_OK;
 }
 

@@ -410,6 +410,8 @@ __device__ __forceinline__ bool back_atom(const og_back_args& a, int i, int sys,
         }
     }
     for (int d = 0; d < 3; ++d) a.force[3 * (size_t)i + d] = f[d];
+    if (a.force_out)
+        for (int d = 0; d < 3; ++d) a.force_out[3 * (size_t)i + d] = f[d];
     // a summed force at or beyond the contribution limit: the int64 sum may
     // have wrapped, so the system is reported as out of range
     if (big && a.sflag) atomicOr(a.sflag + sys, OG_ST_RANGE);

@@ -144,6 +144,43 @@ void og_launch_zero_acc(long long* facc, long long* iacc, int n_atoms, hipStream
     hipLaunchKernelGGL(og_k_zero_acc, dim3((n_atoms + 255) / 256), dim3(256), 0, s, facc, iacc, n_atoms);
 }
 
+// One launch where separate copies and fills of a few KB would each cost as
+// much as a kernel of the evaluation.
+__global__ void __launch_bounds__(256) og_k_begin(og_begin_args a) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, n = gridDim.x * blockDim.x;
+    for (int k = i; k < 3 * a.n_atoms; k += n) {
+        if (a.xyz) a.pos[k] = a.xyz[k];
+        a.facc[k] = 0;
+    }
+    for (int k = i; k < a.n_atoms; k += n) a.iacc[k] = 0;
+    for (int k = i; k < a.n_sys; k += n) {
+        a.sflag[k] = 0;
+        if (a.clamped) a.clamped[k] = 0;
+    }
+    if (a.eacc)
+        for (int k = i; k < a.n_sys * OG_NE; k += n) a.eacc[k] = 0;
+}
+
+void og_launch_begin(const og_begin_args& a, hipStream_t s) {
+    int g = (3 * a.n_atoms + 255) / 256;
+    if (g > 4096) g = 4096;
+    hipLaunchKernelGGL(og_k_begin, dim3(g), dim3(256), 0, s, a);
+}
+
+__global__ void __launch_bounds__(256) og_k_publish(og_publish_args a) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, n = gridDim.x * blockDim.x;
+    for (int q = 0; q < 4; ++q)
+        for (int k = i; k < a.n[q]; k += n) a.dst[q][k] = a.src[q][k];
+}
+
+void og_launch_publish(const og_publish_args& a, hipStream_t s) {
+    int m = 1;
+    for (int q = 0; q < 4; ++q) m = a.n[q] > m ? a.n[q] : m;
+    int g = (m + 255) / 256;
+    if (g > 1024) g = 1024;
+    hipLaunchKernelGGL(og_k_publish, dim3(g), dim3(256), 0, s, a);
+}
+
 // ---------------------------------------------------------------------------
 // Finalise forces (fixed point -> FP64), second half-kick, kinetic energy,
 // divergence flag (langevin.rs:309-319).

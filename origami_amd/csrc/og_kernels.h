@@ -132,6 +132,29 @@ struct og_tunnel_dev {
     int on;
 };
 
+// Start of a force or energy evaluation: positions from the caller's staging
+// buffer (pinned host memory, may be null) and every accumulator cleared.
+struct og_begin_args {
+    const double* xyz;               // [3N] or null (positions stay)
+    double* pos;
+    long long* facc; long long* iacc;
+    int n_atoms;
+    long long* eacc;                 // [S*OG_NE] or null
+    int* sflag;                      // [S]
+    int* clamped;                    // [S] or null
+    int n_sys;
+};
+void og_launch_begin(const og_begin_args& a, hipStream_t s);
+
+// Device words copied into pinned host memory (or between buffers) by one
+// launch; unused entries have n = 0.
+struct og_publish_args {
+    const uint32_t* src[4];
+    uint32_t* dst[4];
+    int n[4];
+};
+void og_launch_publish(const og_publish_args& a, hipStream_t s);
+
 struct og_back_args {
     const double* pos;               // read for the external tunnel only
     double* vel; double* force;
@@ -147,6 +170,7 @@ struct og_back_args {
     int* sflag;                      // [S] status bits of this evaluation: with do_kick, a flagged
                                      //   system gets them in diverged and is not kicked
     og_tunnel_dev tun;               // added to every atom's force when tun.on
+    double* force_out;               // if set: the forces, in pinned host memory, too
 };
 
 void og_launch_pair_descreen(const og_pair_args& a, bool mode_a, hipStream_t s);

@@ -232,7 +232,7 @@ class Engine:
         return dict(zip(keys, [int(x) for x in out]))
 
     def _state(self, getter):
-        out = np.zeros((self.n_atoms, 3))
+        out = np.empty((self.n_atoms, 3))
         _check(getter(self._h, _d(out)))
         return out
 
@@ -263,7 +263,7 @@ class Engine:
         (total_force_with_scratch's cutoff_a, forces.rs:82); otherwise all pairs."""
         flags = ((MODE_A if mode_a else 0) | (SASA if include_sasa else 0)
                  | (SURROGATE if surrogate else 0))
-        f = np.zeros((self.n_atoms, 3))
+        f = np.empty((self.n_atoms, 3))
         e = np.zeros((self.n_systems, len(ENERGY_TERMS))) if energies else None
         x = None
         if xyz is not None:
