@@ -1697,6 +1697,7 @@ extern "C" int og_minimize(og_engine* e, const og_minimize_params* prm, og_minim
     a.n_sys = S;
     a.n_atoms = e->n_atoms;
     a.history = P.history;
+    a.max_n3 = 3 * *std::max_element(e->sys_n.begin(), e->sys_n.end());
     double* d = (double*)ws;
     a.x0 = d; a.g = d + n3; a.p = d + 2 * n3;
     a.hs = d + 3 * n3; a.hy = a.hs + hist_n;

@@ -76,6 +76,80 @@ __global__ void og_k_lb_init(og_lbfgs_args a) {
     }
 }
 
+// The start of an iteration for one system.  E > 0: the direction is held in
+// registers, E degrees of freedom per thread (k = tid + 256 u, the order in
+// which the strided loops of E = 0 add), and the history vectors of the next
+// pass of the two-loop recursion load while the block sum of this one runs.
+// With the strided loops a pass waits for one load after another (the vectors
+// come from L2, and the stores to p keep the loads behind them from moving
+// up): 87 us at 1 425 atoms and up to 10 pairs, 37 us this way; both forms have the
+// same products and sums in the same order.
+template <int E>
+__device__ void lb_direction(const og_lbfgs_args& a, const og_lb_sys& st, const SysView& v, int s, double* red,
+                             double* alph) {
+    const int tid = threadIdx.x, m = st.count;
+    double* pg = a.p + v.base;
+    const double* gg = a.g + v.base;
+    auto slot_of = [&](int i) { return (st.head + i) % a.history; };
+    auto load = [&](double (&x)[E], const double* src) {
+#pragma unroll
+        for (int u = 0; u < E; ++u) x[u] = tid + kThreads * u < v.n3 ? src[tid + kThreads * u] : 0.0;
+    };
+    double p[E], sv[E], yv[E];
+    load(p, gg);
+    // two_loop_recursion (lbfgs.rs:212-254), q and r in p; logical entry i
+    // (0 = oldest) sits in ring slot (head + i) % history
+    load(sv, hist(a.hs, a, slot_of(m - 1), v.base));
+    double a_prev = 0.0;
+    for (int i = m - 1; i >= 0; --i) {
+        const int slot = slot_of(i);
+        double acc = 0.0;
+#pragma unroll
+        for (int u = 0; u < E; ++u) {
+            if (i < m - 1) p[u] = fma(-a_prev, yv[u], p[u]);
+            acc = fma(sv[u], p[u], acc);
+        }
+        load(yv, hist(a.hy, a, slot, v.base));
+        if (i > 0) load(sv, hist(a.hs, a, slot_of(i - 1), v.base));
+        const double ai = a.rho[s * OG_LB_MAX_HISTORY + slot] * block_sum(acc, red);
+        if (tid == 0) alph[i] = ai;
+        a_prev = ai;
+    }
+    double sl[E], yl[E];
+    load(sl, hist(a.hs, a, slot_of(m - 1), v.base));
+    load(yl, hist(a.hy, a, slot_of(m - 1), v.base));
+    double sy = 0.0, yy = 0.0;
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+        p[u] = fma(-a_prev, yv[u], p[u]);
+        sy = fma(sl[u], yl[u], sy);
+        yy = fma(yl[u], yl[u], yy);
+    }
+    load(yv, hist(a.hy, a, slot_of(0), v.base));
+    sy = block_sum(sy, red);
+    yy = block_sum(yy, red);
+    const double gamma = yy > 0.0 ? sy / yy : 1.0;
+    __syncthreads();
+    double coef_prev = 0.0;
+    for (int i = 0; i < m; ++i) {
+        const int slot = slot_of(i);
+        double acc = 0.0;
+#pragma unroll
+        for (int u = 0; u < E; ++u) {
+            p[u] = i == 0 ? gamma * p[u] : fma(coef_prev, sv[u], p[u]);
+            acc = fma(yv[u], p[u], acc);
+        }
+        load(sv, hist(a.hs, a, slot, v.base));
+        if (i + 1 < m) load(yv, hist(a.hy, a, slot_of(i + 1), v.base));
+        const double beta = a.rho[s * OG_LB_MAX_HISTORY + slot] * block_sum(acc, red);
+        coef_prev = alph[i] - beta;
+    }
+#pragma unroll
+    for (int u = 0; u < E; ++u)
+        if (tid + kThreads * u < v.n3) pg[tid + kThreads * u] = -fma(coef_prev, sv[u], p[u]);
+}
+
+template <int E>
 __global__ void __launch_bounds__(kThreads) og_k_lb_begin(og_lbfgs_args a, int step) {
     __shared__ double red[kThreads / 64];
     __shared__ double alph[OG_LB_MAX_HISTORY];
@@ -88,9 +162,11 @@ __global__ void __launch_bounds__(kThreads) og_k_lb_begin(og_lbfgs_args a, int s
     double* p = a.p + v.base;
     const double* f = a.force + v.base;
     double mx = 0.0;
+#pragma unroll 4
     for (int k = tid; k < v.n3; k += kThreads) {
-        g[k] = -f[k];
-        mx = fmax(mx, fabs(f[k]));
+        const double fk = f[k];
+        g[k] = -fk;
+        mx = fmax(mx, fabs(fk));
     }
     const double maxf = block_max(mx, red);
     if (tid == 0) {
@@ -104,6 +180,8 @@ __global__ void __launch_bounds__(kThreads) og_k_lb_begin(og_lbfgs_args a, int s
     const int m = st.count;
     if (m == 0) {
         for (int k = tid; k < v.n3; k += kThreads) p[k] = -g[k];
+    } else if constexpr (E > 0) {
+        lb_direction<E>(a, st, v, s, red, alph);
     } else {
         // two_loop_recursion (lbfgs.rs:212-254), q and r in p; logical entry i
         // (0 = oldest) sits in ring slot (head + i) % history
@@ -116,9 +194,9 @@ __global__ void __launch_bounds__(kThreads) og_k_lb_begin(og_lbfgs_args a, int s
             double acc = 0.0;
             for (int k = tid; k < v.n3; k += kThreads) {
                 double q = p[k];
-                if (y_prev) q -= a_prev * y_prev[k];
+                if (y_prev) q = fma(-a_prev, y_prev[k], q);
                 p[k] = q;
-                acc += si[k] * q;
+                acc = fma(si[k], q, acc);
             }
             const double ai = a.rho[s * OG_LB_MAX_HISTORY + slot] * block_sum(acc, red);
             if (tid == 0) alph[i] = ai;
@@ -130,10 +208,10 @@ __global__ void __launch_bounds__(kThreads) og_k_lb_begin(og_lbfgs_args a, int s
         const double* yl = hist(a.hy, a, last, v.base);
         double sy = 0.0, yy = 0.0;
         for (int k = tid; k < v.n3; k += kThreads) {
-            const double q = p[k] - a_prev * y_prev[k];
+            const double q = fma(-a_prev, y_prev[k], p[k]);
             p[k] = q;
-            sy += sl[k] * yl[k];
-            yy += yl[k] * yl[k];
+            sy = fma(sl[k], yl[k], sy);
+            yy = fma(yl[k], yl[k], yy);
         }
         sy = block_sum(sy, red);
         yy = block_sum(yy, red);
@@ -146,21 +224,23 @@ __global__ void __launch_bounds__(kThreads) og_k_lb_begin(og_lbfgs_args a, int s
             const double* yi = hist(a.hy, a, slot, v.base);
             double acc = 0.0;
             for (int k = tid; k < v.n3; k += kThreads) {
-                double r = (i == 0) ? gamma * p[k] : p[k] + coef_prev * s_prev[k];
+                double r = (i == 0) ? gamma * p[k] : fma(coef_prev, s_prev[k], p[k]);
                 p[k] = r;
-                acc += yi[k] * r;
+                acc = fma(yi[k], r, acc);
             }
             const double beta = a.rho[s * OG_LB_MAX_HISTORY + slot] * block_sum(acc, red);
             coef_prev = alph[i] - beta;
             s_prev = hist(a.hs, a, slot, v.base);
         }
-        for (int k = tid; k < v.n3; k += kThreads) p[k] = -(p[k] + coef_prev * s_prev[k]);
+        for (int k = tid; k < v.n3; k += kThreads) p[k] = -fma(coef_prev, s_prev[k], p[k]);
     }
     __syncthreads();
     double mp = 0.0, gp = 0.0;
+#pragma unroll 4
     for (int k = tid; k < v.n3; k += kThreads) {
-        mp = fmax(mp, fabs(p[k]));
-        gp += p[k] * g[k];
+        const double pk = p[k];
+        mp = fmax(mp, fabs(pk));
+        gp = fma(pk, g[k], gp);
         a.x0[v.base + k] = a.pos[v.base + k];
     }
     const double maxp = block_max(mp, red);
@@ -328,7 +408,14 @@ void og_launch_lbfgs(int phase, const og_lbfgs_args& a, int step, hipStream_t s)
         hipLaunchKernelGGL(og_k_lb_init, dim3(1), dim3(kThreads), 0, s, a);
         break;
     case OG_LB_K_BEGIN:
-        hipLaunchKernelGGL(og_k_lb_begin, dim3(a.n_sys), dim3(kThreads), 0, s, a, step);
+        // registers for the largest system of the batch, up to 64 degrees of
+        // freedom per thread (5 461 atoms)
+        if (a.max_n3 <= 8 * kThreads) hipLaunchKernelGGL(og_k_lb_begin<8>, dim3(a.n_sys), dim3(kThreads), 0, s, a, step);
+        else if (a.max_n3 <= 20 * kThreads)
+            hipLaunchKernelGGL(og_k_lb_begin<20>, dim3(a.n_sys), dim3(kThreads), 0, s, a, step);
+        else if (a.max_n3 <= 64 * kThreads)
+            hipLaunchKernelGGL(og_k_lb_begin<64>, dim3(a.n_sys), dim3(kThreads), 0, s, a, step);
+        else hipLaunchKernelGGL(og_k_lb_begin<0>, dim3(a.n_sys), dim3(kThreads), 0, s, a, step);
         break;
     case OG_LB_K_TRIAL:
         hipLaunchKernelGGL(og_k_lb_trial, dim3(a.n_sys), dim3(kThreads), 0, s, a);

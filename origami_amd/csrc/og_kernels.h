@@ -244,6 +244,7 @@ struct og_lb_sys {                 // one system's minimiser state
 
 struct og_lbfgs_args {
     int n_sys, n_atoms, history;
+    int max_n3;                    // degrees of freedom of the largest system
     const int* atom_off;           // [S+1]
     double* pos;                   // engine positions (trial points are written here)
     const double* force;           // engine forces (FP64, after the last force evaluation)

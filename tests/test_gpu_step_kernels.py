@@ -111,3 +111,19 @@ def test_sasa_terms_forms_agree(E, chains):
     assert np.array_equal(a, b)
     ref = np.concatenate([O.Oracle(s).sasa_forces(p)[0] for s, p in zip(systems, x)])
     assert np.abs(a - ref).max() < 1e-8
+
+
+@pytest.mark.parametrize("chains", [[(3, 3)], [(2, 40)], [(2, 70)], [(2, 70), (3, 3)]])
+def test_minimiser_direction_forms_agree(E, chains):
+    """The L-BFGS direction with its vectors in registers (a form per system
+    size) equals the strided form: a system's iterates do not depend on the
+    largest system beside it (5 462 atoms and more select the strided form)."""
+    from origami_amd.minimize import minimize_device
+    systems = [S.seeded_chain(*c) for c in chains]
+    big = S.seeded_chain(5, 340)
+    assert big.n_atoms > 64 * 256 // 3
+    n = sum(s.n_atoms for s in systems)
+    alone, beside = E.Engine(systems), E.Engine(systems + [big])
+    for eng in (alone, beside):
+        minimize_device(eng, max_steps=14, mode_a=True)
+    assert np.array_equal(alone.positions(), beside.positions()[:n])
