@@ -888,6 +888,16 @@ static og_pair_args pair_args(og_engine* e, double cutoff_a) {
     return a;
 }
 
+static og_energy64_args energy_args(const og_engine* e, double cutoff_a) {
+    og_energy64_args en{};
+    en.charge = e->charge; en.eps = e->eps; en.rmin = e->rmin; en.eps14 = e->eps14;
+    en.rmin14 = e->rmin14; en.radii = e->radii;
+    en.rc2_nb = cutoff_a * cutoff_a;
+    en.kappa = 1.0 / (2.0 * cutoff_a * cutoff_a * cutoff_a);
+    en.crf = 3.0 / (2.0 * cutoff_a);
+    return en;
+}
+
 // The LJ / Coulomb cutoff of a call: cutoff_a under OG_MODE_A (finite and
 // positive), none otherwise (the value is then not used).
 static int check_cutoff(uint32_t flags, double cutoff_a) {
@@ -948,7 +958,10 @@ static int launch_forces(og_engine* e, uint32_t flags, double cutoff_a, double s
     const bool lean = !energy && !sur && !e->prof;
     const bool wide = lean && forces && e->n_tile_pairs <= OG_WIDE_FORCE_MAX;
     const bool wide_d = wide && e->n_work <= OG_WIDE_DESCREEN_MAX;
-    const bool fuse = wide || (lean && e->n_atoms < OG_GATHER_LDS_MAX_ATOMS);
+    // energies only, the same way
+    const bool wide_e = energy && !forces && !sur && !e->prof &&
+                        e->n_work <= OG_WIDE_ENERGY_MAX && e->nb + e->na + e->nd + e->ni > 0;
+    const bool fuse = wide_e || wide || (lean && e->n_atoms < OG_GATHER_LDS_MAX_ATOMS);
     og_bonded_args b{};
     {
         ProfScope p(e, OG_K_BONDED);
@@ -985,7 +998,7 @@ static int launch_forces(og_engine* e, uint32_t flags, double cutoff_a, double s
         ProfScope p(e, OG_K_DESCREEN);
         og_pair_args ad = a;
         ad.skip_sys = (sur && !check) ? sur->mode : (!forces ? e->eval_skip : nullptr);
-        if (wide_d) og_launch_wide_descreen(ad, b, mode_a, e->stream);
+        if (wide_d || wide_e) og_launch_wide_descreen(ad, b, mode_a, wide_e, e->stream);
         else if (fuse) og_launch_descreen_bonded(ad, b, mode_a, e->stream);
         else og_launch_pair_descreen(ad, mode_a, e->stream);
     }
@@ -997,7 +1010,11 @@ static int launch_forces(og_engine* e, uint32_t flags, double cutoff_a, double s
         r.eacc = e->eacc; r.n_atoms = e->n_atoms;
         r.sflag = e->sflag;
         if (sur) { r.sur_mode = sur->mode; r.r_sur = sur->r_sur; r.dev = sur->dev; r.check = check ? 1 : 0; }
-        if (wide) og_launch_wide_force(a, r, b, mode_a, e->stream);
+        if (wide_e) {
+            og_pair_args ae = a;
+            ae.skip_sys = e->eval_skip;
+            og_launch_wide_energy(ae, energy_args(e, cutoff_a), r, b, mode_a, e->stream);
+        } else if (wide) og_launch_wide_force(a, r, b, mode_a, e->stream);
         else if (fuse) og_launch_radii_gather(r, b, e->stream);
         else og_launch_radii(r, energy, e->stream);
         if (sur && check && og_sur_check_apply(sur)) {
@@ -1011,15 +1028,9 @@ static int launch_forces(og_engine* e, uint32_t flags, double cutoff_a, double s
     }
     if (energy) {
         ProfScope p(e, OG_K_OTHER);
-        og_energy64_args en{};
-        en.charge = e->charge; en.eps = e->eps; en.rmin = e->rmin; en.eps14 = e->eps14;
-        en.rmin14 = e->rmin14; en.radii = e->radii;
-        en.rc2_nb = cutoff_a * cutoff_a;
-        en.kappa = 1.0 / (2.0 * cutoff_a * cutoff_a * cutoff_a);
-        en.crf = 3.0 / (2.0 * cutoff_a);
         og_pair_args ae = a;
         ae.skip_sys = forces ? nullptr : e->eval_skip;
-        og_launch_pair_energy64(ae, en, mode_a, e->stream);
+        if (!wide_e) og_launch_pair_energy64(ae, energy_args(e, cutoff_a), mode_a, e->stream);
         if (flags & OG_SASA_SR) {
             const int rc = og_sasa_sr_launch(&e->sasa, e->pos, e->sr_dots, OG_SR_DOTS, e->stream, e->eacc,
                                              e->atom_sys, e->sflag);
@@ -1744,12 +1755,14 @@ extern "C" int og_minimize(og_engine* e, const og_minimize_params* prm, og_minim
             HIPCHK(hipStreamSynchronize(e->stream));
             return OG_OK;
         };
+        auto probe = [&]() -> int {
+            og_launch_lbfgs(OG_LB_K_TRIAL, a, 0, e->stream);
+            if (int r = energies(true)) return r;
+            return read_counts(OG_LB_K_ACCEPT);
+        };
         auto probes = [&]() -> int {
-            while (cnt[0] > 0) {
-                og_launch_lbfgs(OG_LB_K_TRIAL, a, 0, e->stream);
-                if (int r = energies(true)) return r;
-                if (int r = read_counts(OG_LB_K_ACCEPT)) return r;
-            }
+            while (cnt[0] > 0)
+                if (int r = probe()) return r;
             return OG_OK;
         };
         if (int r = energies(false)) return r;
@@ -1758,9 +1771,12 @@ extern "C" int og_minimize(og_engine* e, const og_minimize_params* prm, og_minim
             if (int r = forces()) return r;
         for (int step = 0; step < P.max_steps; ++step) {
             og_launch_lbfgs(OG_LB_K_BEGIN, a, step, e->stream);
-            if (int r = read_counts(OG_LB_K_COUNT)) return r;
-            if (cnt[0] == 0 && cnt[1] == 0) break;          // every system converged or stopped
+            // the first probe goes out with the direction, before the host
+            // knows whether any system searches (nearly always one does; if
+            // none, the probe evaluates nothing): one wait less per iteration
+            if (int r = probe()) return r;
             if (int r = probes()) return r;
+            if (cnt[1] == 0 && cnt[3] == 0) break;          // every system converged or stopped
             if (cnt[1] > 0) {                               // steepest-descent retries
                 og_launch_lbfgs(OG_LB_K_FALLBACK, a, 0, e->stream);
                 if (int r = read_counts(OG_LB_K_COUNT)) return r;

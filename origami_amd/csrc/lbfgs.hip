@@ -23,6 +23,7 @@
 namespace {
 
 constexpr int kThreads = 256;
+#define LB_CHUNK 16                     // values per thread of a chunk in the memory form of the direction
 
 // deterministic block sum / max (every thread gets the result)
 __device__ double block_sum(double v, double* red) {
@@ -78,12 +79,12 @@ __global__ void og_k_lb_init(og_lbfgs_args a) {
 
 // The start of an iteration for one system.  E > 0: the direction is held in
 // registers, E degrees of freedom per thread (k = tid + 256 u, the order in
-// which the strided loops of E = 0 add), and the history vectors of the next
-// pass of the two-loop recursion load while the block sum of this one runs.
-// With the strided loops a pass waits for one load after another (the vectors
-// come from L2, and the stores to p keep the loads behind them from moving
-// up): 87 us at 1 425 atoms and up to 10 pairs, 37 us this way; both forms have the
-// same products and sums in the same order.
+// which the chunks of E = 0 add), and the history vectors of the next pass of
+// the two-loop recursion load while the block sum of this one runs.  What
+// bounds the kernel is the latency of those loads (the vectors come from L2):
+// as plain strided loops each load waited for the one before, because the
+// stores to p kept later loads from moving up.  Both forms have the same
+// products and sums in the same order.
 template <int E>
 __device__ void lb_direction(const og_lbfgs_args& a, const og_lb_sys& st, const SysView& v, int s, double* red,
                              double* alph) {
@@ -155,7 +156,9 @@ __global__ void __launch_bounds__(kThreads) og_k_lb_begin(og_lbfgs_args a, int s
     __shared__ double alph[OG_LB_MAX_HISTORY];
     const int s = blockIdx.x;
     og_lb_sys& st = a.sys[s];
-    if (st.state != OG_LB_ACTIVE) return;
+    const bool active = st.state == OG_LB_ACTIVE;
+    if (threadIdx.x == 0) a.skip[s] = 1;       // until this system searches
+    if (!active) return;
     const SysView v = view(a, s);
     const int tid = threadIdx.x;
     double* g = a.g + v.base;
@@ -183,20 +186,35 @@ __global__ void __launch_bounds__(kThreads) og_k_lb_begin(og_lbfgs_args a, int s
     } else if constexpr (E > 0) {
         lb_direction<E>(a, st, v, s, red, alph);
     } else {
-        // two_loop_recursion (lbfgs.rs:212-254), q and r in p; logical entry i
-        // (0 = oldest) sits in ring slot (head + i) % history
-        for (int k = tid; k < v.n3; k += kThreads) p[k] = g[k];
+        // larger systems: p in memory, LB_CHUNK values per thread at a time so
+        // that a chunk's loads are in flight together
+        double q[LB_CHUNK], x[LB_CHUNK], y[LB_CHUNK];
+        auto load = [&](double (&d)[LB_CHUNK], const double* src, int k0) {
+#pragma unroll
+            for (int u = 0; u < LB_CHUNK; ++u) d[u] = k0 + kThreads * u < v.n3 ? src[k0 + kThreads * u] : 0.0;
+        };
+        auto store = [&](int k0) {
+#pragma unroll
+            for (int u = 0; u < LB_CHUNK; ++u)
+                if (k0 + kThreads * u < v.n3) p[k0 + kThreads * u] = q[u];
+        };
+        constexpr int stride = kThreads * LB_CHUNK;
         double a_prev = 0.0;
         const double* y_prev = nullptr;
         for (int i = m - 1; i >= 0; --i) {
             const int slot = (st.head + i) % a.history;
             const double* si = hist(a.hs, a, slot, v.base);
             double acc = 0.0;
-            for (int k = tid; k < v.n3; k += kThreads) {
-                double q = p[k];
-                if (y_prev) q = fma(-a_prev, y_prev[k], q);
-                p[k] = q;
-                acc = fma(si[k], q, acc);
+            for (int k0 = tid; k0 < v.n3; k0 += stride) {
+                load(q, y_prev ? p : g, k0);
+                load(x, si, k0);
+                if (y_prev) load(y, y_prev, k0);
+#pragma unroll
+                for (int u = 0; u < LB_CHUNK; ++u) {
+                    if (y_prev) q[u] = fma(-a_prev, y[u], q[u]);
+                    acc = fma(x[u], q[u], acc);
+                }
+                store(k0);
             }
             const double ai = a.rho[s * OG_LB_MAX_HISTORY + slot] * block_sum(acc, red);
             if (tid == 0) alph[i] = ai;
@@ -207,11 +225,14 @@ __global__ void __launch_bounds__(kThreads) og_k_lb_begin(og_lbfgs_args a, int s
         const double* sl = hist(a.hs, a, last, v.base);
         const double* yl = hist(a.hy, a, last, v.base);
         double sy = 0.0, yy = 0.0;
-        for (int k = tid; k < v.n3; k += kThreads) {
-            const double q = fma(-a_prev, y_prev[k], p[k]);
-            p[k] = q;
-            sy = fma(sl[k], yl[k], sy);
-            yy = fma(yl[k], yl[k], yy);
+        for (int k0 = tid; k0 < v.n3; k0 += stride) {
+            load(x, sl, k0);
+            load(y, yl, k0);
+#pragma unroll
+            for (int u = 0; u < LB_CHUNK; ++u) {
+                sy = fma(x[u], y[u], sy);
+                yy = fma(y[u], y[u], yy);
+            }
         }
         sy = block_sum(sy, red);
         yy = block_sum(yy, red);
@@ -223,16 +244,28 @@ __global__ void __launch_bounds__(kThreads) og_k_lb_begin(og_lbfgs_args a, int s
             const int slot = (st.head + i) % a.history;
             const double* yi = hist(a.hy, a, slot, v.base);
             double acc = 0.0;
-            for (int k = tid; k < v.n3; k += kThreads) {
-                double r = (i == 0) ? gamma * p[k] : fma(coef_prev, s_prev[k], p[k]);
-                p[k] = r;
-                acc = fma(yi[k], r, acc);
+            for (int k0 = tid; k0 < v.n3; k0 += stride) {
+                load(q, p, k0);
+                load(x, i == 0 ? y_prev : s_prev, k0);       // i == 0: y_0 finishes the first loop's update
+                load(y, yi, k0);
+#pragma unroll
+                for (int u = 0; u < LB_CHUNK; ++u) {
+                    q[u] = i == 0 ? gamma * fma(-a_prev, x[u], q[u]) : fma(coef_prev, x[u], q[u]);
+                    acc = fma(y[u], q[u], acc);
+                }
+                store(k0);
             }
             const double beta = a.rho[s * OG_LB_MAX_HISTORY + slot] * block_sum(acc, red);
             coef_prev = alph[i] - beta;
             s_prev = hist(a.hs, a, slot, v.base);
         }
-        for (int k = tid; k < v.n3; k += kThreads) p[k] = -fma(coef_prev, s_prev[k], p[k]);
+        for (int k0 = tid; k0 < v.n3; k0 += stride) {
+            load(q, p, k0);
+            load(x, s_prev, k0);
+#pragma unroll
+            for (int u = 0; u < LB_CHUNK; ++u) q[u] = -fma(coef_prev, x[u], q[u]);
+            store(k0);
+        }
     }
     __syncthreads();
     double mp = 0.0, gp = 0.0;
@@ -251,6 +284,7 @@ __global__ void __launch_bounds__(kThreads) og_k_lb_begin(og_lbfgs_args a, int s
         st.e_now = st.e_prev;
         st.phase = 0;
         st.state = pdg >= 0.0 ? OG_LB_FAILED : OG_LB_SEARCHING;   // not a descent direction
+        if (pdg < 0.0) a.skip[s] = 0;
     }
 }
 
@@ -408,13 +442,10 @@ void og_launch_lbfgs(int phase, const og_lbfgs_args& a, int step, hipStream_t s)
         hipLaunchKernelGGL(og_k_lb_init, dim3(1), dim3(kThreads), 0, s, a);
         break;
     case OG_LB_K_BEGIN:
-        // registers for the largest system of the batch, up to 64 degrees of
-        // freedom per thread (5 461 atoms)
+        // in registers up to 20 values per thread (1 706 atoms)
         if (a.max_n3 <= 8 * kThreads) hipLaunchKernelGGL(og_k_lb_begin<8>, dim3(a.n_sys), dim3(kThreads), 0, s, a, step);
         else if (a.max_n3 <= 20 * kThreads)
             hipLaunchKernelGGL(og_k_lb_begin<20>, dim3(a.n_sys), dim3(kThreads), 0, s, a, step);
-        else if (a.max_n3 <= 64 * kThreads)
-            hipLaunchKernelGGL(og_k_lb_begin<64>, dim3(a.n_sys), dim3(kThreads), 0, s, a, step);
         else hipLaunchKernelGGL(og_k_lb_begin<0>, dim3(a.n_sys), dim3(kThreads), 0, s, a, step);
         break;
     case OG_LB_K_TRIAL:

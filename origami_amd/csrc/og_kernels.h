@@ -206,9 +206,16 @@ void og_launch_bonded_terms(const og_bonded_args& a, hipStream_t s);
 //   to 4 tile pairs per CU in strips: 41 -> 29 at 21 tile pairs, 49 -> 33 at
 //   210, 54 -> 48 at 861; even at 1 326, 72 -> 90 at 2 850
 #define OG_WIDE_SPLIT_MAX 1024
+//   energies, up to 8 items per CU (us per call): 64 -> 36 at 6 tile pairs, 71
+//   -> 38 at 210, 117 -> 88 at 1 326; even at 2 136 (4 chains), 164 -> 190 at
+//   4 271
+#define OG_WIDE_ENERGY_MAX 2048
 #define OG_WIDE_FORCE_MAX 4864
 #define OG_WIDE_DESCREEN_MAX 512
-void og_launch_wide_descreen(const og_pair_args& a, const og_bonded_args& b, bool mode_a, hipStream_t s);
+void og_launch_wide_descreen(const og_pair_args& a, const og_bonded_args& b, bool mode_a, bool energy, hipStream_t s);
+struct og_energy64_args;
+void og_launch_wide_energy(const og_pair_args& a, const og_energy64_args& e, const og_radii_args& r,
+                           const og_bonded_args& b, bool mode_a, hipStream_t s);
 void og_launch_wide_force(const og_pair_args& a, const og_radii_args& r, const og_bonded_args& b, bool mode_a,
                           hipStream_t s);
 // Born radii (forces only, no surrogate) and the bonded gather's LDS form

@@ -287,4 +287,147 @@ __device__ __forceinline__ bool strip_far(const StripBound& b, const LaneData& d
     return rmn > 0.0f && rmn * rmn * (b.gw * gw_j) >= 33.0f;
 }
 
+// ---------------------------------------------------------------------------
+// FP64 pair energies (og_k_energy64, og_k_wide_energy)
+// ---------------------------------------------------------------------------
+// 1/sqrt(x) for x > 0 in FP64: the hardware estimate refined by two Newton
+// steps (each doubles the number of correct bits), in place of a correctly
+// rounded square root and division.
+__device__ __forceinline__ double rsqrt64(double x) {
+    double y = __builtin_amdgcn_rsq(x);
+    double h = x * y;
+    double e = fma(-h, y, 1.0);
+    y = fma(0.5 * y, e, y);
+    h = x * y;
+    e = fma(-h, y, 1.0);
+    return fma(0.5 * y, e, y);
+}
+
+// j atom data for the FP64 energy pass, one entry per j atom of the tile in
+// the wave's LDS: every lane reads the same entry in a step (a broadcast).
+struct EJ {
+    double x, y, z, q;
+    double rm, se, rm14, se14;     // Rmin/2, sqrt(eps), 1-4 variants
+    double R, iR;                  // Born radius and its reciprocal
+};
+
+
+// The lane's i atom.
+struct EI {
+    double x, y, z, q, rm, se, rm14, se14, R, iR;
+    bool valid;
+};
+struct ESum {
+    double lj, c, g;
+};
+
+__device__ __forceinline__ EI energy_i(const og_pair_args& a, const og_energy64_args& e, int gi, bool valid, double R) {
+    return {a.pos[3 * (size_t)gi], a.pos[3 * (size_t)gi + 1], a.pos[3 * (size_t)gi + 2], e.charge[gi], e.rmin[gi],
+            sqrt(e.eps[gi]), e.rmin14[gi], sqrt(e.eps14[gi]), R, 1.0 / R, valid};
+}
+
+__device__ __forceinline__ EJ energy_j(const og_pair_args& a, const og_energy64_args& e, int gj, double R) {
+    EJ m;
+    m.x = a.pos[3 * (size_t)gj]; m.y = a.pos[3 * (size_t)gj + 1]; m.z = a.pos[3 * (size_t)gj + 2];
+    m.q = e.charge[gj];
+    m.rm = e.rmin[gj]; m.se = sqrt(e.eps[gj]);
+    m.rm14 = e.rmin14[gj]; m.se14 = sqrt(e.eps14[gj]);
+    m.R = R; m.iR = 1.0 / R;
+    return m;
+}
+
+// j atoms [j0, j1) of an off-diagonal tile pair without excluded or 1-4
+// pairs: the terms with the mask and 1-4 selects left out.
+template <bool MODEA>
+__device__ __forceinline__ void energy_plain(const og_energy64_args& e, const EI& I, const EJ* J, int j0, int j1,
+                                             ESum& t) {
+    const double xo = I.valid ? I.x : I.x + 1.0e6;       // padding lanes: far away, added as 0
+    for (int jj = j0; jj < j1; ++jj) {
+        const EJ d = J[jj];
+        const double dx = xo - d.x, dy = I.y - d.y, dz = I.z - d.z;
+        const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+        const double qq = I.q * d.q;
+        const double inv_r = rsqrt64(r2);
+        const double s = (I.rm + d.rm) * inv_r;
+        const double t2 = s * s;
+        const double t6 = t2 * t2 * t2;
+        const double lj = (I.se * d.se) * fma(t6, t6, -2.0 * t6);
+        double c = qq * inv_r;
+        bool nb = I.valid;
+        if (MODEA) {
+            c = qq * (inv_r + e.kappa * r2 - e.crf);
+            nb = nb && (r2 <= e.rc2_nb);
+        }
+        t.lj += nb ? lj : 0.0;
+        t.c += nb ? c : 0.0;
+        // f_GB^2 = r^2 + R_i R_j exp(-x), x = r^2 / (4 R_i R_j).  From
+        // x >= 60 on, R_i R_j exp(-x) < 1e-12 x 2^-52 r^2 (r^2 = 4 x R_i R_j),
+        // far below half an ulp of r^2, so the fma rounds to r^2 exactly
+        // and 1/f_GB is the 1/r above: the exponential and the second
+        // square root are left out there, bit for bit.
+        const double x = 0.25 * r2 * (I.iR * d.iR);
+        double inv_f = inv_r;
+        if (!(x >= 60.0)) inv_f = rsqrt64(fma(I.R * d.R, exp(-x), r2));
+        t.g += I.valid ? qq * inv_f : 0.0;
+    }
+}
+
+// The same where every pair is beyond the LJ and Coulomb cutoff and has
+// x >= 60 (energy_tiles_far): only q_i q_j / r is left, the same bits.
+__device__ __forceinline__ void energy_far(const EI& I, const EJ* J, int j0, int j1, ESum& t) {
+    for (int jj = j0; jj < j1; ++jj) {
+        const double dx = I.x - J[jj].x, dy = I.y - J[jj].y, dz = I.z - J[jj].z;
+        const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+        t.g += I.valid ? I.q * J[jj].q * rsqrt64(r2) : 0.0;
+    }
+}
+
+// j atoms [j0, j1) of a diagonal or masked tile pair.
+template <bool MODEA>
+__device__ __forceinline__ void energy_masked(const og_energy64_args& e, const EI& I, const EJ* J, int j0, int j1,
+                                              int lane, bool diag, unsigned long long xm, unsigned long long m14,
+                                              ESum& t) {
+    for (int jj = j0; jj < j1; ++jj) {
+        const EJ d = J[jj];
+        const double dx = I.x - d.x, dy = I.y - d.y, dz = I.z - d.z;
+        const bool ok = I.valid && (!diag || jj > lane);
+        const double r2 = ok ? fma(dx, dx, fma(dy, dy, dz * dz)) : 1.0;
+        const double qq = I.q * d.q;
+        const bool one4 = (m14 >> jj) & 1ull;
+        bool nb = ok && !((xm >> jj) & 1ull);
+        if (MODEA) nb = nb && (r2 <= e.rc2_nb);
+        const double inv_r = rsqrt64(r2);
+        const double rmij = one4 ? I.rm14 + d.rm14 : I.rm + d.rm;
+        const double eij = one4 ? I.se14 * d.se14 : I.se * d.se;
+        const double s = rmij * inv_r;
+        const double t2 = s * s;
+        const double t6 = t2 * t2 * t2;
+        const double lj = eij * fma(t6, t6, -2.0 * t6);
+        double c = qq * inv_r;
+        if (MODEA) c = qq * (inv_r + e.kappa * r2 - e.crf);
+        t.lj += nb ? lj : 0.0;
+        t.c += nb ? c : 0.0;
+        const double x = 0.25 * r2 * (I.iR * d.iR);      // as in energy_plain
+        double inv_f = inv_r;
+        if (!(x >= 60.0)) inv_f = rsqrt64(fma(I.R * d.R, exp(-x), r2));
+        t.g += ok ? qq * inv_f : 0.0;
+    }
+}
+
+// Every pair of the tile pair is beyond the LJ and Coulomb cutoff and has
+// r^2 / (4 R_i R_j) >= 60 (tiles_beyond's bound against the larger distance;
+// 1 % to spare on R).
+__device__ __forceinline__ bool energy_tiles_far(const og_pair_args& a, int a0i, int ci, int a0j, int cj, int lane,
+                                                 double iRi, double iRj) {
+    const double* o = a.pos + 3 * (size_t)a0i;
+    LaneData di, dj;
+    const double* p = a.pos + 3 * (size_t)(a0i + (lane < ci ? lane : 0));
+    di.x = (float)(p[0] - o[0]); di.y = (float)(p[1] - o[1]); di.z = (float)(p[2] - o[2]);
+    p = a.pos + 3 * (size_t)(a0j + (lane < cj ? lane : 0));
+    dj.x = (float)(p[0] - o[0]); dj.y = (float)(p[1] - o[1]); dj.z = (float)(p[2] - o[2]);
+    const float g = -wave_max_f(-(float)iRi) * -wave_max_f(-(float)iRj);     // smallest 1 / (R_i R_j)
+    const float rc2 = fmaxf(a.rc2_nb, 245.0f / g);
+    return g > 0.0f && tiles_beyond(tile_radius(di, ci, lane, 0.0f, 0.0f, 0.0f), dj, cj, lane, rc2);
+}
+
 }  // namespace

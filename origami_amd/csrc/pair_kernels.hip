@@ -502,27 +502,6 @@ void og_launch_pair_force(const og_pair_args& a, bool mode_a, hipStream_t s) {
 // ---------------------------------------------------------------------------
 namespace {
 
-// 1/sqrt(x) for x > 0 in FP64: the hardware estimate refined by two Newton
-// steps (each doubles the number of correct bits), in place of a correctly
-// rounded square root and division.
-__device__ __forceinline__ double rsqrt64(double x) {
-    double y = __builtin_amdgcn_rsq(x);
-    double h = x * y;
-    double e = fma(-h, y, 1.0);
-    y = fma(0.5 * y, e, y);
-    h = x * y;
-    e = fma(-h, y, 1.0);
-    return fma(0.5 * y, e, y);
-}
-
-// j atom data for the FP64 energy pass, one entry per j atom of the tile in
-// the wave's LDS: every lane reads the same entry in a step (a broadcast).
-struct EJ {
-    double x, y, z, q;
-    double rm, se, rm14, se14;     // Rmin/2, sqrt(eps), 1-4 variants
-    double R, iR;                  // Born radius and its reciprocal
-};
-
 template <bool MODEA>
 __device__ void energy_body(const og_pair_args& a, const og_energy64_args& e) {
     __shared__ EJ s_j[4][OG_TILE];
@@ -540,85 +519,25 @@ __device__ void energy_body(const og_pair_args& a, const og_energy64_args& e) {
         const int a0j = a.tile_atom0[it.tj], cj = a.tile_cnt[it.tj];
         const bool vi = lane < ci, vj = lane < cj;
         const int gi = a0i + (vi ? lane : 0), gj = a0j + (vj ? lane : 0);
-        const double xi = a.pos[3 * (size_t)gi], yi = a.pos[3 * (size_t)gi + 1], zi = a.pos[3 * (size_t)gi + 2];
-        const double qi = e.charge[gi];
-        const double rmi = e.rmin[gi], sei = sqrt(e.eps[gi]);
-        const double rm14i = e.rmin14[gi], se14i = sqrt(e.eps14[gi]);
-        const double Ri = e.radii[gi], iRi = 1.0 / Ri;
+        const EI I = energy_i(a, e, gi, vi, e.radii[gi]);
         unsigned long long xm = 0, m14 = 0;
         if (it.mask >= 0) {
             xm = a.masks[(size_t)it.mask * 128 + lane];
             m14 = a.masks[(size_t)it.mask * 128 + 64 + lane];
         }
-        EJ mine;
-        mine.x = a.pos[3 * (size_t)gj]; mine.y = a.pos[3 * (size_t)gj + 1]; mine.z = a.pos[3 * (size_t)gj + 2];
-        mine.q = e.charge[gj];
-        mine.rm = e.rmin[gj]; mine.se = sqrt(e.eps[gj]);
-        mine.rm14 = e.rmin14[gj]; mine.se14 = sqrt(e.eps14[gj]);
-        mine.R = e.radii[gj]; mine.iR = 1.0 / mine.R;
+        const EJ mine = energy_j(a, e, gj, e.radii[gj]);
         wave_lds_order();                           // the previous tile's reads are done
         J[lane] = mine;
         wave_lds_order();
         const bool diag = it.ti == it.tj;
-        double elj = 0.0, ec = 0.0, eg = 0.0;
+        ESum t = {0.0, 0.0, 0.0};
         if (!diag && it.mask < 0) {
-            // off-diagonal tile pair without excluded or 1-4 pairs: the same
-            // terms with the mask and 1-4 selects left out
-            const double xo = vi ? xi : xi + 1.0e6;      // padding lanes: far away, added as 0
-            for (int jj = 0; jj < cj; ++jj) {
-                const EJ d = J[jj];
-                const double dx = xo - d.x, dy = yi - d.y, dz = zi - d.z;
-                const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-                const double qq = qi * d.q;
-                const double inv_r = rsqrt64(r2);
-                const double t = (rmi + d.rm) * inv_r;
-                const double t2 = t * t;
-                const double t6 = t2 * t2 * t2;
-                const double lj = (sei * d.se) * fma(t6, t6, -2.0 * t6);
-                double c = qq * inv_r;
-                bool nb = vi;
-                if (MODEA) {
-                    c = qq * (inv_r + e.kappa * r2 - e.crf);
-                    nb = nb && (r2 <= e.rc2_nb);
-                }
-                elj += nb ? lj : 0.0;
-                ec += nb ? c : 0.0;
-                const double x = 0.25 * r2 * (iRi * d.iR);
-                double inv_f = inv_r;
-                if (!(x >= 60.0)) inv_f = rsqrt64(fma(Ri * d.R, exp(-x), r2));
-                eg += vi ? qq * inv_f : 0.0;
-            }
-        } else
-        for (int jj = 0; jj < cj; ++jj) {
-            const EJ d = J[jj];
-            const double dx = xi - d.x, dy = yi - d.y, dz = zi - d.z;
-            const bool ok = vi && (!diag || jj > lane);
-            const double r2 = ok ? fma(dx, dx, fma(dy, dy, dz * dz)) : 1.0;
-            const double qq = qi * d.q;
-            const bool one4 = (m14 >> jj) & 1ull;
-            bool nb = ok && !((xm >> jj) & 1ull);
-            if (MODEA) nb = nb && (r2 <= e.rc2_nb);
-            const double inv_r = rsqrt64(r2);
-            const double rmij = one4 ? rm14i + d.rm14 : rmi + d.rm;
-            const double eij = one4 ? se14i * d.se14 : sei * d.se;
-            const double t = rmij * inv_r;
-            const double t2 = t * t;
-            const double t6 = t2 * t2 * t2;
-            const double lj = eij * fma(t6, t6, -2.0 * t6);
-            double c = qq * inv_r;
-            if (MODEA) c = qq * (inv_r + e.kappa * r2 - e.crf);
-            elj += nb ? lj : 0.0;
-            ec += nb ? c : 0.0;
-            // f_GB^2 = r^2 + R_i R_j exp(-x), x = r^2 / (4 R_i R_j).  From
-            // x >= 60 on, R_i R_j exp(-x) < 1e-12 x 2^-52 r^2 (r^2 = 4 x R_i R_j),
-            // far below half an ulp of r^2, so the fma rounds to r^2 exactly
-            // and 1/f_GB is the 1/r above: the exponential and the second
-            // square root are left out there, bit for bit.
-            const double x = 0.25 * r2 * (iRi * d.iR);
-            double inv_f = inv_r;
-            if (!(x >= 60.0)) inv_f = rsqrt64(fma(Ri * d.R, exp(-x), r2));
-            eg += ok ? qq * inv_f : 0.0;
+            if (MODEA && energy_tiles_far(a, a0i, ci, a0j, cj, lane, I.iR, mine.iR)) energy_far(I, J, 0, cj, t);
+            else energy_plain<MODEA>(e, I, J, 0, cj, t);
+        } else {
+            energy_masked<MODEA>(e, I, J, 0, cj, lane, diag, xm, m14, t);
         }
+        double elj = t.lj, ec = t.c, eg = t.g;
         elj = og_wave_sum_d(elj * OG_KCAL_TO_KJ);
         ec = og_wave_sum_d(ec * kc);
         eg = og_wave_sum_d(eg * pref);

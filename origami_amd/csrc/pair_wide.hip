@@ -12,6 +12,7 @@
 // The Born radii are formed where the force pass loads its atoms, so that the
 // force evaluation is two dependent launches instead of three:
 //   og_k_wide_descreen  descreening items | bonded terms
+//   og_k_wide_energy    energies only: tile pairs | radii, GB self | gather
 //   og_k_wide_force     strips, force items | radii (stored for the readers
 //                       after this pass) | bonded gather and next step's noise
 #include "og_device.h"
@@ -443,14 +444,15 @@ __device__ __forceinline__ void wide_force_strip(WideForce& L, const og_pair_arg
 // blocks [0, n_work): descreening items; the rest: bonded terms
 // (four waves per SIMD, so that two blocks share a CU: left to itself the
 // compiler spends 149-164 registers on the bonded and noise code)
-template <bool MODEA>
+template <bool MODEA, bool ENERGY>
 __global__ void __launch_bounds__(OG_WIDE_THREADS) og_k_wide_descreen(og_pair_args a, og_bonded_args b) {
     __shared__ WideDescreen L;
     if ((int)blockIdx.x < a.n_work) {
         const og_work it = a.work[blockIdx.x];
+        if (ENERGY && a.skip_sys && a.skip_sys[it.sys]) return;
         wide_descreen_item<MODEA>(L, a, it, threadIdx.x & 63, threadIdx.x >> 6);
     } else {
-        bonded_body<false>(b, blockIdx.x - a.n_work, gridDim.x - a.n_work);
+        bonded_body<ENERGY>(b, blockIdx.x - a.n_work, gridDim.x - a.n_work);
     }
 }
 
@@ -483,11 +485,95 @@ og_k_wide_force(og_pair_args a, og_radii_args r, og_bonded_args b, int ns, int n
     else gather_lds_body<NOISE, OG_WIDE_THREADS>(b, k - nr, L.t);
 }
 
-void og_launch_wide_descreen(const og_pair_args& a, const og_bonded_args& b, bool mode_a, hipStream_t s) {
+// Energies only: blocks [0, n_work) tile pairs (a split pair whole, once), nr
+// blocks of radii and GB self energies, the rest the gather (its sums are
+// range-checked as in a force evaluation).  Each wave takes 8 of the 64 j
+// atoms; one fixed-point value per tile pair and term, as in the one-wave form.
+template <bool MODEA>
+__global__ void __launch_bounds__(OG_WIDE_THREADS) og_k_wide_energy(og_pair_args a, og_energy64_args e, og_radii_args r,
+                                                                    og_bonded_args b, int nr) {
+    __shared__ union {
+        struct {
+            EJ j[OG_TILE];
+            double part[OG_WIDE_WAVES][3];
+            int far_pair;
+        } e;
+        double t[3 * OG_GATHER_CHUNK];
+    } L;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int k = blockIdx.x;
+    if (k >= a.n_work) {
+        k -= a.n_work;
+        if (k < nr) radii_body<true>(r, k * OG_WIDE_THREADS + threadIdx.x);
+        else gather_lds_body<false, OG_WIDE_THREADS>(b, k - nr, L.t);
+        return;
+    }
+    const og_work it = a.work[k];
+    if (it.part == 1 || (a.skip_sys && a.skip_sys[it.sys])) return;
+    const int a0i = a.tile_atom0[it.ti], ci = a.tile_cnt[it.ti];
+    const int a0j = a.tile_atom0[it.tj], cj = a.tile_cnt[it.tj];
+    const bool vi = lane < ci, diag = it.ti == it.tj, plain = !diag && it.mask < 0;
+    const int gi = a0i + (vi ? lane : 0), gj = a0j + (lane < cj ? lane : 0);
+    auto radius = [&](int g) {
+        bool clamped;
+        return born_radius((double)a.iacc[g] * OG_FIX_INV, r.rho[g], clamped);
+    };
+    const EI I = energy_i(a, e, gi, vi, radius(gi));
+    unsigned long long xm = 0, m14 = 0;
+    if (it.mask >= 0) {
+        xm = a.masks[(size_t)it.mask * 128 + lane];
+        m14 = a.masks[(size_t)it.mask * 128 + 64 + lane];
+    }
+    if (wave == 0) {
+        const EJ mine = energy_j(a, e, gj, radius(gj));
+        L.e.j[lane] = mine;
+        const bool far = MODEA && plain && energy_tiles_far(a, a0i, ci, a0j, cj, lane, I.iR, mine.iR);
+        if (lane == 0) L.e.far_pair = far;
+    }
+    __syncthreads();
+    ESum t = {0.0, 0.0, 0.0};
+    constexpr int N = OG_TILE / OG_WIDE_WAVES;
+    const int j0 = wave * N, j1 = j0 + N < cj ? j0 + N : cj;
+    if (MODEA && L.e.far_pair) energy_far(I, L.e.j, j0, j1, t);
+    else if (plain) energy_plain<MODEA>(e, I, L.e.j, j0, j1, t);
+    else energy_masked<MODEA>(e, I, L.e.j, j0, j1, lane, diag, xm, m14, t);
+    t.lj = og_wave_sum_d(t.lj);
+    t.c = og_wave_sum_d(t.c);
+    t.g = og_wave_sum_d(t.g);
+    if (lane == 0) {
+        L.e.part[wave][0] = t.lj;
+        L.e.part[wave][1] = t.c;
+        L.e.part[wave][2] = t.g;
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) {
+        const double unit = threadIdx.x == 0   ? OG_KCAL_TO_KJ
+                            : threadIdx.x == 1 ? OG_COULOMB_KCAL * OG_KCAL_TO_KJ
+                                               : -(1.0 - 1.0 / OG_EPS_WATER) * OG_COULOMB_KCAL * OG_KCAL_TO_KJ;
+        const int term = threadIdx.x == 0 ? OG_E_LJ : threadIdx.x == 1 ? OG_E_COUL : OG_E_GB_PAIR;
+        double sum = 0.0;
+        for (int w = 0; w < OG_WIDE_WAVES; ++w) sum += L.e.part[w][threadIdx.x];
+        og_atomic_add_fix(a.eacc + (size_t)it.sys * OG_NE + term,
+                          og_to_fix_chk(sum * unit, a.sflag ? a.sflag + it.sys : nullptr));
+    }
+}
+
+void og_launch_wide_energy(const og_pair_args& a, const og_energy64_args& e, const og_radii_args& r,
+                           const og_bonded_args& b, bool mode_a, hipStream_t s) {
+    const int nr = (r.n_atoms + OG_WIDE_THREADS - 1) / OG_WIDE_THREADS;
+    const int ng = (b.n_atoms + OG_GATHER_ATOMS - 1) / OG_GATHER_ATOMS;
+    const dim3 g(a.n_work + nr + ng), t(OG_WIDE_THREADS);
+    if (mode_a) hipLaunchKernelGGL(og_k_wide_energy<true>, g, t, 0, s, a, e, r, b, nr);
+    else hipLaunchKernelGGL(og_k_wide_energy<false>, g, t, 0, s, a, e, r, b, nr);
+}
+
+void og_launch_wide_descreen(const og_pair_args& a, const og_bonded_args& b, bool mode_a, bool energy, hipStream_t s) {
     const int total = b.nb + b.na + b.nd + b.ni;
-    const dim3 g(a.n_work + (total + OG_WIDE_THREADS - 1) / OG_WIDE_THREADS);
-    if (mode_a) hipLaunchKernelGGL(og_k_wide_descreen<true>, g, dim3(OG_WIDE_THREADS), 0, s, a, b);
-    else hipLaunchKernelGGL(og_k_wide_descreen<false>, g, dim3(OG_WIDE_THREADS), 0, s, a, b);
+    const dim3 g(a.n_work + (total + OG_WIDE_THREADS - 1) / OG_WIDE_THREADS), t(OG_WIDE_THREADS);
+    if (mode_a && energy) hipLaunchKernelGGL((og_k_wide_descreen<true, true>), g, t, 0, s, a, b);
+    else if (mode_a) hipLaunchKernelGGL((og_k_wide_descreen<true, false>), g, t, 0, s, a, b);
+    else if (energy) hipLaunchKernelGGL((og_k_wide_descreen<false, true>), g, t, 0, s, a, b);
+    else hipLaunchKernelGGL((og_k_wide_descreen<false, false>), g, t, 0, s, a, b);
 }
 
 void og_launch_wide_force(const og_pair_args& a, const og_radii_args& r, const og_bonded_args& b, bool mode_a,

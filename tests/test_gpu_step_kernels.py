@@ -127,3 +127,23 @@ def test_minimiser_direction_forms_agree(E, chains):
     for eng in (alone, beside):
         minimize_device(eng, max_steps=14, mode_a=True)
     assert np.array_equal(alone.positions(), beside.positions()[:n])
+
+
+@pytest.mark.parametrize("stretch", [1.0, 1.7, 40.0])
+@pytest.mark.parametrize("profiled", [False, True])
+@pytest.mark.parametrize("mode_a", [False, True])
+@pytest.mark.parametrize("chains", [[(16, 4)], [(3, 3), (9, 15), (13, 16)], [(2, 70)]])
+def test_energies_of_both_forms_against_oracle(E, chains, mode_a, profiled, stretch):
+    """Pair energies by both forms (the profiled path runs the one-wave
+    form), tile pairs on either side of the cutoff and of the distance where
+    only q_i q_j / r is left: relative 1e-9 with a floor of 1e-6 kJ/mol, the
+    engine's energy bar (one unit of 2^-32 kJ/mol per contribution)."""
+    systems = [S.seeded_chain(*c) for c in chains]
+    rng = np.random.default_rng(12)
+    x = [stretch * (s.pos + rng.normal(scale=0.02, size=s.pos.shape)) for s in systems]
+    eng = E.Engine(systems)
+    eng.profile(profiled)
+    for s, p, got in zip(systems, x, eng.total_energy(np.concatenate(x), mode_a=mode_a)):
+        ref = O.Oracle(s).total_energy(p, *((10.0, 20.0) if mode_a else ()))
+        for k in ("lj", "coulomb", "gb_self", "gb_pair"):
+            assert abs(got[k] - ref[k]) <= 1e-9 * abs(ref[k]) + 1e-6, (k, got[k], ref[k])
