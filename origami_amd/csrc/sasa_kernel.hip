@@ -237,16 +237,6 @@ __device__ __forceinline__ void sasa_capacity_exceeded(const og_sasa_data& d, in
     atomicOr(d.sflag + d.atom_sys[ia], OG_ST_SASA);
 }
 
-__device__ __forceinline__ double wave_min_d(double v) {
-    for (int o = 32; o >= 1; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
-    return v;
-}
-
-__device__ __forceinline__ int wave_min_i(int v) {
-    for (int o = 32; o >= 1; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
-    return v;
-}
-
 // Accessible area of one atom from its boundary (area.rs:19-126):
 // A = R^2 (2 pi (2c - L) - sum_arcs cos(a) theta - sum_vertices eps), clamped
 // to [0, 4 pi R^2]; L and the vertex sum from the face walk
@@ -258,97 +248,158 @@ template <class LT>
 __device__ void atom_area(LT& L, const og_sasa_data& d, int ia, double ri, int nc, int na, int lane,
                           const double* wd, const int* wi) {
     const double two_pi = 2.0 * 3.14159265358979323846;
+    // ---- face walk ----
+    // Each arc's successor and exterior angle depend on that arc alone, so
+    // they are formed first, a lane per arc: the arcs that start where it ends
+    // (usually one besides itself), among several the one turned to by the
+    // smallest angle (ties to the lower index).  The walk itself is then one
+    // lane following indices and adding angles in its order.  (Formed inside
+    // the walk, each step waited for two wave-wide reductions and an atan2:
+    // the walk was two thirds of an area.)
     unsigned char* visited = L.perm;                                  // [na] (na <= 256)
-    for (int a = lane; a < na; a += 64) visited[a] = 0;
-    wave_sync();
-    // ---- face walk: lanes over candidate arcs, the walk itself is uniform ----
-    int loops = 0;
-    double vsum = 0.0;
-    for (int start = 0; start < na; ++start) {
-        if (visited[start]) continue;
-        if (wi[WI_ARC + 2 * start + 1]) {          // full circle: a loop, no vertices
-            if (lane == 0) visited[start] = 1;
-            wave_sync();
-            ++loops;
-            continue;
+    unsigned char* next = L.rm;                                       // [na]
+    unsigned char* kind = L.est;                                      // [na] 0 arc, 1 open end, 2 full circle
+    double* turn = L.ta;                                              // [na]
+    for (int base = 0; base < na; base += 64) {
+        const int A = base + lane;
+        const bool arc = A < na && !wi[WI_ARC + 2 * A + 1];
+        v3 end_pt = mk(0, 0, 0), t_in = mk(0, 0, 0);
+        if (arc) {
+            const double* Ac = wd + WD_ARC + 7 * A;
+            end_pt = mk(Ac[3], Ac[4], Ac[5]);
+            t_in = normalize(cross(end_pt, cap_at(L, wi[WI_ARC + 2 * A]).axis));
         }
-        int cur = start;
-        for (int guard = 0; guard <= na; ++guard) {   // origami's walk has no guard
-            if (lane == 0) visited[cur] = 1;
-            wave_sync();
-            const double* Ac = wd + WD_ARC + 7 * cur;
-            const v3 end_pt = mk(Ac[3], Ac[4], Ac[5]);
-            const v3 t_in = normalize(cross(end_pt, cap_at(L, wi[WI_ARC + 2 * cur]).axis));
-            int first = 0x7fffffff, best_i = 0x7fffffff;
-            double best_a = INFINITY;
-            for (int base = 0; base < na; base += 64) {
-                const int c = base + lane;
-                double ang = INFINITY;
-                if (c < na && !wi[WI_ARC + 2 * c + 1]) {
-                    const double* Cc = wd + WD_ARC + 7 * c;
-                    if (norm2(mk(Cc[0], Cc[1], Cc[2]) - end_pt) < 1e-10) {
-                        first = min(first, c);
-                        if (c != cur) {
-                            const v3 t_out = normalize(cross(end_pt, cap_at(L, wi[WI_ARC + 2 * c]).axis));
-                            const double dt = fmin(fmax(dot(t_in, t_out), -1.0), 1.0);
-                            ang = atan2(dot(end_pt, cross(t_in, t_out)), dt);
-                            if (ang <= 1e-9) ang += two_pi;
-                        }
+        int first = 0x7fffffff, only = -1, n_cand = 0;
+        for (int cb = 0; cb < na; cb += 64) {
+            v3 st = mk(0, 0, 0);
+            int full = 1;
+            if (cb + lane < na) {
+                const double* Cc = wd + WD_ARC + 7 * (cb + lane);
+                st = mk(Cc[0], Cc[1], Cc[2]);
+                full = wi[WI_ARC + 2 * (cb + lane) + 1];
+            }
+            const int lim = na - cb < 64 ? na - cb : 64;
+            for (int j = 0; j < lim; ++j) {
+                const v3 q = mk(rld(st.x, j), rld(st.y, j), rld(st.z, j));
+                const int c = cb + j;
+                if (__builtin_amdgcn_readlane(full, j) == 0 && norm2(q - end_pt) < 1e-10) {
+                    first = min(first, c);
+                    if (c != A) {
+                        only = n_cand == 0 ? c : only;
+                        ++n_cand;
                     }
                 }
-                // first strictly smaller angle in candidate order = argmin, ties to the lower index
-                const double m = wave_min_d(ang);
-                const int who = wave_min_i(ang == m && m < best_a ? c : 0x7fffffff);
-                if (m < best_a) { best_a = m; best_i = who; }
             }
-            first = wave_min_i(first);
-            if (first == 0x7fffffff) break;           // open path
-            const int best = best_i != 0x7fffffff ? best_i : first;
-            const v3 t_out = normalize(cross(end_pt, cap_at(L, wi[WI_ARC + 2 * best]).axis));
-            const double dt = fmin(fmax(dot(t_in, t_out), -1.0), 1.0);
-            vsum += atan2(dot(end_pt, cross(t_in, t_out)), dt);
-            if (best == start) break;
-            cur = best;
         }
-        ++loops;
+        int best = n_cand >= 1 ? only : first;
+        if (__ballot(arc && n_cand > 1)) {
+            double best_a = INFINITY;
+            int best_i = -1;
+            for (int c = 0; c < na; ++c) {
+                if (!arc || n_cand <= 1 || c == A || wi[WI_ARC + 2 * c + 1]) continue;
+                const double* Cc = wd + WD_ARC + 7 * c;
+                if (!(norm2(mk(Cc[0], Cc[1], Cc[2]) - end_pt) < 1e-10)) continue;
+                const v3 t_out = normalize(cross(end_pt, cap_at(L, wi[WI_ARC + 2 * c]).axis));
+                const double dt = fmin(fmax(dot(t_in, t_out), -1.0), 1.0);
+                double ang = atan2(dot(end_pt, cross(t_in, t_out)), dt);
+                if (ang <= 1e-9) ang += two_pi;
+                if (ang < best_a) { best_a = ang; best_i = c; }
+            }
+            if (arc && n_cand > 1) best = best_i >= 0 ? best_i : first;
+        }
+        if (A < na) {
+            const bool open = arc && first == 0x7fffffff;
+            visited[A] = 0;
+            kind[A] = arc ? (open ? 1 : 0) : 2;
+            if (arc && !open) {
+                const v3 t_out = normalize(cross(end_pt, cap_at(L, wi[WI_ARC + 2 * best]).axis));
+                const double dt = fmin(fmax(dot(t_in, t_out), -1.0), 1.0);
+                turn[A] = atan2(dot(end_pt, cross(t_in, t_out)), dt);
+                next[A] = (unsigned char)best;
+            }
+        }
     }
     wave_sync();
-    // ---- accessible probe components ----
-    unsigned char* acc = L.tk;                                        // [OG_SASA_PROBES] (tk..tq, 768 bytes)
-    int* label = reinterpret_cast<int*>(L.ta);                        // [OG_SASA_PROBES] (ta, 2 KB)
-    bool any_acc = false;
-    for (int i = lane; i < OG_SASA_PROBES; i += 64) {
-        const double4 pr = d.probes[i];
-        bool buried = false;
-        for (int k = 0; k < nc && !buried; ++k) buried = contains_strict(cap_at(L, k), mk(pr.x, pr.y, pr.z));
-        acc[i] = buried ? 0 : 1;
-        label[i] = buried ? 0x7fffffff : i;
-        any_acc = any_acc || !buried;
+    int loops = 0;
+    double vsum = 0.0;
+    if (lane == 0) {
+        for (int start = 0; start < na; ++start) {
+            if (visited[start]) continue;
+            ++loops;
+            if (kind[start] == 2) {                   // full circle: a loop, no vertices
+                visited[start] = 1;
+                continue;
+            }
+            int cur = start;
+            for (int guard = 0; guard <= na; ++guard) {   // origami's walk has no guard
+                visited[cur] = 1;
+                if (kind[cur] != 0) break;            // open path
+                vsum += turn[cur];
+                cur = next[cur];
+                if (cur == start) break;
+            }
+        }
     }
-    int comps = 0;
-    if (__ballot(any_acc)) {
+    loops = __shfl(loops, 0, 64);
+    wave_sync();
+    // ---- accessible probe components ----
+    // c is capped at L and at least 1, so with one loop (or none) it is 1
+    // whatever the probes say; only atoms with several loops run them (they
+    // were most of an area's cost: 500 probes against every cap, then label
+    // passes over their 12 000 links).
+    int comps = loops;
+    if (loops >= 2) {
+        // accessible probes are listed first, so that the label passes run over
+        // those alone (a tenth of the sphere or less); a pass takes the least
+        // label among a probe's accessible neighbours and then follows labels
+        // (a label is a probe of the same component), and the passes end when
+        // none changes: every label is then its component's least probe
+        unsigned char* acc = L.tk;                                        // [OG_SASA_PROBES] (tk..tq, 768 bytes)
+        int* label = reinterpret_cast<int*>(L.ta);                        // [OG_SASA_PROBES] (ta, 2 KB)
+        unsigned short* open = reinterpret_cast<unsigned short*>(L.tx);   // [OG_SASA_PROBES] accessible ones
+        int n_open = 0;
+        for (int base = 0; base < OG_SASA_PROBES; base += 64) {
+            const int i = base + lane;
+            bool buried = i >= OG_SASA_PROBES;
+            if (!buried) {
+                const double4 pr = d.probes[i];
+                for (int k = 0; k < nc && !buried; ++k) buried = contains_strict(cap_at(L, k), mk(pr.x, pr.y, pr.z));
+                acc[i] = buried ? 0 : 1;
+                label[i] = i;
+            }
+            const unsigned long long om = __ballot(!buried);
+            if (!buried) open[n_open + popc(om & lanemask_lt(lane))] = (unsigned short)i;
+            n_open += popc(om);
+        }
         wave_sync();
         for (int it = 0; it < OG_SASA_PROBES; ++it) {
             bool changed = false;
-            for (int i = lane; i < OG_SASA_PROBES; i += 64) {
-                if (!acc[i]) continue;
-                int m = label[i];
+            for (int x = lane; x < n_open; x += 64) {
+                const int i = open[x], l0 = label[i];
+                int m = l0;
                 for (int q = d.padj_start[i]; q < d.padj_start[i + 1]; ++q) {
                     const int j = d.padj[q];
                     if (acc[j]) m = min(m, label[j]);
                 }
-                if (m < label[i]) { label[i] = m; changed = true; }
+                m = min(m, label[m]);
+                if (m < l0) { label[i] = m; changed = true; }
             }
             wave_sync();
             if (!__ballot(changed)) break;
         }
-        for (int i = lane; i < OG_SASA_PROBES; i += 64) comps += (acc[i] && label[i] == i) ? 1 : 0;
+        comps = 0;
+        for (int x = lane; x < n_open; x += 64) comps += label[open[x]] == open[x] ? 1 : 0;
         for (int o = 32; o >= 1; o >>= 1) comps += __shfl_xor(comps, o, 64);
     }
     // ---- area ----
+    double arc_sum = 0.0;
+    for (int base = 0; base < na; base += 64) {
+        const int A = base + lane;
+        const double t = A < na ? cap_at(L, wi[WI_ARC + 2 * A]).ca * wd[WD_ARC + 7 * A + 6] : 0.0;
+        const int lim = na - base < 64 ? na - base : 64;
+        for (int j = 0; j < lim; ++j) arc_sum += rld(t, j);
+    }
     if (lane == 0) {
-        double arc_sum = 0.0;
-        for (int a = 0; a < na; ++a) arc_sum += cap_at(L, wi[WI_ARC + 2 * a]).ca * wd[WD_ARC + 7 * a + 6];
         double area = 0.0;
         if (loops > 0) {
             int c = comps < loops ? comps : loops;
@@ -1610,19 +1661,19 @@ int og_sasa_launch(og_sasa_data* d, const double* pos, long long* facc, double g
     d->sflag = sflag;
     hipLaunchKernelGGL(og_k_tile_bounds, dim3(d->n_tiles > 0 ? d->n_tiles : 1), dim3(64), 0, s, pos,
                        d->tile_atom0, d->tile_cnt, d->n_tiles, d->tile_bound, d->counters);
-    // Until a width is chosen, a force evaluation takes at most
-    // SA_FORCE_BLOCKS_CU blocks per CU, so that the pair kernels beside it
-    // find room: a grid that fills the CUs (8 blocks) keeps them waiting until
-    // the arrangement ends.  Measured per step on 64 chains with 51 918 SASA
-    // atoms: 4.2, 2.35, 1.84, 1.99, 2.3 and 2.24 ms at 1 to 5 and 8 blocks per
-    // CU; on 4 chains with 3 493 atoms 0.27 ms at 3 against 0.30 at 8.  Up to
-    // SA_ONE_EACH_CU blocks per CU are launched where that gives every atom a
-    // wave of its own (one chain with 1 666 atoms: 0.383 ms per force call at
-    // 4, 0.397 at 3, where some waves take a second atom).  Areas (energies) have little beside them and take the full width (16 chains,
-    // 12 011 atoms: 1.01 ms at 6 to 8 blocks, 1.23 at 3).
-    const int own_wave = (d->n_work + SA_WAVES - 1) / SA_WAVES;
-    const int width = own_wave <= SA_ONE_EACH_CU * d->n_cu ? own_wave : SA_FORCE_BLOCKS_CU * d->n_cu;
-    const int blocks = d->blocks_set || area ? d->blocks : std::min(d->blocks, width);
+    // Until a width is chosen, the grid leaves the pair kernels beside it room
+    // (a grid that fills the CUs, 8 blocks, keeps them waiting until the
+    // arrangement ends): up to SA_ONE_EACH_CU blocks per CU where that gives
+    // every atom a wave of its own (one chain with 1 666
+    // atoms: 0.383 ms per force call at 4, 0.397 at 3), else
+    // SA_FORCE_BLOCKS_CU for forces.  Measured per step on 64 chains with
+    // 51 918 SASA atoms: 4.2, 2.35, 1.84, 1.99, 2.3 and 2.24 ms at 1 to 5 and 8
+    // blocks per CU.  Areas, with the FP64 pair energies beside them, take
+    // SA_ONE_EACH_CU (12 011 atoms: 0.817 ms at 4, 0.836 at 8; 26 788: 1.50 and
+    // 1.54; 52 214: 2.61 and 2.66).
+    const int one = (d->n_work + SA_WAVES - 1) / SA_WAVES, wide = SA_ONE_EACH_CU * d->n_cu;
+    const int width = one <= wide ? one : area ? wide : SA_FORCE_BLOCKS_CU * d->n_cu;
+    const int blocks = d->blocks_set ? d->blocks : std::min(d->blocks, width);
     // One pass with MAXC caps when the grid fits its LDS; otherwise the
     // SA_NC_MAIN pass and the second pass over the atoms it deferred (usually
     // few or none), one block per CU.

@@ -147,3 +147,27 @@ def test_energies_of_both_forms_against_oracle(E, chains, mode_a, profiled, stre
         ref = O.Oracle(s).total_energy(p, *((10.0, 20.0) if mode_a else ()))
         for k in ("lj", "coulomb", "gb_self", "gb_pair"):
             assert abs(got[k] - ref[k]) <= 1e-9 * abs(ref[k]) + 1e-6, (k, got[k], ref[k])
+
+
+@pytest.mark.parametrize("seed", [0, 1, 2])
+@pytest.mark.parametrize("n_atoms", [1, 2, 7, 40])
+def test_areas_of_clusters_against_oracle(E, n_atoms, seed):
+    """Accessible areas (face walk, probe components) of isolated atoms, pairs
+    and loose clusters with several boundary loops per atom, against the FP64
+    oracle: 1e-9 relative, with a unit of the fixed-point sum per atom."""
+    base = S.seeded_chain(2, 10)
+    rng = np.random.default_rng(100 * n_atoms + seed)
+    import copy
+    s = copy.copy(base)
+    m = base.n_atoms
+    # spheres only: no bonded terms, no pair interactions
+    for k in ("bonds", "bond_params", "angles", "angle_params", "dihedrals", "dihedral_params", "impropers",
+              "improper_params", "constraints", "constraint_len"):
+        setattr(s, k, getattr(base, k)[:0])
+    s.charge, s.epsilon, s.epsilon_14 = np.zeros(m), np.zeros(m), np.zeros(m)
+    # the first n_atoms atoms in a loose ball, the rest far from it and each other
+    x = np.cumsum(np.full((m, 3), 40.0), axis=0) + 1000.0
+    x[:n_atoms] = rng.uniform(-1.0, 1.0, size=(n_atoms, 3)) * 1.9 * n_atoms ** (1.0 / 3.0)
+    got = E.Engine([s]).total_energy(x, include_sasa=True)[0]["sasa"]
+    ref = float((O.Oracle(s).sasa_area(x)[1] * s.sasa_gamma).sum())
+    assert abs(got - ref) <= 1e-9 * abs(ref) + m * 2.0 ** -32
