@@ -2005,10 +2005,7 @@ extern "C" int og_surrogate_train(og_engine* e, int32_t n_steps, int32_t batch, 
                                   float* loss_per_step) {
     SUR_CHECK(e);
     if (n_steps < 0 || !(lr > 0.0)) return fail(OG_ERR_ARG, "n_steps must be >= 0 and lr > 0");
-    for (int t = 0; t < n_steps; ++t) {
-        const uint64_t sd = seed * 0x9E3779B97F4A7C15ull + (uint64_t)t;
-        SUR_CALL(og_sur_train_step(e->sur, batch, lr, sd, loss_per_step ? loss_per_step + t : nullptr));
-    }
+    SUR_CALL(og_sur_train(e->sur, n_steps, batch, lr, seed, loss_per_step));
     HIPCHK(hipStreamSynchronize(e->stream));
     return OG_OK;
 }

@@ -24,6 +24,7 @@
 #define OG_SUR_RS 0.25
 #define OG_SUR_BIN 0.375      // Å, 32 bins up to 12 Å
 #define OG_SUR_BMAX 8192      // largest training batch
+#define OG_SUR_LOSSES 1024   // step losses held on the device before they are copied out
 
 struct og_sur {
     int n_atoms = 0, n_pad = 0, n_tiles = 0, n_sys = 0;
@@ -55,7 +56,7 @@ struct og_sur {
     // batch scratch
     unsigned short *Xb = nullptr, *XbT = nullptr, *H1T = nullptr, *dZ1T = nullptr, *dZ2T = nullptr;
     float *dZ1Tf = nullptr, *dZ2Tf = nullptr, *H2Tf = nullptr, *tb = nullptr, *dy = nullptr;
-    float *lossr = nullptr, *loss1 = nullptr;
+    float *lossr = nullptr, *loss = nullptr;   // per row; per step [OG_SUR_LOSSES]
     // fallback checking
     bool enabled = false;
     int check_every = 0, calls = 0;
@@ -75,8 +76,8 @@ int og_sur_descriptors(og_sur* s, bool all);
 int og_sur_infer(og_sur* s);
 // append (descriptor, plain radius) rows for every atom; radii_dev = plain radii
 int og_sur_collect(og_sur* s, const double* radii_dev);
-// one Adam step on a sampled batch; loss (mean squared, normalised units) if not null
-int og_sur_train_step(og_sur* s, int batch, double lr, unsigned long long seed, float* loss);
+// Adam steps, each on a sampled batch; each step's loss (mean squared, normalised units) if not null
+int og_sur_train(og_sur* s, int n_steps, int batch, double lr, unsigned long long seed, float* loss_per_step);
 // gradient of the mean squared loss on an explicit batch (x: n x 161, target radii)
 int og_sur_gradient(og_sur* s, const float* x, const float* r_target, int n, float* grad, double* loss);
 // zero the per-system deviations / turn systems above tol back to plain GB

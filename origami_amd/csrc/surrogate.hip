@@ -16,7 +16,7 @@
 //   W1t  [128][192]   layer-1 weights, output-major  -> B operand, layer 1
 //   W2t  [128][128]   layer-2 weights, output-major  -> B operand, layer 2
 //   W2i  [128][128]   layer-2 weights, input-major   -> B operand, dH1 = dZ2 W2^T
-//   *T   [feature][batch] transposed activations      -> operands of the
+//   *T   [batch/16][feature][16] activations          -> operands of the
 //        weight-gradient GEMMs, whose reduction runs over the batch.
 #include <hip/hip_runtime.h>
 
@@ -61,10 +61,8 @@ __device__ __forceinline__ og_f32x4 mfma(og_bf16x8 a, og_bf16x8 b, og_f32x4 c) {
 
 __device__ __forceinline__ float sigm(float z) { return 1.0f / (1.0f + expf(-z)); }
 __device__ __forceinline__ float silu(float z) { return z * sigm(z); }
-__device__ __forceinline__ float dsilu(float z) {
-    const float s = sigm(z);
-    return s * (1.0f + z * (1.0f - s));
-}
+// silu'(z) from z and s = sigm(z)
+__device__ __forceinline__ float dsilu(float z, float s) { return s * (1.0f + z * (1.0f - s)); }
 
 __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
@@ -172,12 +170,6 @@ __global__ void __launch_bounds__(64 * SUR_DESC_WAVES) og_k_sur_desc(DescArgs a)
     }
 }
 
-// ---------------------------------------------------------------------------
-// Forward pass for 16 rows per wave (shared by inference and training).
-// z1, z2: pre-activations (bias included) in the D layout; h2: SiLU(z2).
-// hs: this wave's LDS tile [16][136] (bf16).  Returns y for rows 4g..4g+3
-// (every lane of a 16-lane group holds its group's four sums).
-// ---------------------------------------------------------------------------
 namespace {
 
 struct MlpParams {
@@ -187,57 +179,21 @@ struct MlpParams {
     const float* p;            // FP32 master (b1, b2, w3, b3)
 };
 
-__device__ __forceinline__ void mlp_forward(const unsigned short* X, int row0, const MlpParams& P,
-                                            unsigned short (*hs)[136], int lane, og_f32x4 (&z1)[8],
-                                            og_f32x4 (&z2)[8], float (&y)[4]) {
-    const int r = lane & 15, g = lane >> 4;
-    og_bf16x8 a1[6];
-#pragma unroll
-    for (int kk = 0; kk < 6; ++kk) a1[kk] = ld8(X + (size_t)(row0 + r) * OG_SUR_K1 + kk * 32 + g * 8);
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {
-        og_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < 6; ++kk)
-            acc = mfma(a1[kk], ld8(P.W1t + (size_t)(nt * 16 + r) * OG_SUR_K1 + kk * 32 + g * 8), acc);
-        const float b = P.p[OG_SUR_OFF_B1 + nt * 16 + r];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            acc[i] += b;
-            hs[g * 4 + i][nt * 16 + r] = f2bf(silu(acc[i]));
-        }
-        z1[nt] = acc;
+struct MlpOperands {
+    unsigned short *W1t, *W2t, *W2i;
+};
+
+// BF16 operand copy (copies, of W2) of parameter q
+__device__ __forceinline__ void store_operand(const MlpOperands& o, int q, float w) {
+    if (q < OG_SUR_OFF_B1) {
+        const int k = q / OG_SUR_H, j = q % OG_SUR_H;
+        o.W1t[j * OG_SUR_K1 + k] = f2bf(w);
+    } else if (q >= OG_SUR_OFF_W2 && q < OG_SUR_OFF_B2) {
+        const int e = q - OG_SUR_OFF_W2;
+        const int k = e / OG_SUR_H, j = e % OG_SUR_H;
+        o.W2t[j * OG_SUR_H + k] = f2bf(w);
+        o.W2i[k * OG_SUR_H + j] = f2bf(w);
     }
-    wave_sync();
-    og_bf16x8 a2[4];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) a2[kk] = ld8(&hs[r][kk * 32 + g * 8]);
-    float ys[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {
-        og_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk)
-            acc = mfma(a2[kk], ld8(P.W2t + (size_t)(nt * 16 + r) * OG_SUR_H + kk * 32 + g * 8), acc);
-        const float b = P.p[OG_SUR_OFF_B2 + nt * 16 + r];
-        const float w = P.p[OG_SUR_OFF_W3 + nt * 16 + r];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            acc[i] += b;
-            ys[i] += silu(acc[i]) * w;
-        }
-        z2[nt] = acc;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        float v = ys[i];
-        v += __shfl_xor(v, 1, 64);
-        v += __shfl_xor(v, 2, 64);
-        v += __shfl_xor(v, 4, 64);
-        v += __shfl_xor(v, 8, 64);
-        y[i] = v + P.p[OG_SUR_OFF_B3];
-    }
-    wave_sync();   // hs is reused by the caller
 }
 
 }  // namespace
@@ -331,171 +287,6 @@ __global__ void __launch_bounds__(128) og_k_sur_infer64(const unsigned short* X,
         }
 }
 
-// Training forward + backward for 16 batch rows per wave.
-struct TrainArgs {
-    const unsigned short* Xb;   // [B][K1]
-    const float* tb;            // [B] normalised targets
-    int B;
-    unsigned short *H1T, *dZ1T, *dZ2T;   // [H][B] bf16
-    float *dZ1Tf, *dZ2Tf, *H2Tf;         // [H][B] fp32
-    float *dy, *lossr;                   // [B]
-};
-
-__global__ void __launch_bounds__(256) og_k_sur_fwdbwd(TrainArgs a, MlpParams P) {
-    __shared__ __attribute__((aligned(16))) unsigned short hs[4][16][136];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int r = lane & 15, g = lane >> 4;
-    const int row0 = (blockIdx.x * 4 + w) * 16;
-    if (row0 >= a.B) return;
-    og_f32x4 z1[8], z2[8];
-    float y[4];
-    mlp_forward(a.Xb, row0, P, hs[w], lane, z1, z2, y);
-    const float inv_b2 = 2.0f / (float)a.B;
-    float dyv[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = row0 + g * 4 + i;
-        const float d = y[i] - a.tb[row];
-        dyv[i] = d * inv_b2;
-        if (r == 0) {
-            a.dy[row] = dyv[i];
-            a.lossr[row] = d * d;
-        }
-    }
-    // dZ2 = dy w3 * silu'(z2); activations stored transposed for the weight GEMMs
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {
-        const int j = nt * 16 + r;
-        const float w3 = P.p[OG_SUR_OFF_W3 + j];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = row0 + g * 4 + i;
-            const size_t o = (size_t)j * a.B + row;
-            const float dz2 = dyv[i] * w3 * dsilu(z2[nt][i]);
-            a.dZ2Tf[o] = dz2;
-            const unsigned short dz2b = f2bf(dz2);
-            a.dZ2T[o] = dz2b;
-            a.H2Tf[o] = silu(z2[nt][i]);
-            a.H1T[o] = f2bf(silu(z1[nt][i]));
-            hs[w][g * 4 + i][j] = dz2b;
-        }
-    }
-    wave_sync();
-    // dH1 = dZ2 W2^T, then dZ1 = dH1 * silu'(z1)
-    og_bf16x8 a2[4];
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) a2[kk] = ld8(&hs[w][r][kk * 32 + g * 8]);
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {
-        og_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk)
-            acc = mfma(a2[kk], ld8(P.W2i + (size_t)(nt * 16 + r) * OG_SUR_H + kk * 32 + g * 8), acc);
-        const int k = nt * 16 + r;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = row0 + g * 4 + i;
-            const size_t o = (size_t)k * a.B + row;
-            const float dz1 = acc[i] * dsilu(z1[nt][i]);
-            a.dZ1Tf[o] = dz1;
-            a.dZ1T[o] = f2bf(dz1);
-        }
-    }
-}
-
-// Weight gradients, one wave per task, fixed reduction order (deterministic):
-//   tasks [0, 96)      dW1 tiles: D[j][k] = sum_b dZ1T[j][b] XbT[k][b]
-//   tasks [96, 160)    dW2 tiles: D[j][k] = sum_b dZ2T[j][b] H1T[k][b]
-//   tasks [160, 288)   db1[j] = sum_b dZ1[b][j]
-//   tasks [288, 416)   db2[j] = sum_b dZ2[b][j]
-//   tasks [416, 544)   dW3[j] = sum_b H2[b][j] dy[b]
-//   task 544           db3 = sum_b dy[b];   task 545  loss = mean (y - t)^2
-struct GradArgs {
-    const unsigned short *dZ1T, *XbT, *dZ2T, *H1T;
-    const float *dZ1Tf, *dZ2Tf, *H2Tf, *dy, *lossr;
-    int B;
-    float* grad;
-    float* loss;
-};
-
-__global__ void __launch_bounds__(64) og_k_sur_wgrad(GradArgs a) {
-    const int task = blockIdx.x;
-    const int lane = threadIdx.x;
-    const int r = lane & 15, g = lane >> 4;
-    if (task < 160) {
-        const bool first = task < 96;
-        const int jt = first ? task / 12 : (task - 96) / 8;
-        const int kt = first ? task % 12 : (task - 96) % 8;
-        const unsigned short* A = first ? a.dZ1T : a.dZ2T;
-        const unsigned short* Bm = first ? a.XbT : a.H1T;
-        og_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        for (int kk = 0; kk < a.B / 32; ++kk)
-            acc = mfma(ld8(A + (size_t)(jt * 16 + r) * a.B + kk * 32 + g * 8),
-                       ld8(Bm + (size_t)(kt * 16 + r) * a.B + kk * 32 + g * 8), acc);
-        const int k = kt * 16 + r;
-        const int off = first ? OG_SUR_OFF_W1 : OG_SUR_OFF_W2;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int j = jt * 16 + g * 4 + i;
-            a.grad[off + k * OG_SUR_H + j] = acc[i];
-        }
-        return;
-    }
-    float s = 0.0f;
-    int out = -1;
-    if (task < 288) {
-        const int j = task - 160;
-        for (int b = lane; b < a.B; b += 64) s += a.dZ1Tf[(size_t)j * a.B + b];
-        out = OG_SUR_OFF_B1 + j;
-    } else if (task < 416) {
-        const int j = task - 288;
-        for (int b = lane; b < a.B; b += 64) s += a.dZ2Tf[(size_t)j * a.B + b];
-        out = OG_SUR_OFF_B2 + j;
-    } else if (task < 544) {
-        const int j = task - 416;
-        for (int b = lane; b < a.B; b += 64) s += a.H2Tf[(size_t)j * a.B + b] * a.dy[b];
-        out = OG_SUR_OFF_W3 + j;
-    } else if (task == 544) {
-        for (int b = lane; b < a.B; b += 64) s += a.dy[b];
-        out = OG_SUR_OFF_B3;
-    } else {
-        for (int b = lane; b < a.B; b += 64) s += a.lossr[b];
-    }
-    for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
-    if (lane == 0) {
-        if (out >= 0) a.grad[out] = s;
-        else *a.loss = s / (float)a.B;
-    }
-}
-
-// Adam update of the FP32 master parameters, then the BF16 operand copies.
-__global__ void __launch_bounds__(256) og_k_sur_adam(float* p, float* m, float* v, const float* grad,
-                                                     float lr, float c1, float c2, int update,
-                                                     unsigned short* W1t, unsigned short* W2t,
-                                                     unsigned short* W2i) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= OG_SUR_P) return;
-    float w = p[q];
-    if (update) {
-        const float gq = grad[q];
-        const float mq = 0.9f * m[q] + 0.1f * gq;
-        const float vq = 0.999f * v[q] + 0.001f * gq * gq;
-        m[q] = mq;
-        v[q] = vq;
-        w -= lr * (mq / c1) / (sqrtf(vq / c2) + 1e-8f);
-        p[q] = w;
-    }
-    if (q < OG_SUR_OFF_B1) {
-        const int k = q / OG_SUR_H, j = q % OG_SUR_H;
-        W1t[j * OG_SUR_K1 + k] = f2bf(w);
-    } else if (q >= OG_SUR_OFF_W2 && q < OG_SUR_OFF_B2) {
-        const int e = q - OG_SUR_OFF_W2;
-        const int k = e / OG_SUR_H, j = e % OG_SUR_H;
-        W2t[j * OG_SUR_H + k] = f2bf(w);
-        W2i[k * OG_SUR_H + j] = f2bf(w);
-    }
-}
-
 __device__ __forceinline__ unsigned long long sur_mix(unsigned long long x) {
     x += 0x9E3779B97F4A7C15ull;
     x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
@@ -503,18 +294,332 @@ __device__ __forceinline__ unsigned long long sur_mix(unsigned long long x) {
     return x ^ (x >> 31);
 }
 
-// Batch gather: row b of the batch = training row hash(seed, b) mod n_train.
-__global__ void __launch_bounds__(256) og_k_sur_gather(const unsigned short* Xtr, const float* ttr,
-                                                       long long n_train, int B, unsigned long long seed,
-                                                       unsigned short* Xb, unsigned short* XbT, float* tb) {
-    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= (long long)B * OG_SUR_K1) return;
-    const int b = (int)(q / OG_SUR_K1), f = (int)(q % OG_SUR_K1);
-    const long long idx = (long long)(sur_mix(seed ^ sur_mix((unsigned long long)b)) % (unsigned long long)n_train);
-    const unsigned short x = Xtr[idx * OG_SUR_K1 + f];
-    Xb[(size_t)b * OG_SUR_K1 + f] = x;
-    XbT[(size_t)f * B + b] = x;
-    if (f == 0) tb[b] = ttr[idx];
+// h mod n with inv = (2^64 - 1) / n: the quotient guessed from inv is at most
+// two too small
+__device__ __forceinline__ unsigned long long sur_mod(unsigned long long h, unsigned long long n,
+                                                      unsigned long long inv) {
+    unsigned long long m = h - __umul64hi(h, inv) * n;
+    if (m >= n) m -= n;
+    if (m >= n) m -= n;
+    return m;
+}
+
+// Training forward + backward, 16 batch rows per block: each of the eight
+// waves takes one of the eight 16-column groups of every layer, with the
+// activations exchanged over LDS.  What bounds the kernel at these sizes (a
+// batch of 4 096 is 256 row groups) is one wave's chain of weight loads, MFMA
+// and exponentials, so a group's chain is cut in eight.  Each element keeps its
+// own MFMA chain and the output sum its order over the column groups, so the
+// values are those of one wave per group.  The block also picks its rows out
+// of the training set, row b being hash(seed, b) mod n_rows (n_rows 0: row b
+// itself).  What the weight gradients read is left by groups of 16 rows,
+// [B/16][columns][16]: a block writes whole lines, and a wave there reads the
+// 32 rows of 16 columns as two runs of 512 bytes.  At 4 096 rows 50 us before
+// (40 and a separate gather's 10), 16 now, of which 9 are the chain (2 blocks
+// take as long) and the rest the 11 MB written.
+__device__ __forceinline__ size_t sur_at(int col, int row, int cols) {
+    return ((size_t)(row >> 4) * cols + col) * 16 + (row & 15);
+}
+
+struct TrainArgs {
+    const unsigned short* X;    // [rows][K1]
+    const float* t;             // [rows] normalised targets
+    long long n_rows;
+    unsigned long long inv;     // (2^64 - 1) / n_rows
+    unsigned long long seed;
+    int B;
+    unsigned short* XbT;                 // [B/16][K1][16]
+    unsigned short *H1T, *dZ1T, *dZ2T;   // [B/16][H][16] bf16
+    float *dZ1Tf, *dZ2Tf, *H2Tf;         // [B/16][H][16] fp32
+    float *dy, *lossr;                   // [B]
+};
+
+__device__ __forceinline__ void store4(unsigned short* p, const unsigned short (&v)[4]) {
+    *reinterpret_cast<uint2*>(p) = make_uint2(v[0] | ((unsigned)v[1] << 16), v[2] | ((unsigned)v[3] << 16));
+}
+__device__ __forceinline__ void store4(float* p, const float (&v)[4]) {
+    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+}
+
+__global__ void __launch_bounds__(512) og_k_sur_fwdbwd(TrainArgs a, MlpParams P) {
+    __shared__ __attribute__((aligned(16))) unsigned short xs[16][OG_SUR_K1 + 8];
+    __shared__ __attribute__((aligned(16))) unsigned short h1s[16][136], dz2s[16][136];
+    __shared__ float h2s[8][16][17];                  // silu(z2) by column group, row, column
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int r = lane & 15, g = lane >> 4;
+    const int j = w * 16 + r;                          // this lane's column in every layer
+    const int row0 = blockIdx.x * 16;
+    const int rg = row0 + g * 4;                       // its four rows in the D layout
+    // the weights load first, while the row's index is formed
+    og_bf16x8 a1[6], w1[6], w2[4], w2i[4];
+#pragma unroll
+    for (int kk = 0; kk < 6; ++kk) w1[kk] = ld8(P.W1t + (size_t)j * OG_SUR_K1 + kk * 32 + g * 8);
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) w2[kk] = ld8(P.W2t + (size_t)j * OG_SUR_H + kk * 32 + g * 8);
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) w2i[kk] = ld8(P.W2i + (size_t)j * OG_SUR_H + kk * 32 + g * 8);
+    const float b1 = P.p[OG_SUR_OFF_B1 + j], b2 = P.p[OG_SUR_OFF_B2 + j], w3 = P.p[OG_SUR_OFF_W3 + j];
+    const float b3 = P.p[OG_SUR_OFF_B3];
+    float w3c[8];
+#pragma unroll
+    for (int nt = 0; nt < 8; ++nt) w3c[nt] = P.p[OG_SUR_OFF_W3 + nt * 16 + r];
+    long long src = row0 + r;
+    if (a.n_rows > 0)
+        src = (long long)sur_mod(sur_mix(a.seed ^ sur_mix((unsigned long long)src)), (unsigned long long)a.n_rows, a.inv);
+#pragma unroll
+    for (int kk = 0; kk < 6; ++kk) a1[kk] = ld8(a.X + src * OG_SUR_K1 + kk * 32 + g * 8);
+    const float tr = a.t[src];
+
+    og_f32x4 z1 = {0.f, 0.f, 0.f, 0.f}, s1;            // pre-activation and its sigmoid
+#pragma unroll
+    for (int kk = 0; kk < 6; ++kk) z1 = mfma(a1[kk], w1[kk], z1);
+    unsigned short hb[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        z1[i] += b1;
+        s1[i] = sigm(z1[i]);
+        hb[i] = f2bf(z1[i] * s1[i]);
+        h1s[g * 4 + i][j] = hb[i];
+    }
+#pragma unroll
+    for (int kk = 0; kk < 6; ++kk)
+        if (kk == w) *reinterpret_cast<og_bf16x8*>(&xs[r][kk * 32 + g * 8]) = a1[kk];
+    __syncthreads();
+
+    og_bf16x8 a2[4];
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) a2[kk] = ld8(&h1s[r][kk * 32 + g * 8]);
+    og_f32x4 z2 = {0.f, 0.f, 0.f, 0.f}, s2;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) z2 = mfma(a2[kk], w2[kk], z2);
+    float h2[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        z2[i] += b2;
+        s2[i] = sigm(z2[i]);
+        h2[i] = z2[i] * s2[i];
+        h2s[w][g * 4 + i][r] = h2[i];
+    }
+    __syncthreads();
+
+    // y of the lane's rows (every wave forms them), summed over the column
+    // groups in order, then over the columns
+    const float inv_b2 = 2.0f / (float)a.B;
+    float dyv[4], dr[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float v = 0.0f;
+#pragma unroll
+        for (int nt = 0; nt < 8; ++nt) v += h2s[nt][g * 4 + i][r] * w3c[nt];
+        v += __shfl_xor(v, 1, 64);
+        v += __shfl_xor(v, 2, 64);
+        v += __shfl_xor(v, 4, 64);
+        v += __shfl_xor(v, 8, 64);
+        dr[i] = (v + b3) - __shfl(tr, g * 4 + i, 64);
+        dyv[i] = dr[i] * inv_b2;
+    }
+    // dZ2 = dy w3 * silu'(z2)
+    float dz2[4], dz1[4];
+    unsigned short db2[4], db1[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        dz2[i] = dyv[i] * w3 * dsilu(z2[i], s2[i]);
+        db2[i] = f2bf(dz2[i]);
+        dz2s[g * 4 + i][j] = db2[i];
+    }
+    __syncthreads();
+    // dH1 = dZ2 W2^T, then dZ1 = dH1 * silu'(z1)
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) a2[kk] = ld8(&dz2s[r][kk * 32 + g * 8]);
+    og_f32x4 dh = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) dh = mfma(a2[kk], w2i[kk], dh);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        dz1[i] = dh[i] * dsilu(z1[i], s1[i]);
+        db1[i] = f2bf(dz1[i]);
+    }
+
+    // the weight gradients' operands
+    const size_t o = sur_at(j, rg, OG_SUR_H);
+    store4(a.H1T + o, hb);
+    store4(a.H2Tf + o, h2);
+    store4(a.dZ2Tf + o, dz2);
+    store4(a.dZ2T + o, db2);
+    store4(a.dZ1Tf + o, dz1);
+    store4(a.dZ1T + o, db1);
+    if (w == 0 && r == 0) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            a.dy[rg + i] = dyv[i];
+            a.lossr[rg + i] = dr[i] * dr[i];
+        }
+    }
+    if (threadIdx.x < OG_SUR_K1) {
+        unsigned v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            v[u] = xs[2 * u][threadIdx.x] | ((unsigned)xs[2 * u + 1][threadIdx.x] << 16);
+        uint4* q = reinterpret_cast<uint4*>(a.XbT + sur_at(threadIdx.x, row0, OG_SUR_K1));
+        q[0] = make_uint4(v[0], v[1], v[2], v[3]);
+        q[1] = make_uint4(v[4], v[5], v[6], v[7]);
+    }
+}
+
+// Weight gradients and the Adam step, fixed reduction order (deterministic):
+//   blocks [0, 96)     dW1 tiles: D[j][k] = sum_b dZ1T[j][b] XbT[k][b]
+//   blocks [96, 160)   dW2 tiles: D[j][k] = sum_b dZ2T[j][b] H1T[k][b]
+//   then a wave per sum: db1[j] = sum_b dZ1[b][j], db2[j] = sum_b dZ2[b][j],
+//   dW3[j] = sum_b H2[b][j] dy[b], db3 = sum_b dy[b], loss = mean (y - t)^2
+// A tile is one MFMA chain over the batch (its order is the result's), bound
+// by the wait for its operands, not by the matrix cores: the block's eight
+// waves each load SUR_WG_AHEAD steps at once and take the chain in turn,
+// passing the accumulator on through LDS.  One wave per tile that waits for
+// each step's loads took 34 us at 4 096 rows, one that loads 16 steps ahead
+// 15.5, this 10.8, with the Adam update (6 us as a launch of its own) in it:
+// an element's parameter and moments load before its gradient is formed.
+struct GradArgs {
+    const unsigned short *dZ1T, *XbT, *dZ2T, *H1T;
+    const float *dZ1Tf, *dZ2Tf, *H2Tf, *dy, *lossr;
+    int B;
+    float* grad;               // gradient out, or (null) one Adam step on p, m, v
+    float* loss;
+    float *p, *m, *v;
+    float lr, c1, c2;
+    MlpOperands o;
+};
+
+// Where element q's gradient goes: out, or through Adam (w, m0, v0: the
+// parameter and its moments) into the parameter and its BF16 copies.
+__device__ __forceinline__ void apply_gradient(const GradArgs& a, int q, float gq, float w, float m0, float v0) {
+    if (a.grad) {
+        a.grad[q] = gq;
+        return;
+    }
+    const float mq = 0.9f * m0 + 0.1f * gq;
+    const float vq = 0.999f * v0 + 0.001f * gq * gq;
+    a.m[q] = mq;
+    a.v[q] = vq;
+    w -= a.lr * (mq / a.c1) / (sqrtf(vq / a.c2) + 1e-8f);
+    a.p[q] = w;
+    store_operand(a.o, q, w);
+}
+
+#define SUR_WG_WAVES 8
+#define SUR_WG_AHEAD 16
+#define SUR_WG_TILES 160
+#define SUR_WG_SUMS (3 * OG_SUR_H + 2)
+
+// a lane's sum of x over rows lane, lane + 64, ... in order (stride: of x
+// between those rows; DOT: of x y, y by row), the loads of 32 rows in flight
+// together
+template <bool DOT>
+__device__ __forceinline__ float strided_sum(int B, int lane, const float* x, int stride, const float* y = nullptr) {
+    const int n = (B - lane + 63) / 64;
+    float s = 0.0f;
+    for (int m0 = 0; m0 < n; m0 += 32) {
+        float v[32], c[32];
+#pragma unroll
+        for (int u = 0; u < 32; ++u) {
+            const int m = m0 + u < n ? m0 + u : m0;
+            v[u] = x[(size_t)m * stride];
+            if constexpr (DOT) c[u] = y[m * 64];
+        }
+#pragma unroll
+        for (int u = 0; u < 32; ++u)
+            if (m0 + u < n) {
+                if constexpr (DOT) s += v[u] * c[u];
+                else s += v[u];
+            }
+    }
+    return s;
+}
+
+__global__ void __launch_bounds__(64 * SUR_WG_WAVES) og_k_sur_wgrad(GradArgs a) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (blockIdx.x < SUR_WG_TILES) {
+        __shared__ og_f32x4 part[64];
+        const int task = blockIdx.x;
+        const int r = lane & 15, g = lane >> 4;
+        const bool first = task < 96;
+        const int jt = first ? task / 12 : (task - 96) / 8;
+        const int kt = first ? task % 12 : (task - 96) % 8;
+        const int bc = first ? OG_SUR_K1 : OG_SUR_H;
+        const unsigned short* Ap = (first ? a.dZ1T : a.dZ2T) + sur_at(jt * 16 + r, g * 8, OG_SUR_H);
+        const unsigned short* Bp = (first ? a.XbT : a.H1T) + sur_at(kt * 16 + r, g * 8, bc);
+        const int n = a.B / 32;
+        // thread t < 256 applies element (k, j) = (t / 16, t % 16) of the tile
+        const int t = threadIdx.x;
+        const int q = (first ? OG_SUR_OFF_W1 : OG_SUR_OFF_W2) + (kt * 16 + (t >> 4)) * OG_SUR_H + jt * 16 + (t & 15);
+        float pq = 0.0f, mq = 0.0f, vq = 0.0f;
+        if (t < 256 && !a.grad) {
+            pq = a.p[q];
+            mq = a.m[q];
+            vq = a.v[q];
+        }
+        for (int k0 = 0; k0 < n; k0 += SUR_WG_WAVES * SUR_WG_AHEAD) {
+            const int kw = k0 + w * SUR_WG_AHEAD;
+            og_bf16x8 av[SUR_WG_AHEAD], bv[SUR_WG_AHEAD];
+#pragma unroll
+            for (int u = 0; u < SUR_WG_AHEAD; ++u)
+                if (kw + u < n) {
+                    av[u] = ld8(Ap + (size_t)(kw + u) * (32 * OG_SUR_H));
+                    bv[u] = ld8(Bp + (size_t)(kw + u) * (32 * bc));
+                }
+            for (int turn = 0; turn < SUR_WG_WAVES && k0 + turn * SUR_WG_AHEAD < n; ++turn) {
+                if (turn == w) {
+                    og_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                    if (kw > 0) acc = part[lane];
+#pragma unroll
+                    for (int u = 0; u < SUR_WG_AHEAD; ++u)
+                        if (kw + u < n) acc = mfma(av[u], bv[u], acc);
+                    part[lane] = acc;
+                }
+                __syncthreads();
+            }
+        }
+        if (t < 256) {
+            // D layout: row j = 4 g + i, column k = r
+            const int jl = t & 15, kl = t >> 4;
+            apply_gradient(a, q, reinterpret_cast<const float*>(part)[((jl >> 2) * 16 + kl) * 4 + (jl & 3)], pq, mq, vq);
+        }
+        return;
+    }
+    const int task = (blockIdx.x - SUR_WG_TILES) * SUR_WG_WAVES + w;
+    if (task >= SUR_WG_SUMS) return;
+    float s = 0.0f;
+    int out = -1;
+    if (task < 3 * OG_SUR_H) {
+        const size_t o = sur_at(task & (OG_SUR_H - 1), lane, OG_SUR_H);
+        const int stride = 64 * OG_SUR_H;
+        if (task < OG_SUR_H) {
+            s = strided_sum<false>(a.B, lane, a.dZ1Tf + o, stride);
+            out = OG_SUR_OFF_B1 + task;
+        } else if (task < 2 * OG_SUR_H) {
+            s = strided_sum<false>(a.B, lane, a.dZ2Tf + o, stride);
+            out = OG_SUR_OFF_B2 + task - OG_SUR_H;
+        } else {
+            s = strided_sum<true>(a.B, lane, a.H2Tf + o, stride, a.dy + lane);
+            out = OG_SUR_OFF_W3 + task - 2 * OG_SUR_H;
+        }
+    } else if (task == 3 * OG_SUR_H) {
+        s = strided_sum<false>(a.B, lane, a.dy + lane, 64);
+        out = OG_SUR_OFF_B3;
+    } else {
+        s = strided_sum<false>(a.B, lane, a.lossr + lane, 64);
+    }
+    for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
+    if (lane == 0) {
+        if (out < 0) *a.loss = s / (float)a.B;
+        else if (a.grad) a.grad[out] = s;
+        else apply_gradient(a, out, s, a.p[out], a.m[out], a.v[out]);
+    }
+}
+
+// BF16 operand copies of the FP32 master parameters.
+__global__ void __launch_bounds__(256) og_k_sur_operands(const float* p, MlpOperands o) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q < OG_SUR_P) store_operand(o, q, p[q]);
 }
 
 // Append descriptors and normalised plain radii of atoms [0, n) at row base.
@@ -562,19 +667,25 @@ int fail(const char* m) {
 }
 
 MlpParams params_of(const og_sur* s) { return {s->W1t, s->W2t, s->W2i, s->p}; }
+MlpOperands operands_of(const og_sur* s) { return {s->W1t, s->W2t, s->W2i}; }
 
 int refresh_copies(og_sur* s) {
-    hipLaunchKernelGGL(og_k_sur_adam, dim3((OG_SUR_P + 255) / 256), dim3(256), 0, s->stream, s->p, s->m, s->v,
-                       s->g, 0.0f, 1.0f, 1.0f, 0, s->W1t, s->W2t, s->W2i);
+    hipLaunchKernelGGL(og_k_sur_operands, dim3((OG_SUR_P + 255) / 256), dim3(256), 0, s->stream, s->p, operands_of(s));
     return hipGetLastError() == hipSuccess ? 0 : fail("kernel launch failed");
 }
 
 // forward + backward + weight gradients on the batch already in Xb/XbT/tb
-int batch_gradient(og_sur* s, int B) {
-    TrainArgs t{s->Xb, s->tb, B, s->H1T, s->dZ1T, s->dZ2T, s->dZ1Tf, s->dZ2Tf, s->H2Tf, s->dy, s->lossr};
-    hipLaunchKernelGGL(og_k_sur_fwdbwd, dim3((B / 16 + 3) / 4), dim3(256), 0, s->stream, t, params_of(s));
-    GradArgs ga{s->dZ1T, s->XbT, s->dZ2T, s->H1T, s->dZ1Tf, s->dZ2Tf, s->H2Tf, s->dy, s->lossr, B, s->g, s->loss1};
-    hipLaunchKernelGGL(og_k_sur_wgrad, dim3(546), dim3(64), 0, s->stream, ga);
+// forward, backward and weight gradients of B rows of (X, t); the gradient
+// goes to grad, or (null) one Adam step is taken
+int batch_gradient(og_sur* s, const unsigned short* X, const float* t, long long n_rows, unsigned long long seed,
+                   int B, float* grad, float lr, float c1, float c2, float* loss) {
+    const unsigned long long inv = n_rows > 0 ? ~0ull / (unsigned long long)n_rows : 0;
+    TrainArgs ta{X, t, n_rows, inv, seed, B, s->XbT, s->H1T, s->dZ1T, s->dZ2T, s->dZ1Tf, s->dZ2Tf, s->H2Tf, s->dy, s->lossr};
+    hipLaunchKernelGGL(og_k_sur_fwdbwd, dim3(B / 16), dim3(512), 0, s->stream, ta, params_of(s));
+    GradArgs ga{s->dZ1T, s->XbT, s->dZ2T, s->H1T, s->dZ1Tf, s->dZ2Tf, s->H2Tf, s->dy, s->lossr, B, grad, loss,
+                s->p, s->m, s->v, lr, c1, c2, operands_of(s)};
+    hipLaunchKernelGGL(og_k_sur_wgrad, dim3(SUR_WG_TILES + (SUR_WG_SUMS + SUR_WG_WAVES - 1) / SUR_WG_WAVES),
+                       dim3(64 * SUR_WG_WAVES), 0, s->stream, ga);
     return hipGetLastError() == hipSuccess ? 0 : fail("kernel launch failed");
 }
 
@@ -638,7 +749,7 @@ int og_sur_create(og_sur* s, int n_atoms, int n_sys, const std::vector<double>& 
         !dalloc(&s->Xb, B * OG_SUR_K1) || !dalloc(&s->XbT, B * OG_SUR_K1) || !dalloc(&s->H1T, B * OG_SUR_H) ||
         !dalloc(&s->dZ1T, B * OG_SUR_H) || !dalloc(&s->dZ2T, B * OG_SUR_H) || !dalloc(&s->dZ1Tf, B * OG_SUR_H) ||
         !dalloc(&s->dZ2Tf, B * OG_SUR_H) || !dalloc(&s->H2Tf, B * OG_SUR_H) || !dalloc(&s->tb, B) ||
-        !dalloc(&s->dy, B) || !dalloc(&s->lossr, B) || !dalloc(&s->loss1, 1))
+        !dalloc(&s->dy, B) || !dalloc(&s->lossr, B) || !dalloc(&s->loss, OG_SUR_LOSSES))
         return fail("device allocation failed (training buffers)");
     s->adam_t = 0;
     if (refresh_copies(s)) return -2;
@@ -648,7 +759,7 @@ int og_sur_create(og_sur* s, int n_atoms, int n_sys, const std::vector<double>& 
 void og_sur_free(og_sur* s) {
     void* ptrs[] = {s->cls, s->tile_sys, s->sys_tile_b, s->sys_tile_e, s->tile_bound, s->X, s->r_sur, s->mode,
                     s->dev, s->p, s->m, s->v, s->g, s->W1t, s->W2t, s->W2i, s->Xtr, s->ttr, s->Xb, s->XbT,
-                    s->H1T, s->dZ1T, s->dZ2T, s->dZ1Tf, s->dZ2Tf, s->H2Tf, s->tb, s->dy, s->lossr, s->loss1};
+                    s->H1T, s->dZ1T, s->dZ2T, s->dZ1Tf, s->dZ2Tf, s->H2Tf, s->tb, s->dy, s->lossr, s->loss};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     *s = og_sur{};
@@ -684,43 +795,44 @@ int og_sur_collect(og_sur* s, const double* radii_dev) {
     return 0;
 }
 
-int og_sur_train_step(og_sur* s, int batch, double lr, unsigned long long seed, float* loss) {
-    if (s->n_train <= 0) return fail("no training rows collected");
-    if (batch < 32 || batch > OG_SUR_BMAX || batch % 32) return fail("batch must be a multiple of 32 in [32, 8192]");
-    const long long tot = (long long)batch * OG_SUR_K1;
-    hipLaunchKernelGGL(og_k_sur_gather, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s->stream, s->Xtr,
-                       s->ttr, s->n_train, batch, seed, s->Xb, s->XbT, s->tb);
-    if (batch_gradient(s, batch)) return -2;
-    s->adam_t += 1;
-    const float c1 = (float)(1.0 - std::pow(0.9, s->adam_t)), c2 = (float)(1.0 - std::pow(0.999, s->adam_t));
-    hipLaunchKernelGGL(og_k_sur_adam, dim3((OG_SUR_P + 255) / 256), dim3(256), 0, s->stream, s->p, s->m, s->v,
-                       s->g, (float)lr, c1, c2, 1, s->W1t, s->W2t, s->W2i);
-    if (hipGetLastError() != hipSuccess) return fail("kernel launch failed");
-    if (loss && hipMemcpyAsync(loss, s->loss1, sizeof(float), hipMemcpyDeviceToHost, s->stream) != hipSuccess)
-        return fail("copy failed");
+int og_sur_train(og_sur* s, int n_steps, int batch, double lr, unsigned long long seed, float* loss_per_step) {
+    if (n_steps > 0 && s->n_train <= 0) return fail("no training rows collected");
+    if (n_steps > 0 && (batch < 32 || batch > OG_SUR_BMAX || batch % 32))
+        return fail("batch must be a multiple of 32 in [32, 8192]");
+    // the losses stay on the device and come back OG_SUR_LOSSES at a time: a
+    // copy per step waited for every step
+    for (int t = 0; t < n_steps; ++t) {
+        const int slot = t % OG_SUR_LOSSES;
+        s->adam_t += 1;
+        const float c1 = (float)(1.0 - std::pow(0.9, s->adam_t)), c2 = (float)(1.0 - std::pow(0.999, s->adam_t));
+        if (batch_gradient(s, s->Xtr, s->ttr, s->n_train, seed * 0x9E3779B97F4A7C15ull + (unsigned long long)t, batch,
+                           nullptr, (float)lr, c1, c2, s->loss + slot))
+            return -2;
+        if (loss_per_step && (slot == OG_SUR_LOSSES - 1 || t == n_steps - 1) &&
+            hipMemcpyAsync(loss_per_step + (t - slot), s->loss, (slot + 1) * sizeof(float), hipMemcpyDeviceToHost,
+                           s->stream) != hipSuccess)
+            return fail("copy failed");
+    }
     return 0;
 }
 
 int og_sur_gradient(og_sur* s, const float* x, const float* r_target, int n, float* grad, double* loss) {
     if (n < 32 || n > OG_SUR_BMAX || n % 32) return fail("n must be a multiple of 32 in [32, 8192]");
-    std::vector<unsigned short> xb((size_t)n * OG_SUR_K1, 0), xt((size_t)n * OG_SUR_K1, 0);
+    std::vector<unsigned short> xb((size_t)n * OG_SUR_K1, 0);
     std::vector<float> t(n);
     for (int b = 0; b < n; ++b) {
         for (int f = 0; f < OG_SUR_F; ++f) {
-            const unsigned short h = f2bf(x[(size_t)b * OG_SUR_F + f]);
-            xb[(size_t)b * OG_SUR_K1 + f] = h;
-            xt[(size_t)f * n + b] = h;
+            xb[(size_t)b * OG_SUR_K1 + f] = f2bf(x[(size_t)b * OG_SUR_F + f]);
         }
         t[b] = (float)((r_target[b] - OG_SUR_R0) / OG_SUR_RS);
     }
     if (hipMemcpyAsync(s->Xb, xb.data(), xb.size() * 2, hipMemcpyHostToDevice, s->stream) != hipSuccess ||
-        hipMemcpyAsync(s->XbT, xt.data(), xt.size() * 2, hipMemcpyHostToDevice, s->stream) != hipSuccess ||
         hipMemcpyAsync(s->tb, t.data(), t.size() * 4, hipMemcpyHostToDevice, s->stream) != hipSuccess)
         return fail("copy failed");
-    if (batch_gradient(s, n)) return -2;
+    if (batch_gradient(s, s->Xb, s->tb, 0, 0, n, s->g, 0.0f, 1.0f, 1.0f, s->loss)) return -2;
     float l = 0.0f;
     if (hipMemcpyAsync(grad, s->g, OG_SUR_P * sizeof(float), hipMemcpyDeviceToHost, s->stream) != hipSuccess ||
-        hipMemcpyAsync(&l, s->loss1, sizeof(float), hipMemcpyDeviceToHost, s->stream) != hipSuccess ||
+        hipMemcpyAsync(&l, s->loss, sizeof(float), hipMemcpyDeviceToHost, s->stream) != hipSuccess ||
         hipStreamSynchronize(s->stream) != hipSuccess)
         return fail("copy failed");
     if (loss) *loss = l;

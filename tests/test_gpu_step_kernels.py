@@ -171,3 +171,60 @@ def test_areas_of_clusters_against_oracle(E, n_atoms, seed):
     got = E.Engine([s]).total_energy(x, include_sasa=True)[0]["sasa"]
     ref = float((O.Oracle(s).sasa_area(x)[1] * s.sasa_gamma).sum())
     assert abs(got - ref) <= 1e-9 * abs(ref) + m * 2.0 ** -32
+
+
+def _mix(x):
+    m = (1 << 64) - 1
+    x = (x + 0x9E3779B97F4A7C15) & m
+    x = ((x ^ (x >> 30)) * 0xBF58476D1CE4E5B9) & m
+    x = ((x ^ (x >> 27)) * 0x94D049BB133111EB) & m
+    return x ^ (x >> 31)
+
+
+@pytest.mark.parametrize("rows", [32, 96, 2080, 8192])
+def test_network_batch_sizes(E, c2_system, rows):
+    """Gradient of a batch and one training step at the ends of the batch range, against the oracle.
+
+    The gradient's bounds are those of the network's own tests (bfloat16
+    roundings on either side of a tie).  The step's batch is rebuilt on the
+    host: its loss differs by the targets' rounding to float only (about 1e-6),
+    and a first Adam step moves a parameter by lr against its gradient's sign,
+    checked where the gradient is well clear of zero.
+    """
+    from oracle import surrogate as SO
+    eng = E.Engine([c2_system])
+    eng.surrogate_setup(eng.n_atoms, seed=7)
+    p = SO.init_params(4).astype(np.float32)
+    eng.surrogate_params(p)
+    eng.set_positions(c2_system.pos)
+    n = eng.surrogate_collect()
+    x = eng.surrogate_descriptors(c2_system.pos)
+    eng.total_force(c2_system.pos)
+    r = eng.born_radii()[0]
+    seed, lr = 3, 2e-3
+    sd = seed * 0x9E3779B97F4A7C15 & ((1 << 64) - 1)
+    pick = np.array([_mix(sd ^ _mix(b)) % n for b in range(rows)])
+    g, loss = eng.surrogate_gradient(x[pick], r[pick])
+    gref, lref = SO.gradient(p.astype(np.float64), x[pick].astype(np.float64), r[pick])
+    assert abs(loss - lref) <= 1e-3 * lref
+    for a, b in ((SO.OFF_W1, SO.OFF_B1), (SO.OFF_B1, SO.OFF_W2), (SO.OFF_W2, SO.OFF_B2), (SO.OFF_B2, SO.OFF_W3),
+                 (SO.OFF_W3, SO.OFF_B3), (SO.OFF_B3, SO.P)):
+        assert np.linalg.norm(g[a:b] - gref[a:b]) < 2e-2 * np.linalg.norm(gref[a:b])
+    first = eng.surrogate_train(1, batch=rows, lr=lr, seed=seed)
+    assert abs(first[0] - loss) <= 1e-4 * loss
+    clear = np.abs(g) > 1e-3 * np.abs(g).max()
+    moved = eng.surrogate_params().astype(np.float64) - p
+    assert np.abs(moved + lr * np.sign(g))[clear].max() < 1e-3 * lr
+
+
+def test_network_losses_of_long_runs(E, c1_system):
+    """Every step's loss comes back, also past the number that is held on the device."""
+    eng = E.Engine([c1_system])
+    got = []
+    for steps in (1030, 1024, 3):
+        eng.surrogate_setup(eng.n_atoms, seed=1)
+        eng.set_positions(c1_system.pos)
+        eng.surrogate_collect()
+        got.append(eng.surrogate_train(steps, batch=32, lr=1e-3, seed=9))
+    assert np.all(got[0] > 0.0)
+    assert np.array_equal(got[0][:1024], got[1]) and np.array_equal(got[0][:3], got[2])
