@@ -15,7 +15,7 @@
 #define OG_SUR_H 128          // hidden width
 #define OG_SUR_OFF_W1 0                                   // [K1][H] input-major
 #define OG_SUR_OFF_B1 (OG_SUR_OFF_W1 + OG_SUR_K1 * OG_SUR_H)
-#define OG_SUR_OFF_W2 (OG_SUR_OFF_B1 + OG_SUR_H)          // [H][H] input-major
+#define OG_SUR_OFF_W2 (OG_SUR_OFF_B1 + OG_SUR_H)          // layer 2 transposed, by MFMA operands
 #define OG_SUR_OFF_B2 (OG_SUR_OFF_W2 + OG_SUR_H * OG_SUR_H)
 #define OG_SUR_OFF_W3 (OG_SUR_OFF_B2 + OG_SUR_H)
 #define OG_SUR_OFF_B3 (OG_SUR_OFF_W3 + OG_SUR_H)
@@ -45,9 +45,9 @@ struct og_sur {
     unsigned* dev = nullptr;           // [S] max relative deviation (float bits), last check
     // parameters (FP32 master) and BF16 copies for the MFMA layers
     float *p = nullptr, *m = nullptr, *v = nullptr, *g = nullptr;
-    unsigned short *W1t = nullptr;     // [H][K1] output-major
-    unsigned short *W2t = nullptr;     // [H][H] output-major
-    unsigned short *W2i = nullptr;     // [H][H] input-major
+    unsigned short *W1t = nullptr;     // layer 1, by MFMA operands
+    unsigned short *W2t = nullptr;     // layer 2, by MFMA operands
+    unsigned short *W2i = nullptr;     // layer 2 transposed, by MFMA operands
     int adam_t = 0;
     // training set
     long long cap = 0, n_train = 0;

@@ -13,9 +13,11 @@
 //
 // Layouts (bf16 stored as raw 16-bit words):
 //   X    [rows][192]  descriptors (row-major)       -> A operand, layer 1
-//   W1t  [128][192]   layer-1 weights, output-major  -> B operand, layer 1
-//   W2t  [128][128]   layer-2 weights, output-major  -> B operand, layer 2
-//   W2i  [128][128]   layer-2 weights, input-major   -> B operand, dH1 = dZ2 W2^T
+//   W1t  layer-1 weights                             -> B operand, layer 1
+//   W2t  layer-2 weights                             -> B operand, layer 2
+//   W2i  layer-2 weights transposed                  -> B operand, dH1 = dZ2 W2^T
+//        each by operands, [column / 16][k / 32][lane][8]: a wave's load of
+//        one is 1 KB in a run (by rows it was 16 pieces of 64 bytes)
 //   *T   [batch/16][feature][16] activations          -> operands of the
 //        weight-gradient GEMMs, whose reduction runs over the batch.
 #include <hip/hip_runtime.h>
@@ -92,25 +94,46 @@ struct DescArgs {
 
 }  // namespace
 
-// Descriptor: one 256-thread block per 64-atom tile I.  The block lists the
-// tiles J of the same system whose bounding spheres come within 12 Å of
-// tile I, then its four waves take those tiles in turn: lane = atom i, the
-// atoms j of tile J are broadcast one by one, and every j != i with r < 12 Å
-// adds one count to i's histogram row in LDS (integer counts, so the result
-// does not depend on the order).  The bin floor(r / 0.375 Å) is estimated
-// from a single-precision square root and then settled exactly on r^2
-// against the bin edges (0.375 k)^2 = 0.140625 k^2, which are exact in FP64.
+// Descriptor: one block per 64-atom tile I.  The block lists the tiles J of
+// the same system whose bounding spheres come within 12 Å of tile I, then its
+// eight waves take halves of those tiles in turn: lane = atom i, the atoms j
+// are broadcast one by one, and every j != i with r < 12 Å adds one count to
+// i's histogram row in LDS (integer counts, so the result does not depend on
+// the order).  Instruction issue bounds the kernel, so the bin floor(r / 0.375
+// Å) is read off single-precision distances about tile I's centre; a lane
+// whose r / 0.375 Å comes within SUR_EDGE of a whole number (each bin's edge,
+// the range's end at 32 and a pair of coincident atoms are such) settles the
+// bin on FP64 r^2 against the edges (0.375 k)^2 = 0.140625 k^2, which are
+// exact.  With atoms i within SUR_NEAR_A of the centre a coordinate difference
+// of a pair in range is off by at most 8.1e-6 Å, so r / 0.375 Å by 4.5e-5;
+// a tile that reaches further settles every pair in FP64.  About one wave step
+// in fifty has such a lane.  30 520 atoms of 16 chains: 67 us with FP64
+// distances and four waves, 25 us this way.
 // Counts are 16-bit, two bins to a word (25 KB of LDS per block, so that the
 // kernel fits beside the SASA arrangement on a CU).
-#define SUR_DESC_WAVES 4
+#define SUR_DESC_WAVES 8
 #define SUR_HW ((OG_SUR_F + 1) / 2)                     // words per histogram row (81)
+#define SUR_EDGE 1.0e-4f
+#define SUR_NEAR_A 64.0
+
+// bin of r^2, or 32 and more beyond the range
+__device__ __forceinline__ int desc_bin(double dx, double dy, double dz) {
+    const double r2 = dx * dx + dy * dy + dz * dz;
+    if (!(r2 < 144.0)) return 32;
+    int k = (int)(sqrtf((float)r2) * (1.0f / 0.375f));
+    k = k > 31 ? 31 : (k < 0 ? 0 : k);
+    while (k < 31 && 0.140625 * (double)((k + 1) * (k + 1)) <= r2) ++k;
+    while (k > 0 && 0.140625 * (double)(k * k) > r2) --k;
+    return k;
+}
+
 __global__ void __launch_bounds__(64 * SUR_DESC_WAVES) og_k_sur_desc(DescArgs a) {
     __shared__ unsigned hist[64 * SUR_HW];            // odd stride: conflict-free rows
     __shared__ int near_list[1024];
     __shared__ int n_near;
     const int t = blockIdx.x;
     const int tid = threadIdx.x;
-    const int lane = tid & 63, wv = tid >> 6;
+    const int lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int sys = a.tile_sys[t];
     if (a.mode && !a.mode[sys]) return;
     for (int q = tid; q < 64 * SUR_HW; q += blockDim.x) hist[q] = 0u;
@@ -132,12 +155,16 @@ __global__ void __launch_bounds__(64 * SUR_DESC_WAVES) og_k_sur_desc(DescArgs a)
     const int a0 = a.tile_atom0[t], cnt = a.tile_cnt[t];
     const bool vi = lane < cnt;
     const int i = a0 + lane;
+    const float edge = bi.w <= SUR_NEAR_A ? SUR_EDGE : 1.0f;   // 1: every pair in FP64
     double xi = 0.0, yi = 0.0, zi = 0.0;
     if (vi) { xi = a.pos[3 * (size_t)i]; yi = a.pos[3 * (size_t)i + 1]; zi = a.pos[3 * (size_t)i + 2]; }
+    // lanes without an atom stay out of every range
+    const float fx = vi ? (float)(xi - bi.x) : 1.0e9f, fy = (float)(yi - bi.y), fz = (float)(zi - bi.z);
     unsigned* row = hist + lane * SUR_HW;
-    for (int q = wv; q < nn; q += SUR_DESC_WAVES) {
-        const int J = near_list[q];
-        const int b0 = a.tile_atom0[J], cj = a.tile_cnt[J];
+    for (int q = wv; q < 2 * nn; q += SUR_DESC_WAVES) {
+        const int J = near_list[q >> 1];
+        const int b0 = a.tile_atom0[J] + (q & 1) * 32;
+        const int cj = a.tile_cnt[J] - (q & 1) * 32 < 32 ? a.tile_cnt[J] - (q & 1) * 32 : 32;
         double xj = 0.0, yj = 0.0, zj = 0.0;
         int cl = 0;
         if (lane < cj) {
@@ -145,28 +172,63 @@ __global__ void __launch_bounds__(64 * SUR_DESC_WAVES) og_k_sur_desc(DescArgs a)
             xj = a.pos[j]; yj = a.pos[j + 1]; zj = a.pos[j + 2];
             cl = a.cls[b0 + lane];
         }
-        for (int jj = 0; jj < cj; ++jj) {
-            const double dx = rld(xj, jj) - xi, dy = rld(yj, jj) - yi, dz = rld(zj, jj) - zi;
-            const int c = __builtin_amdgcn_readlane(cl, jj);
-            const double r2 = dx * dx + dy * dy + dz * dz;
-            if (vi && b0 + jj != i && r2 < 144.0) {
-                int k = (int)(sqrtf((float)r2) * (1.0f / 0.375f));
-                k = k > 31 ? 31 : (k < 0 ? 0 : k);
-                while (k < 31 && 0.140625 * (double)((k + 1) * (k + 1)) <= r2) ++k;
-                while (k > 0 && 0.140625 * (double)(k * k) > r2) --k;
-                const int b = c * 32 + k;
-                atomicAdd(row + (b >> 1), 1u << ((b & 1) * 16));
+        // slots past the tile's atoms stay out of every range
+        const int gx = __float_as_int(lane < cj ? (float)(xj - bi.x) : 3.0e9f), gy = __float_as_int((float)(yj - bi.y)),
+                  gz = __float_as_int((float)(zj - bi.z));
+        for (int j0 = 0; j0 < cj; j0 += 4) {
+            int k[4], c[4];
+            bool in[4], near[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int jj = j0 + u;
+                const float dx = __int_as_float(__builtin_amdgcn_readlane(gx, jj)) - fx,
+                            dy = __int_as_float(__builtin_amdgcn_readlane(gy, jj)) - fy,
+                            dz = __int_as_float(__builtin_amdgcn_readlane(gz, jj)) - fz;
+                c[u] = __builtin_amdgcn_readlane(cl, jj);
+                const float s = __builtin_amdgcn_sqrtf(fmaf(dx, dx, fmaf(dy, dy, dz * dz))) * (1.0f / 0.375f);
+                k[u] = (int)s;
+                in[u] = s < 32.0f;
+                near[u] = vi && !(s >= 32.0f + edge) && !(fabsf(s - rintf(s)) > edge);
             }
+            if (__any(near[0] | near[1] | near[2] | near[3])) {
+#pragma unroll 1
+                for (int u = 0; u < 4; ++u) {
+                    const int jj = j0 + u;
+                    const bool nu = u == 0 ? near[0] : u == 1 ? near[1] : u == 2 ? near[2] : near[3];
+                    const int b = nu && jj < cj && b0 + jj != i
+                                      ? desc_bin(rld(xj, jj) - xi, rld(yj, jj) - yi, rld(zj, jj) - zi) : 32;
+#pragma unroll
+                    for (int q4 = 0; q4 < 4; ++q4)
+                        if (nu && q4 == u) {
+                            k[q4] = b;
+                            in[q4] = b < 32;
+                        }
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (in[u]) {
+                    const int b = c[u] * 32 + k[u];
+                    atomicAdd(row + (b >> 1), 1u << ((b & 1) * 16));
+                }
         }
     }
     __syncthreads();
-    // write the 64 rows: thread per (row, feature)
-    for (int q = tid; q < cnt * OG_SUR_K1; q += blockDim.x) {
-        const int rr = q / OG_SUR_K1, f = q % OG_SUR_K1;
-        unsigned short v = 0;
-        if (f < 160) v = f2bf((float)((hist[rr * SUR_HW + (f >> 1)] >> ((f & 1) * 16)) & 0xFFFFu) * 0.125f);
-        else if (f == 160) v = f2bf((float)((a.rho[a0 + rr] - 1.5) * 4.0));
-        a.X[(size_t)(a0 + rr) * OG_SUR_K1 + f] = v;
+    // write the rows, eight features at a time
+    constexpr int V = OG_SUR_K1 / 8;
+    for (int q = tid; q < cnt * V; q += blockDim.x) {
+        const int rr = q / V, f = (q % V) * 8;
+        unsigned v[4] = {0u, 0u, 0u, 0u};
+        if (f < 160) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const unsigned h = hist[rr * SUR_HW + (f >> 1) + u];
+                v[u] = f2bf((float)(h & 0xFFFFu) * 0.125f) | ((unsigned)f2bf((float)(h >> 16) * 0.125f) << 16);
+            }
+        } else if (f == 160) {
+            v[0] = f2bf((float)((a.rho[a0 + rr] - 1.5) * 4.0));
+        }
+        *reinterpret_cast<uint4*>(a.X + (size_t)(a0 + rr) * OG_SUR_K1 + f) = make_uint4(v[0], v[1], v[2], v[3]);
     }
 }
 
@@ -183,108 +245,91 @@ struct MlpOperands {
     unsigned short *W1t, *W2t, *W2i;
 };
 
+// place of column j, input k in a B operand with kk_n steps of 32 inputs, and
+// a lane's eight inputs of step kk for the 16 columns nt
+__device__ __forceinline__ int operand_at(int j, int k, int kk_n) {
+    return (((j >> 4) * kk_n + (k >> 5)) * 64 + ((k >> 3) & 3) * 16 + (j & 15)) * 8 + (k & 7);
+}
+__device__ __forceinline__ og_bf16x8 operand(const unsigned short* w, int nt, int kk, int kk_n, int lane) {
+    return ld8(w + ((nt * kk_n + kk) * 64 + lane) * 8);
+}
+
 // BF16 operand copy (copies, of W2) of parameter q
 __device__ __forceinline__ void store_operand(const MlpOperands& o, int q, float w) {
     if (q < OG_SUR_OFF_B1) {
         const int k = q / OG_SUR_H, j = q % OG_SUR_H;
-        o.W1t[j * OG_SUR_K1 + k] = f2bf(w);
+        o.W1t[operand_at(j, k, OG_SUR_K1 / 32)] = f2bf(w);
     } else if (q >= OG_SUR_OFF_W2 && q < OG_SUR_OFF_B2) {
         const int e = q - OG_SUR_OFF_W2;
         const int k = e / OG_SUR_H, j = e % OG_SUR_H;
-        o.W2t[j * OG_SUR_H + k] = f2bf(w);
-        o.W2i[k * OG_SUR_H + j] = f2bf(w);
+        o.W2t[operand_at(j, k, OG_SUR_H / 32)] = f2bf(w);
+        o.W2i[operand_at(k, j, OG_SUR_H / 32)] = f2bf(w);
     }
 }
 
 }  // namespace
 
-// Inference, 64 rows per wave: four 16-row groups share every weight
-// fragment load (the weights are read once per 64 rows instead of once per
-// 16).  Each row goes through the 16-row forward's exact operations, so the
-// radii are unchanged.
-// Two waves per block (35 KB of LDS, so that the kernel fits beside the SASA
-// arrangement on a CU).
-__global__ void __launch_bounds__(128) og_k_sur_infer64(const unsigned short* X, int n_valid, int n_rows,
-                                                        MlpParams P, double* r_out) {
-    __shared__ __attribute__((aligned(16))) unsigned short hs[2][64][136];
+// Inference, SUR_INFER_ROWS rows per block: each of the eight waves holds the
+// weights of one 16-column group of both layers in registers and takes the
+// 16-row groups in turn, with the activations exchanged over LDS (26 KB, so
+// that the kernel fits beside the SASA arrangement on a CU).  Every element
+// keeps its MFMA chain and the output sum its order over the column groups.
+// 64 rows per wave, both layers unrolled over the column groups, took 26 us
+// for 30 520 rows; columns over the waves with the rows and weights read in
+// pieces of 64 bytes, eight waves the same rows, 24; rows through LDS and the
+// weights in runs 12, of which about 10 are the exponentials and divisions.
+#define SUR_INFER_ROWS 32
+__global__ void __launch_bounds__(512) og_k_sur_infer(const unsigned short* X, int n_valid, int n_rows,
+                                                      MlpParams P, double* r_out) {
+    __shared__ __attribute__((aligned(16))) unsigned short h1s[SUR_INFER_ROWS][136];
+    __shared__ __attribute__((aligned(16))) union {
+        unsigned short x[SUR_INFER_ROWS][OG_SUR_K1 + 8];
+        float h2[8][SUR_INFER_ROWS][17];
+    } sh;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int r = lane & 15, g = lane >> 4;
-    const int row0 = (blockIdx.x * 2 + w) * 64;
-    if (row0 >= n_valid) return;
-    unsigned short (*h)[136] = hs[w];
-    og_bf16x8 a1[4][6];
+    const int j = w * 16 + r;
+    const int row0 = blockIdx.x * SUR_INFER_ROWS;
+    og_bf16x8 w1[6], w2[4];
 #pragma unroll
-    for (int rg = 0; rg < 4; ++rg) {
-        const int rr = row0 + rg * 16 + r;
-        const int rs = rr < n_rows ? rr : 0;
+    for (int kk = 0; kk < 6; ++kk) w1[kk] = operand(P.W1t, w, kk, OG_SUR_K1 / 32, lane);
 #pragma unroll
-        for (int kk = 0; kk < 6; ++kk) a1[rg][kk] = ld8(X + (size_t)rs * OG_SUR_K1 + kk * 32 + g * 8);
+    for (int kk = 0; kk < 4; ++kk) w2[kk] = operand(P.W2t, w, kk, OG_SUR_H / 32, lane);
+    const float b1 = P.p[OG_SUR_OFF_B1 + j], b2 = P.p[OG_SUR_OFF_B2 + j];
+    for (int q = threadIdx.x; q < SUR_INFER_ROWS * (OG_SUR_K1 / 8); q += 512) {
+        const int rr = q / (OG_SUR_K1 / 8), c = q % (OG_SUR_K1 / 8) * 8;
+        *reinterpret_cast<og_bf16x8*>(&sh.x[rr][c]) = ld8(X + (size_t)(row0 + rr < n_rows ? row0 + rr : 0) * OG_SUR_K1 + c);
     }
+    __syncthreads();
 #pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {
-        og_f32x4 acc[4];
+    for (int rg = 0; rg < SUR_INFER_ROWS; rg += 16) {
+        og_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int rg = 0; rg < 4; ++rg) acc[rg] = og_f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int kk = 0; kk < 6; ++kk) acc = mfma(ld8(&sh.x[rg + r][kk * 32 + g * 8]), w1[kk], acc);
 #pragma unroll
-        for (int kk = 0; kk < 6; ++kk) {
-            const og_bf16x8 bw = ld8(P.W1t + (size_t)(nt * 16 + r) * OG_SUR_K1 + kk * 32 + g * 8);
-#pragma unroll
-            for (int rg = 0; rg < 4; ++rg) acc[rg] = mfma(a1[rg][kk], bw, acc[rg]);
-        }
-        const float b = P.p[OG_SUR_OFF_B1 + nt * 16 + r];
-#pragma unroll
-        for (int rg = 0; rg < 4; ++rg)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float z = acc[rg][i] + b;
-                h[rg * 16 + g * 4 + i][nt * 16 + r] = f2bf(silu(z));
-            }
+        for (int i = 0; i < 4; ++i) h1s[rg + g * 4 + i][j] = f2bf(silu(acc[i] + b1));
     }
-    wave_sync();
-    og_bf16x8 a2[4][4];
+    __syncthreads();
 #pragma unroll
-    for (int rg = 0; rg < 4; ++rg)
+    for (int rg = 0; rg < SUR_INFER_ROWS; rg += 16) {
+        og_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) a2[rg][kk] = ld8(&h[rg * 16 + r][kk * 32 + g * 8]);
-    float ys[4][4];
+        for (int kk = 0; kk < 4; ++kk) acc = mfma(ld8(&h1s[rg + r][kk * 32 + g * 8]), w2[kk], acc);
 #pragma unroll
-    for (int rg = 0; rg < 4; ++rg)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ys[rg][i] = 0.f;
-#pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {
-        og_f32x4 acc[4];
-#pragma unroll
-        for (int rg = 0; rg < 4; ++rg) acc[rg] = og_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            const og_bf16x8 bw = ld8(P.W2t + (size_t)(nt * 16 + r) * OG_SUR_H + kk * 32 + g * 8);
-#pragma unroll
-            for (int rg = 0; rg < 4; ++rg) acc[rg] = mfma(a2[rg][kk], bw, acc[rg]);
-        }
-        const float b = P.p[OG_SUR_OFF_B2 + nt * 16 + r];
-        const float wv = P.p[OG_SUR_OFF_W3 + nt * 16 + r];
-#pragma unroll
-        for (int rg = 0; rg < 4; ++rg)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float z = acc[rg][i] + b;
-                ys[rg][i] += silu(z) * wv;
-            }
+        for (int i = 0; i < 4; ++i) sh.h2[w][rg + g * 4 + i][r] = silu(acc[i] + b2);
     }
+    __syncthreads();
+    // a wave sums four rows: over the column groups in order, then the columns
+    const int row = w * 4 + g;
+    float v = 0.0f;
 #pragma unroll
-    for (int rg = 0; rg < 4; ++rg)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float v = ys[rg][i];
-            v += __shfl_xor(v, 1, 64);
-            v += __shfl_xor(v, 2, 64);
-            v += __shfl_xor(v, 4, 64);
-            v += __shfl_xor(v, 8, 64);
-            const float y = v + P.p[OG_SUR_OFF_B3];
-            const int row = row0 + rg * 16 + g * 4 + i;
-            if (r == 0 && row < n_valid) r_out[row] = OG_SUR_R0 + OG_SUR_RS * (double)y;
-        }
+    for (int nt = 0; nt < 8; ++nt) v += sh.h2[nt][row][r] * P.p[OG_SUR_OFF_W3 + nt * 16 + r];
+    v += __shfl_xor(v, 1, 64);
+    v += __shfl_xor(v, 2, 64);
+    v += __shfl_xor(v, 4, 64);
+    v += __shfl_xor(v, 8, 64);
+    const float y = v + P.p[OG_SUR_OFF_B3];
+    if (r == 0 && row0 + row < n_valid) r_out[row0 + row] = OG_SUR_R0 + OG_SUR_RS * (double)y;
 }
 
 __device__ __forceinline__ unsigned long long sur_mix(unsigned long long x) {
@@ -315,7 +360,7 @@ __device__ __forceinline__ unsigned long long sur_mod(unsigned long long h, unsi
 // itself).  What the weight gradients read is left by groups of 16 rows,
 // [B/16][columns][16]: a block writes whole lines, and a wave there reads the
 // 32 rows of 16 columns as two runs of 512 bytes.  At 4 096 rows 50 us before
-// (40 and a separate gather's 10), 16 now, of which 9 are the chain (2 blocks
+// (40 and a separate gather's 10), 14 now, of which 7 are the chain (2 blocks
 // take as long) and the rest the 11 MB written.
 __device__ __forceinline__ size_t sur_at(int col, int row, int cols) {
     return ((size_t)(row >> 4) * cols + col) * 16 + (row & 15);
@@ -353,11 +398,11 @@ __global__ void __launch_bounds__(512) og_k_sur_fwdbwd(TrainArgs a, MlpParams P)
     // the weights load first, while the row's index is formed
     og_bf16x8 a1[6], w1[6], w2[4], w2i[4];
 #pragma unroll
-    for (int kk = 0; kk < 6; ++kk) w1[kk] = ld8(P.W1t + (size_t)j * OG_SUR_K1 + kk * 32 + g * 8);
+    for (int kk = 0; kk < 6; ++kk) w1[kk] = operand(P.W1t, w, kk, OG_SUR_K1 / 32, lane);
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) w2[kk] = ld8(P.W2t + (size_t)j * OG_SUR_H + kk * 32 + g * 8);
+    for (int kk = 0; kk < 4; ++kk) w2[kk] = operand(P.W2t, w, kk, OG_SUR_H / 32, lane);
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) w2i[kk] = ld8(P.W2i + (size_t)j * OG_SUR_H + kk * 32 + g * 8);
+    for (int kk = 0; kk < 4; ++kk) w2i[kk] = operand(P.W2i, w, kk, OG_SUR_H / 32, lane);
     const float b1 = P.p[OG_SUR_OFF_B1 + j], b2 = P.p[OG_SUR_OFF_B2 + j], w3 = P.p[OG_SUR_OFF_W3 + j];
     const float b3 = P.p[OG_SUR_OFF_B3];
     float w3c[8];
@@ -777,8 +822,7 @@ int og_sur_descriptors(og_sur* s, bool all) {
 
 int og_sur_infer(og_sur* s) {
     if (s->n_atoms == 0) return 0;
-    const int waves64 = (s->n_atoms + 63) / 64;
-    hipLaunchKernelGGL(og_k_sur_infer64, dim3((waves64 + 1) / 2), dim3(128), 0, s->stream, s->X, s->n_atoms,
+    hipLaunchKernelGGL(og_k_sur_infer, dim3((s->n_atoms + SUR_INFER_ROWS - 1) / SUR_INFER_ROWS), dim3(512), 0, s->stream, s->X, s->n_atoms,
                        s->n_pad, params_of(s), s->r_sur);
     return hipGetLastError() == hipSuccess ? 0 : fail("kernel launch failed");
 }

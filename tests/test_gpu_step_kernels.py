@@ -228,3 +228,41 @@ def test_network_losses_of_long_runs(E, c1_system):
         got.append(eng.surrogate_train(steps, batch=32, lr=1e-3, seed=9))
     assert np.all(got[0] > 0.0)
     assert np.array_equal(got[0][:1024], got[1]) and np.array_equal(got[0][:3], got[2])
+
+
+@pytest.mark.parametrize("chains", [[(16, 4)], [(21, 4), (3, 3)], [(9, 15), (16, 4)], [(2, 70)]])
+@pytest.mark.parametrize("places", ["lattice", "nudged", "far", "spread"])
+def test_descriptors_at_bin_edges(E, chains, places):
+    """Neighbour counts with distances on and next to the bin edges, coincident atoms, far origins and wide tiles.
+
+    The counts are whole numbers and exact.  On a lattice of the bin width
+    every distance along an axis is an edge; the nudged one is off by 1e-9 of
+    itself either way; the spread one reaches beyond the range in which the
+    kernel forms single-precision distances.  The radii that follow are those
+    of the network's own test's bound.
+    """
+    from oracle import surrogate as SO
+    systems = [S.seeded_chain(*c) for c in chains]
+    rng = np.random.default_rng(5)
+    pos = []
+    for s in systems:
+        x = 0.375 * rng.integers(-16, 17, size=(s.n_atoms, 3)).astype(np.float64)
+        x[::5, 1:] = 0.0                        # a fifth on one axis
+        if places == "nudged":
+            x *= 1.0 + 1e-9 * rng.choice([-1.0, 1.0], size=x.shape)
+        elif places == "far":
+            x += 375.0 * 64
+        elif places == "spread":
+            x[1::3] *= 24.0
+        pos.append(x)
+    pos = np.concatenate(pos)
+    eng = E.Engine(systems)
+    eng.surrogate_setup(0, seed=1)
+    x = eng.surrogate_descriptors(pos)
+    mass = np.concatenate([s.mass for s in systems])
+    rho = np.concatenate([s.gb_rho for s in systems])
+    assert np.array_equal(x.astype(np.float64), SO.descriptors(pos, mass, rho, eng.offsets))
+    p = SO.init_params(3)
+    eng.surrogate_params(p.astype(np.float32))
+    ref = SO.radius(SO.forward(p, x.astype(np.float64))[0])
+    assert np.abs(eng.surrogate_radii(pos) / ref - 1.0).max() < 1e-3
