@@ -139,36 +139,92 @@ OG_HD int intersect_count_fast(const Cap& c1, const Cap& c2) {
 // (orthonormal in-plane basis u, v) on which cap m's containment value
 // dot(X, n_m) - cos a_m is at least SA_COV_DELTA, as start angle a and width
 // w2 (radians, FP32).  w2 < 0: no usable arc; w2 = SA_COV_FULL: the whole
-// circle.  FP64 up to the final angles; acosf / atan2f only see arguments
-// where they are well conditioned (|cos| <= 1 - 1e-3, amplitude >= 1e-3),
-// nearly full arcs are cut to width 2 (pi - 0.05) and tiny ones dropped, so
-// both ends lie within 2e-6 rad of the exact arc or inside it.
-// SA_COV_DELTA is also the depth the arrangement kernel requires before it
-// leaves a covered circle's transitions out of the other circles' boundaries
-// (it exceeds the 2.6e-4 that chains of deduplicated points can span).
+// circle.  SA_COV_DELTA is also the depth the arrangement kernel requires
+// before it leaves a covered circle's transitions out of the other circles'
+// boundaries (it exceeds the 2.6e-4 that chains of deduplicated points can
+// span).
+// The value on the circle is g + d + amp cos(phi - phi_m) with g = B - d, d
+// the depth asked for.  Formed in FP32 from the rounded axes and basis, B and
+// amp are off by at most 1e-6 and the arc's ends by an angle that moves the
+// value by at most 2e-6 more (an end's error is the value's divided by its
+// slope), so asking for d = SA_COV_DELTA + SA_COV_SLACK leaves SA_COV_DELTA at
+// every claimed angle, and at angles 1e-5 rad beyond.  Nearly full arcs are
+// cut to width 2 (pi - 0.05), tiny ones (|cos| > 1 - 1e-3) and those of a
+// small amplitude (< 1e-3) dropped.
 #define SA_COV_DELTA 1e-3
+#define SA_COV_SLACK 2e-5
 #define SA_COV_FULL 100.0f
-// The containment value on the circle is g + SA_COV_DELTA + amp cos(phi -
-// phi_m) with g = B - SA_COV_DELTA; the whole-circle and no-arc cases are
-// settled on amp^2 (no square root), the arc itself from amp.
+
+OG_HD inline float cover_rcp(float x) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_rcpf(x);
+#else
+    return 1.0f / x;
+#endif
+}
+OG_HD inline float cover_sqrt(float x) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_sqrtf(x);
+#else
+    return sqrtf(x);
+#endif
+}
+// arc cosine, Abramowitz and Stegun 4.4.46 (2e-8 before rounding)
+OG_HD inline float cover_acos(float x) {
+    const float y = fabsf(x);
+    float p = fmaf(-0.0012624911f, y, 0.0066700901f);
+    p = fmaf(p, y, -0.0170881256f);
+    p = fmaf(p, y, 0.0308918810f);
+    p = fmaf(p, y, -0.0501743046f);
+    p = fmaf(p, y, 0.0889789874f);
+    p = fmaf(p, y, -0.2145988016f);
+    p = fmaf(p, y, 1.5707963050f);
+    p *= cover_sqrt(1.0f - y);
+    return x < 0.0f ? 3.14159265358979f - p : p;
+}
+// angle of (x, y) != 0 from the arc tangent, Abramowitz and Stegun 4.4.49 (2e-8)
+OG_HD inline float cover_atan2(float y, float x) {
+    const float ax = fabsf(x), ay = fabsf(y);
+    const float t = fminf(ax, ay) * cover_rcp(fmaxf(ax, ay)), q = t * t;
+    float p = fmaf(0.0028662257f, q, -0.0161657367f);
+    p = fmaf(p, q, 0.0429096138f);
+    p = fmaf(p, q, -0.0752896400f);
+    p = fmaf(p, q, 0.1065626393f);
+    p = fmaf(p, q, -0.1420889944f);
+    p = fmaf(p, q, 0.1999355085f);
+    p = fmaf(p, q, -0.3333314528f);
+    p = fmaf(p * q, t, t);
+    p = ay > ax ? 1.57079632679490f - p : p;
+    p = x < 0.0f ? 3.14159265358979f - p : p;
+    return y < 0.0f ? -p : p;
+}
+
+// circle k for the cover test: axis and cosine, basis, squared sine
+struct CoverCircle {
+    float nx, ny, nz, ca, ux, uy, uz, vx, vy, vz, s2;
+};
+OG_HD inline CoverCircle cover_circle(const Cap& c, v3 u, v3 v) {
+    return {(float)c.axis.x, (float)c.axis.y, (float)c.axis.z, (float)c.ca, (float)u.x, (float)u.y, (float)u.z,
+            (float)v.x, (float)v.y, (float)v.z, (float)fmax(1.0 - c.ca * c.ca, 0.0)};
+}
+// cap m as (axis, cosine) in FP32.  The whole-circle and no-arc cases are
+// settled on amp^2.
+OG_HD inline void cover_arc(const CoverCircle& k, float mx, float my, float mz, float mc, float& a, float& w2) {
+    const float ct = fmaf(k.nz, mz, fmaf(k.ny, my, k.nx * mx));
+    const float x = fmaf(k.uz, mz, fmaf(k.uy, my, k.ux * mx));
+    const float y = fmaf(k.vz, mz, fmaf(k.vy, my, k.vx * mx));
+    const float amp2 = k.s2 * fmaf(x, x, y * y);
+    const float g = fmaf(k.ca, ct, -mc) - (float)(SA_COV_DELTA + SA_COV_SLACK);
+    const float amp = cover_sqrt(amp2);
+    const float c = -g * cover_rcp(amp);
+    float w = c <= -1.0f + 1e-3f ? (float)(3.14159265358979323846 - 0.05) : cover_acos(c);
+    const bool arc = amp2 >= 1e-6f && c < 1.0f - 1e-3f;
+    const bool full = g >= amp;
+    a = arc && !full ? cover_atan2(y, x) - w : 0.0f;
+    w2 = full ? SA_COV_FULL : arc ? 2.0f * w : -1.0f;
+}
 OG_HD inline void cover_arc(const Cap& ck, const Cap& cm, v3 u, v3 v, float& a, float& w2) {
-    const double ct = dot(ck.axis, cm.axis);
-    const double x = dot(cm.axis, u), y = dot(cm.axis, v);
-    const double amp2 = fmax(1.0 - ck.ca * ck.ca, 0.0) * (x * x + y * y);
-    const double g = (ck.ca * ct - cm.ca) - SA_COV_DELTA;
-    a = 0.0f;
-    w2 = -1.0f;
-    if (g >= 0.0 && g * g >= amp2) {
-        w2 = SA_COV_FULL;                              // g >= amp
-    } else if (amp2 >= 1e-6 && !(g <= 0.0 && g * g >= 0.998001 * amp2)) {
-        // amp >= 1e-3, and not -g >= (1 - 1e-3) amp (no arc)
-        const double c = -g / sqrt(amp2);
-        if (c < 1.0 - 1e-3) {
-            const float w = c <= -1.0 + 1e-3 ? (float)(3.14159265358979323846 - 0.05) : acosf((float)c);
-            a = atan2f((float)y, (float)x) - w;
-            w2 = 2.0f * w;
-        }
-    }
+    cover_arc(cover_circle(ck, u, v), (float)cm.axis.x, (float)cm.axis.y, (float)cm.axis.z, (float)cm.ca, a, w2);
 }
 
 // In-plane basis of a circle (arrangement.rs:233-248): u from the helper

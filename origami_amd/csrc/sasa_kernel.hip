@@ -53,8 +53,6 @@
 #define SA_WAVES 2                    // waves per block (arrangement, scatter)
 #define SA_TMAX 256                   // transitions per chunk (>= 2 * (MAXC - 1))
 #define SA_NC_MAIN 80                 // caps per atom in the main arrangement pass
-#define SA_COV_CAPS (SA_TMAX / 6)     // union cover test: circles per batch (bases in ta)
-#define SA_COV_PAIRS (3 * SA_TMAX)    // union cover test: arcs per batch (in tx..tz)
 #define SA_COV_EPS 1e-5f              // cover margin on angles (rad)
 #define SA_FORCE_BLOCKS_CU 3          // default arrangement blocks per CU beside the pair kernels
 #define SA_ONE_EACH_CU 4              // up to so many where every atom then has its own wave
@@ -108,7 +106,8 @@ static_assert(offsetof(ArrLds<SA_NC_MAIN>, est) == offsetof(ArrLds<SA_NC_MAIN>, 
 // the caps phase buffers atom indices in perm (64 ints)
 static_assert(offsetof(ArrLds<SA_NC_MAIN>, perm) % 4 == 0 && offsetof(ArrLds<MAXC>, perm) % 4 == 0,
               "perm must be 4-aligned");
-// the union cover test stores its arcs across tx, ty and tz
+// the union cover test stores its caps in ta, its circles across tx and ty
+static_assert(SA_TMAX * sizeof(double) >= MAXC * sizeof(float4), "ta holds the caps in FP32");
 static_assert(offsetof(ArrLds<SA_NC_MAIN>, tz) == offsetof(ArrLds<SA_NC_MAIN>, tx) + 2 * SA_TMAX * sizeof(double),
               "tx, ty, tz must be contiguous");
 static_assert(offsetof(ArrLds<MAXC>, tz) == offsetof(ArrLds<MAXC>, tx) + 2 * SA_TMAX * sizeof(double),
@@ -681,10 +680,8 @@ __device__ int4 arrange_atom(ArrLds<NC>& L, const og_sasa_data& d, const double*
     // sin a_k (cos(phi) u + sin(phi) v)), cap m's test value is
     // f_m(phi) = B + sin a_k sin(t) cos(phi - phi_m) with B = cos a_k cos(t)
     // - cos a_m (t: angle between the axes), so f_m >= SA_COV_DELTA on the
-    // arc |phi - phi_m| <= w_m.  Those arcs are formed in FP64 up to the
-    // angles, which come from atan2f/acosf on well-conditioned arguments
-    // (|cos w_m| <= 1 - 1e-3, sin a_k sin t >= 1e-3; nearly full arcs are
-    // cut to pi - 0.05, tiny ones dropped): each angle is within 2e-6 rad.
+    // arc |phi - phi_m| <= w_m.  Those arcs are formed in FP32, SA_COV_SLACK
+    // inside that depth (see cover_arc).
     // A greedy walk from the end of the widest arc then steps, each time, to
     // the end of the arc that contains the current angle with SA_COV_EPS
     // (1e-5 rad) to spare and reaches furthest; reaching back into the
@@ -708,90 +705,92 @@ __device__ int4 arrange_atom(ArrLds<NC>& L, const og_sasa_data& d, const double*
     }
     wave_sync();
     if (n_cand > 0 && nc > 1) {
-        double* bas = L.ta;                                      // [SA_COV_CAPS] x (u, v)
-        float2* iv = reinterpret_cast<float2*>(L.tx);            // [SA_COV_PAIRS] (start, width)
-        const int per_batch = SA_COV_CAPS < SA_COV_PAIRS / nper ? SA_COV_CAPS : SA_COV_PAIRS / nper;
-        for (int c0 = 0; c0 < n_cand; c0 += per_batch) {
-            const int nb = n_cand - c0 < per_batch ? n_cand - c0 : per_batch;
-            for (int ci = lane; ci < nb; ci += 64) {
-                v3 u, v;
-                circle_basis(cap_at(L, L.hl[c0 + ci]), u, v);
-                double* o = bas + 6 * ci;
-                o[0] = u.x; o[1] = u.y; o[2] = u.z; o[3] = v.x; o[4] = v.y; o[5] = v.z;
-            }
-            wave_sync();
-            for (int p = lane; p < nb * nper; p += 64) {
-                const int ci = pair_q(pdiv, p), mi = p - ci * nper;
-                const int k = L.hl[c0 + ci];
-                const int m = mi < k ? mi : mi + 1;
-                const double* o = bas + 6 * ci;
-                float a, wd2;
-                cover_arc(cap_at(L, k), cap_at(L, m), mk(o[0], o[1], o[2]), mk(o[3], o[4], o[5]), a, wd2);
-                iv[p] = make_float2(a, wd2);
-            }
-            wave_sync();
-            // The walk, four circles at a time, one per 16-lane row (lane l
-            // of row r holds arcs l, l + 16, ... of circle g0 + r): each
-            // circle takes exactly its own steps, from the end of its widest
-            // arc (the first of equal widths), each step to the furthest
-            // reach of the arcs that contain the current angle with
-            // SA_COV_EPS to spare; rows that are done stay as they are.  The
-            // slots per lane (NS) are a compile-time count, the smallest of
-            // 1, 2, 3, 4 and 8 that holds the circle's nper arcs (the extra
-            // slots are empty), so the step loop has no branches per slot.
-            const int row = lane >> 4, lr = lane & 15;
-            auto walk = [&](auto ns) {
-                constexpr int NS = decltype(ns)::value;
-                for (int g0 = 0; g0 < nb; g0 += 4) {
-                    const int ci = g0 + row;
-                    const bool rv = ci < nb;
-                    float2 e[NS];
-                    bool full = false;
-                    float wl = 0.0f;
-#pragma unroll
-                    for (int q = 0; q < NS; ++q) {
-                        const int mi = lr + 16 * q;
-                        e[q] = (rv && mi < nper) ? iv[ci * nper + mi] : make_float2(0.0f, -1.0f);
-                        full = full || e[q].y >= SA_COV_FULL;
-                        wl = fmaxf(wl, e[q].y);
-                    }
-                    const bool rfull = ((__ballot(full) >> (16 * row)) & 0xFFFFull) != 0;
-                    const float wm = __uint_as_float(row_lane15(row_umax(__float_as_uint(wl)), row));
-                    unsigned first = 0xFFFFu;
-#pragma unroll
-                    for (int q = NS - 1; q >= 0; --q)
-                        first = e[q].y == wm ? (unsigned)(lr + 16 * q) : first;
-                    first = row_lane15(row_umin(first), row);
-                    bool act = rv && !rfull && wm > 0.0f;
-                    bool cov = rv && rfull;
-                    float start = 0.0f, len = 0.0f, t = 0.0f;
-                    if (act) {
-                        start = iv[ci * nper + (int)first].x + wm;
-                        len = 6.28318530717958647692f - wm;
-                    }
-                    for (int step = 0; step <= nper + 1; ++step) {
-                        if (!__ballot(act)) break;
-                        const float p = start + t;
-                        float ext = 0.0f;
-#pragma unroll
-                        for (int q = 0; q < NS; ++q) ext = fmaxf(ext, cover_ext(p, e[q]));
-                        const float best = __uint_as_float(row_lane15(row_umax(__float_as_uint(act ? ext : 0.0f)), row));
-                        const bool adv = act && best > 0.0f;
-                        t = adv ? t + best : t;
-                        const bool done = adv && t >= len + SA_COV_EPS;
-                        cov = cov || done;
-                        act = adv && !done;
-                    }
-                    if (lr == 0 && cov) L.skip[L.hl[c0 + ci]] = 10;
-                }
-            };
-            if (nper <= 16) walk(std::integral_constant<int, 1>{});
-            else if (nper <= 32) walk(std::integral_constant<int, 2>{});
-            else if (nper <= 48) walk(std::integral_constant<int, 3>{});
-            else if (nper <= 64) walk(std::integral_constant<int, 4>{});
-            else walk(std::integral_constant<int, 8>{});
-            wave_sync();
+        float4* capf = reinterpret_cast<float4*>(L.ta);          // [nc] caps in FP32
+        float4* bas = reinterpret_cast<float4*>(L.tx);           // [n_cand] x (u, s2), (v, -)
+        for (int m = lane; m < nc; m += 64) {
+            const double4 c = L.cap4[m];
+            capf[m] = make_float4((float)c.x, (float)c.y, (float)c.z, (float)c.w);
         }
+        for (int ci = lane; ci < n_cand; ci += 64) {
+            v3 u, v;
+            const Cap ck = cap_at(L, L.hl[ci]);
+            circle_basis(ck, u, v);
+            const CoverCircle cc = cover_circle(ck, u, v);
+            bas[2 * ci] = make_float4(cc.ux, cc.uy, cc.uz, cc.s2);
+            bas[2 * ci + 1] = make_float4(cc.vx, cc.vy, cc.vz, 0.0f);
+        }
+        wave_sync();
+        // Arcs and walk, four circles at a time, one per 16-lane row (lane l of
+        // row r forms and holds the arcs by caps l, l + 16, ... of circle
+        // g0 + r; its own index gives an empty one): each circle takes exactly
+        // its own steps, from the end of its widest arc (the first of equal
+        // widths), each step to the furthest reach of the arcs that contain
+        // the current angle with SA_COV_EPS to spare; rows that are done stay
+        // as they are.  The slots per lane (NS) are a compile-time count, the
+        // smallest of 1, 2, 3, 4 and 8 that holds nc arcs (the extra slots are
+        // empty), so the step loop has no branches per slot.
+        const int row = lane >> 4, lr = lane & 15;
+        auto walk = [&](auto ns) {
+            constexpr int NS = decltype(ns)::value;
+            for (int g0 = 0; g0 < n_cand; g0 += 4) {
+                const int ci = g0 + row;
+                const bool rv = ci < n_cand;
+                const int k = L.hl[rv ? ci : 0];
+                const float4 nk = capf[k], uk = bas[rv ? 2 * ci : 0], vk = bas[rv ? 2 * ci + 1 : 1];
+                const CoverCircle cc = {nk.x, nk.y, nk.z, nk.w, uk.x, uk.y, uk.z, vk.x, vk.y, vk.z, uk.w};
+                float2 e[NS];
+                bool full = false;
+                float wl = 0.0f;
+#pragma unroll
+                for (int q = 0; q < NS; ++q) {
+                    const int m = lr + 16 * q;
+                    const float4 cm = capf[m < nc ? m : 0];
+                    cover_arc(cc, cm.x, cm.y, cm.z, cm.w, e[q].x, e[q].y);
+                    if (!rv || m >= nc || m == k) e[q] = make_float2(0.0f, -1.0f);
+                    full = full || e[q].y >= SA_COV_FULL;
+                    wl = fmaxf(wl, e[q].y);
+                }
+                const bool rfull = ((__ballot(full) >> (16 * row)) & 0xFFFFull) != 0;
+                const float wm = __uint_as_float(row_lane15(row_umax(__float_as_uint(wl)), row));
+                // the widest arc's start, from the lane that holds it
+                unsigned first = 0xFFFFu;
+                float sw = 0.0f;
+#pragma unroll
+                for (int q = NS - 1; q >= 0; --q) {
+                    first = e[q].y == wm ? (unsigned)(lr + 16 * q) : first;
+                    sw = e[q].y == wm ? e[q].x : sw;
+                }
+                first = row_lane15(row_umin(first), row);
+                const float s0 = __shfl(sw, 16 * row + (int)(first & 15u), 64);
+                bool act = rv && !rfull && wm > 0.0f;
+                bool cov = rv && rfull;
+                float start = 0.0f, len = 0.0f, t = 0.0f;
+                if (act) {
+                    start = s0 + wm;
+                    len = 6.28318530717958647692f - wm;
+                }
+                for (int step = 0; step <= nc; ++step) {
+                    if (!__ballot(act)) break;
+                    const float p = start + t;
+                    float ext = 0.0f;
+#pragma unroll
+                    for (int q = 0; q < NS; ++q) ext = fmaxf(ext, cover_ext(p, e[q]));
+                    const float best = __uint_as_float(row_lane15(row_umax(__float_as_uint(act ? ext : 0.0f)), row));
+                    const bool adv = act && best > 0.0f;
+                    t = adv ? t + best : t;
+                    const bool done = adv && t >= len + SA_COV_EPS;
+                    cov = cov || done;
+                    act = adv && !done;
+                }
+                if (lr == 0 && cov) L.skip[k] = 10;
+            }
+        };
+        if (nc <= 16) walk(std::integral_constant<int, 1>{});
+        else if (nc <= 32) walk(std::integral_constant<int, 2>{});
+        else if (nc <= 48) walk(std::integral_constant<int, 3>{});
+        else if (nc <= 64) walk(std::integral_constant<int, 4>{});
+        else walk(std::integral_constant<int, 8>{});
+        wave_sync();
     }
 
     // active caps, ascending
