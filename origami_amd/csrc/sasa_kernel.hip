@@ -30,7 +30,8 @@
 //      ballot-compacted in slot order, which is origami's (k, segment) order.
 //      Vertex root signs and arc->vertex links follow, and the atom's arcs,
 //      vertices and cap owners are appended to a pool.
-//  og_k_sasa_terms    thread per arc or vertex: its JVP terms (role x axis),
+//  og_k_sasa_terms    thread per arc or vertex (og_k_sasa_terms_lanes, for few
+//      atoms: thread per direction of one): its JVP terms (role x axis),
 //      the primal geometry formed once.
 //  og_k_sasa_scatter  one wave per atom, lane per affected atom x: the terms
 //      of every arc (in arc order) and then every vertex (in vertex order)
