@@ -288,6 +288,11 @@ int og_set_temperature(og_engine* e, int32_t system, double temperature_k);
  * lists (checked against a hash taken at og_engine_create). */
 int og_swap_systems(og_engine* e, int32_t a, int32_t b);
 
+/* The exchanges of one round at once: og_swap_systems for the n pairs
+ * (pairs[2k], pairs[2k + 1]), no system in two of them (OG_ERR_ARG
+ * otherwise; nothing is swapped then). */
+int og_swap_pairs(og_engine* e, const int32_t* pairs, int32_t n);
+
 /* Per-system status (OG_STATUS_* bits; 0 = running), SHAKE failure counts,
  * Born-radius clamp counts. */
 int og_get_status(og_engine* e, int32_t* diverged, int32_t* shake_failures, int32_t* clamped);

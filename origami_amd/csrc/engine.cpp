@@ -1889,19 +1889,41 @@ extern "C" int og_frames_read(og_engine* e, double* xyz, uint32_t* steps, int32_
     return OG_OK;
 }
 
-extern "C" int og_swap_systems(og_engine* e, int32_t a, int32_t b) {
-    if (!e || a < 0 || b < 0 || a >= e->n_sys || b >= e->n_sys || a == b)
-        return fail(OG_ERR_ARG, "bad system indices");
-    if (e->sys_n[a] != e->sys_n[b]) return fail(OG_ERR_ARG, "systems %d and %d differ in size", a, b);
-    if (e->topo_hash[a] != e->topo_hash[b])
-        return fail(OG_ERR_ARG, "systems %d and %d differ in parameters or topology", a, b);
-    if (!(e->temps[a] > 0.0) || !(e->temps[b] > 0.0)) return fail(OG_ERR_STATE, "temperatures not set");
-    const double sa = std::sqrt(e->temps[a] / e->temps[b]);
-    const double sb = std::sqrt(e->temps[b] / e->temps[a]);
-    og_launch_swap(e->pos, e->vel, e->force, e->atom_off[a], e->atom_off[b], e->sys_n[a], sa, sb, e->stream);
+extern "C" int og_swap_pairs(og_engine* e, const int32_t* pairs, int32_t n) {
+    if (!e || n < 0 || (n > 0 && !pairs)) return fail(OG_ERR_ARG, "bad arguments");
+    std::vector<char> seen(e->n_sys, 0);
+    for (int k = 0; k < n; ++k) {
+        const int a = pairs[2 * k], b = pairs[2 * k + 1];
+        if (a < 0 || b < 0 || a >= e->n_sys || b >= e->n_sys || a == b) return fail(OG_ERR_ARG, "bad system indices");
+        if (seen[a] || seen[b]) return fail(OG_ERR_ARG, "system %d is in two pairs", seen[a] ? a : b);
+        seen[a] = seen[b] = 1;
+        if (e->sys_n[a] != e->sys_n[b]) return fail(OG_ERR_ARG, "systems %d and %d differ in size", a, b);
+        if (e->topo_hash[a] != e->topo_hash[b])
+            return fail(OG_ERR_ARG, "systems %d and %d differ in parameters or topology", a, b);
+        if (!(e->temps[a] > 0.0) || !(e->temps[b] > 0.0)) return fail(OG_ERR_STATE, "temperatures not set");
+    }
+    if (n == 0) return OG_OK;
+    for (int k0 = 0; k0 < n; k0 += OG_SWAP_MAX) {
+        og_swap_args p{};
+        const int count = std::min(n - k0, OG_SWAP_MAX);
+        for (int w = 0; w < count; ++w) {
+            const int a = pairs[2 * (k0 + w)], b = pairs[2 * (k0 + w) + 1];
+            p.off_a[w] = e->atom_off[a];
+            p.off_b[w] = e->atom_off[b];
+            p.n[w] = e->sys_n[a];
+            p.scale_a[w] = std::sqrt(e->temps[a] / e->temps[b]);
+            p.scale_b[w] = std::sqrt(e->temps[b] / e->temps[a]);
+        }
+        og_launch_swap(e->pos, e->vel, e->force, p, count, e->stream);
+    }
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(e->stream));
     return OG_OK;
+}
+
+extern "C" int og_swap_systems(og_engine* e, int32_t a, int32_t b) {
+    const int32_t pair[2] = {a, b};
+    return og_swap_pairs(e, pair, 1);
 }
 
 extern "C" int og_get_status(og_engine* e, int32_t* div, int32_t* fails, int32_t* clamped) {

@@ -214,21 +214,21 @@ void og_launch_back(const og_back_args& a, hipStream_t s) {
     hipLaunchKernelGGL(og_k_back, dim3((a.n_atoms + 255) / 256), dim3(256), 0, s, a);
 }
 
-__global__ void og_k_swap(double* pos, double* vel, double* force, int off_a, int off_b, int n,
-                          double sa, double sb) {
+__global__ void og_k_swap(double* pos, double* vel, double* force, og_swap_args p) {
+    const int w = blockIdx.y;
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= 3 * n) return;
-    const size_t ia = 3 * (size_t)off_a + k, ib = 3 * (size_t)off_b + k;
+    if (k >= 3 * p.n[w]) return;
+    const size_t ia = 3 * (size_t)p.off_a[w] + k, ib = 3 * (size_t)p.off_b[w] + k;
     double t = pos[ia]; pos[ia] = pos[ib]; pos[ib] = t;
     t = force[ia]; force[ia] = force[ib]; force[ib] = t;
-    const double va = vel[ib] * sa, vb = vel[ia] * sb;
+    const double va = vel[ib] * p.scale_a[w], vb = vel[ia] * p.scale_b[w];
     vel[ia] = va;
     vel[ib] = vb;
 }
 
-void og_launch_swap(double* pos, double* vel, double* force, int off_a, int off_b, int n,
-                    double scale_a, double scale_b, hipStream_t s) {
+void og_launch_swap(double* pos, double* vel, double* force, const og_swap_args& p, int count, hipStream_t s) {
+    int n = 0;
+    for (int w = 0; w < count; ++w) n = p.n[w] > n ? p.n[w] : n;
     if (n <= 0) return;
-    hipLaunchKernelGGL(og_k_swap, dim3((3 * n + 255) / 256), dim3(256), 0, s, pos, vel, force,
-                       off_a, off_b, n, scale_a, scale_b);
+    hipLaunchKernelGGL(og_k_swap, dim3((3 * n + 255) / 256, count), dim3(256), 0, s, pos, vel, force, p);
 }

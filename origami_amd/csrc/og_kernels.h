@@ -228,8 +228,16 @@ void og_launch_back(const og_back_args& a, hipStream_t s);
 void og_launch_set_u32(uint32_t* p, uint32_t v, hipStream_t s);
 // p[0..n) = 0 with a kernel (no memset node when a caller captures the stream)
 void og_launch_zero_i64(long long* p, long long n, hipStream_t s);
-void og_launch_swap(double* pos, double* vel, double* force, int off_a, int off_b, int n,
-                    double scale_a, double scale_b, hipStream_t s);
+// exchanges of a launch: first atoms, atoms and velocity factors of each pair.
+// One launch and one wait serve a round's exchanges: with a launch and a wait
+// each, the 28 or so of a 64-replica round cost 0.28 ms more (two rounds and
+// their 80 steps with SASA 20.9 -> 20.35 ms).
+#define OG_SWAP_MAX 32
+struct og_swap_args {
+    int off_a[OG_SWAP_MAX], off_b[OG_SWAP_MAX], n[OG_SWAP_MAX];
+    double scale_a[OG_SWAP_MAX], scale_b[OG_SWAP_MAX];
+};
+void og_launch_swap(double* pos, double* vel, double* force, const og_swap_args& p, int count, hipStream_t s);
 
 // ---------------------------------------------------------------------------
 // Device-resident batched L-BFGS (lbfgs.hip); one block per system.

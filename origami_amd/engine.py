@@ -129,6 +129,7 @@ def lib():
         L.og_frames_read.argtypes = [vp, _dp, C.POINTER(C.c_uint32), C.c_int32, C.POINTER(C.c_int32)]
         L.og_set_temperature.argtypes = [vp, C.c_int32, C.c_double]
         L.og_swap_systems.argtypes = [vp, C.c_int32, C.c_int32]
+        L.og_swap_pairs.argtypes = [vp, _ip, C.c_int32]
         L.og_get_status.argtypes = [vp, _ip, _ip, _ip]
         L.og_profile_enable.argtypes = [vp, C.c_int32]
         L.og_profile_read.argtypes = [vp, _dp, C.POINTER(C.c_int64)]
@@ -379,6 +380,11 @@ class Engine:
 
     def swap(self, a, b):
         _check(lib().og_swap_systems(self._h, int(a), int(b)))
+
+    def swap_pairs(self, pairs):
+        """Exchange each (a, b) of pairs, no system in two of them."""
+        p = np.ascontiguousarray(pairs, dtype=np.int32).reshape(-1, 2)
+        _check(lib().og_swap_pairs(self._h, _i(p), len(p)))
 
     def set_tunnel(self, tunnel=None):
         """External cylindrical exit tunnel for the dynamics (an object with
@@ -648,6 +654,7 @@ def run_remd(sys: S.ResolvedSystem, temperatures: Sequence[float], total_time_fs
         eng.run(n, allow_stopped=True)
         stopped = eng.status()["diverged"] != 0
         energies = swap_energies(eng, include_sasa)
+        accepted = []                       # disjoint pairs: exchanged in one launch
         for pair in range(rnd % 2, n_rep - 1, 2):
             a, b = pair, pair + 1
             if stopped[a] or stopped[b]:
@@ -659,8 +666,10 @@ def run_remd(sys: S.ResolvedSystem, temperatures: Sequence[float], total_time_fs
             p_acc = 1.0 if delta >= 0.0 else math.exp(delta)
             if swap_rng.next_f64() < p_acc:
                 accepts[pair] += 1
-                eng.swap(a, b)
+                accepted.append((a, b))
                 energies[a], energies[b] = energies[b], energies[a]
+        if accepted:
+            eng.swap_pairs(accepted)
     final = swap_energies(eng, include_sasa)
     stopped = [bool(x) for x in eng.status()["diverged"]]
     return eng, RemdSummary(n_rep, sys.n_atoms, attempts, accepts, temps, final, stopped)

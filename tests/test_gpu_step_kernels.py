@@ -173,6 +173,31 @@ def test_areas_of_clusters_against_oracle(E, n_atoms, seed):
     assert abs(got - ref) <= 1e-9 * abs(ref) + m * 2.0 ** -32
 
 
+@pytest.mark.parametrize("replicas", [2, 7, 66, 70])
+def test_exchanges_of_a_round_at_once(E, replicas):
+    """Pairs exchanged in one call leave the bits that one call each leaves, up to and past a launch's pairs."""
+    s = S.seeded_chain(3, 2)
+    pairs = [(k, k + 1) for k in range(0, replicas - 1, 2)]
+    state = []
+    for together in (True, False):
+        eng = E.Engine([s] * replicas)
+        rng = np.random.default_rng(1)
+        eng.set_positions(np.concatenate([s.pos + rng.normal(scale=0.02, size=s.pos.shape) for _ in range(replicas)]))
+        eng.set_velocities(rng.normal(scale=0.002, size=(eng.n_atoms, 3)))
+        eng.dynamics_setup(list(300.0 + np.arange(replicas)), dt_fs=0.5, friction_ps_inv=1.0, seed=3)
+        if together:
+            eng.swap_pairs(pairs)
+            with pytest.raises(E.EngineError):
+                eng.swap_pairs([(0, 1), (1, 0)])
+        else:
+            for a, b in pairs:
+                eng.swap(a, b)
+        state.append((eng.positions(), eng.velocities()))
+        eng.run(2)
+        state[-1] += (eng.positions(), eng.velocities())
+    assert all(np.array_equal(x, y) for x, y in zip(*state))
+
+
 def _mix(x):
     m = (1 << 64) - 1
     x = (x + 0x9E3779B97F4A7C15) & m
