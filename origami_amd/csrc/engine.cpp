@@ -1009,6 +1009,7 @@ static int launch_forces(og_engine* e, uint32_t flags, double cutoff_a, double s
         r.charge = e->charge; r.gb = e->gb; r.radii = e->radii; r.clamped = e->clamped;
         r.eacc = e->eacc; r.n_atoms = e->n_atoms;
         r.sflag = e->sflag;
+        r.skip_sys = !forces ? e->eval_skip : nullptr;
         if (sur) { r.sur_mode = sur->mode; r.r_sur = sur->r_sur; r.dev = sur->dev; r.check = check ? 1 : 0; }
         if (wide_e) {
             og_pair_args ae = a;
@@ -1725,21 +1726,24 @@ extern "C" int og_minimize(og_engine* e, const og_minimize_params* prm, og_minim
     int rc = OG_OK;
     auto run = [&]() -> int {
         HIPCHK(hipMemcpy(ip, off.data(), (S + 1) * sizeof(int), hipMemcpyHostToDevice));
-        auto clear = [&](long long* eacc) {
+        auto clear = [&](long long* eacc, const int* skip) {
             og_begin_args bg{};
             bg.facc = e->facc; bg.iacc = e->iacc; bg.n_atoms = e->n_atoms;
             bg.eacc = eacc; bg.sflag = e->sflag; bg.n_sys = S;
+            bg.skip_sys = skip; bg.atom_sys = e->atom_sys;
             og_launch_begin(bg, e->stream);
         };
+        // a system that does not search keeps the integrals and radii of its
+        // last evaluation: og_born_radii returns those of the final positions
         auto energies = [&](bool probes) -> int {
-            clear(e->eacc);
             e->eval_skip = probes ? a.skip : nullptr;
+            clear(e->eacc, e->eval_skip);
             const int r = launch_forces(e, P.flags | OG_ENERGY, P.cutoff_a, P.sasa_gamma_scale, true, -1, false);
             e->eval_skip = nullptr;
             return r;
         };
         auto forces = [&]() -> int {
-            clear(nullptr);
+            clear(nullptr, nullptr);
             if (int r = launch_forces(e, P.flags & ~OG_ENERGY, P.cutoff_a, P.sasa_gamma_scale, false, -1, true)) return r;
             og_back_args b{};
             b.pos = e->pos; b.vel = e->vel; b.force = e->force; b.facc = e->facc; b.mass = e->mass;
@@ -1771,10 +1775,17 @@ extern "C" int og_minimize(og_engine* e, const og_minimize_params* prm, og_minim
             if (int r = forces()) return r;
         for (int step = 0; step < P.max_steps; ++step) {
             og_launch_lbfgs(OG_LB_K_BEGIN, a, step, e->stream);
-            // the first probe goes out with the direction, before the host
-            // knows whether any system searches (nearly always one does; if
-            // none, the probe evaluates nothing): one wait less per iteration
-            if (int r = probe()) return r;
+            // The first probe goes out with the direction, before the host
+            // knows whether any system searches (nearly always one does): one
+            // wait less per iteration.  If none does, it leaves the tile pairs
+            // and radii out and evaluates bonded terms in vain, once per call.
+            // With OG_SASA that would be a whole set of areas (the arrangement
+            // takes no skip list), so the count is read first.
+            if (P.flags & OG_SASA) {
+                if (int r = read_counts(OG_LB_K_COUNT)) return r;
+            } else if (int r = probe()) {
+                return r;
+            }
             if (int r = probes()) return r;
             if (cnt[1] == 0 && cnt[3] == 0) break;          // every system converged or stopped
             if (cnt[1] > 0) {                               // steepest-descent retries

@@ -106,8 +106,8 @@ __device__ __forceinline__ void radii_body(const og_radii_args& a, int i) {
     int sys = 0;
     long long e_fix = 0;
     bool has_e = false;
-    if (i < a.n_atoms) {
-        sys = a.atom_sys[i];
+    if (i < a.n_atoms) sys = a.atom_sys[i];
+    if (i < a.n_atoms && !(a.skip_sys && a.skip_sys[sys])) {
         const bool sur = a.sur_mode && a.sur_mode[sys];
         double R = 0.0;
         if (!sur || a.check) {

@@ -152,7 +152,8 @@ __global__ void __launch_bounds__(256) og_k_begin(og_begin_args a) {
         if (a.xyz) a.pos[k] = a.xyz[k];
         a.facc[k] = 0;
     }
-    for (int k = i; k < a.n_atoms; k += n) a.iacc[k] = 0;
+    for (int k = i; k < a.n_atoms; k += n)
+        if (!(a.skip_sys && a.skip_sys[a.atom_sys[k]])) a.iacc[k] = 0;
     for (int k = i; k < a.n_sys; k += n) {
         a.sflag[k] = 0;
         if (a.clamped) a.clamped[k] = 0;

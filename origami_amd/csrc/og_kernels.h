@@ -96,6 +96,7 @@ struct og_radii_args {
     unsigned* dev;                   // [S] max |R_sur - R_plain| / R_plain (float bits), when check
     int check;                       // plain radii were computed for every system this call
     int* sflag;                      // [S] status bits
+    const int* skip_sys;             // [S] nonzero: the system keeps its radii (may be null)
 };
 
 #define OG_MAX_CL 8                  // atoms per SHAKE cluster (X + up to 7 H)
@@ -143,6 +144,8 @@ struct og_begin_args {
     int* sflag;                      // [S]
     int* clamped;                    // [S] or null
     int n_sys;
+    const int* skip_sys;             // [S] nonzero: the system keeps its descreening integrals (may be null)
+    const int* atom_sys;             // read with skip_sys
 };
 void og_launch_begin(const og_begin_args& a, hipStream_t s);
 
