@@ -155,7 +155,7 @@ __global__ void __launch_bounds__(64 * SUR_DESC_WAVES) og_k_sur_desc(DescArgs a)
     const int a0 = a.tile_atom0[t], cnt = a.tile_cnt[t];
     const bool vi = lane < cnt;
     const int i = a0 + lane;
-    const float edge = bi.w <= SUR_NEAR_A ? SUR_EDGE : 1.0f;   // 1: every pair in FP64
+    const bool wide = !(bi.w <= SUR_NEAR_A);          // every pair in FP64
     double xi = 0.0, yi = 0.0, zi = 0.0;
     if (vi) { xi = a.pos[3 * (size_t)i]; yi = a.pos[3 * (size_t)i + 1]; zi = a.pos[3 * (size_t)i + 2]; }
     // lanes without an atom stay out of every range
@@ -188,7 +188,7 @@ __global__ void __launch_bounds__(64 * SUR_DESC_WAVES) og_k_sur_desc(DescArgs a)
                 const float s = __builtin_amdgcn_sqrtf(fmaf(dx, dx, fmaf(dy, dy, dz * dz))) * (1.0f / 0.375f);
                 k[u] = (int)s;
                 in[u] = s < 32.0f;
-                near[u] = vi && !(s >= 32.0f + edge) && !(fabsf(s - rintf(s)) > edge);
+                near[u] = vi && (wide || (!(s >= 32.0f + SUR_EDGE) && !(fabsf(s - rintf(s)) > SUR_EDGE)));
             }
             if (__any(near[0] | near[1] | near[2] | near[3])) {
 #pragma unroll 1

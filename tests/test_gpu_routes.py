@@ -48,3 +48,22 @@ def test_integrals_after_a_converged_minimisation(E, chains, tol, profiled, mode
     assert np.array_equal(integral, h)
     assert np.array_equal(radii, r)
     assert np.array_equal(clamped, fresh.status()["clamped"])
+
+
+@pytest.mark.parametrize("apart", [1e7, 1e8, 1e12])
+@pytest.mark.parametrize("chains", [[(16, 4)], [(9, 15), (16, 4)]])
+def test_descriptors_of_tiles_that_reach_far(E, chains, apart):
+    """Neighbour counts of tiles whose atoms lie in two groups so far apart
+    that single-precision positions about the tile's centre would be off by
+    more than the range: the counts are exact."""
+    from oracle import surrogate as SO
+    systems = [S.seeded_chain(*c) for c in chains]
+    rng = np.random.default_rng(11)
+    x = rng.uniform(-5.0, 5.0, size=(sum(s.n_atoms for s in systems), 3))
+    x[::3, 0] += apart
+    eng = E.Engine(systems)
+    eng.surrogate_setup(0, seed=1)
+    got = eng.surrogate_descriptors(x)
+    mass = np.concatenate([s.mass for s in systems])
+    rho = np.concatenate([s.gb_rho for s in systems])
+    assert np.array_equal(got.astype(np.float64), SO.descriptors(x, mass, rho, eng.offsets))
