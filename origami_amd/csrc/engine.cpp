@@ -898,6 +898,12 @@ static og_energy64_args energy_args(const og_engine* e, double cutoff_a) {
     return en;
 }
 
+// Force passes (forces only) of the block-per-item form: short lists, plain
+// radii, no per-kernel profile.
+static bool wide_force(const og_engine* e, bool surrogate) {
+    return !surrogate && !e->prof && e->n_tile_pairs <= OG_WIDE_FORCE_MAX;
+}
+
 // The LJ / Coulomb cutoff of a call: cutoff_a under OG_MODE_A (finite and
 // positive), none otherwise (the value is then not used).
 static int check_cutoff(uint32_t flags, double cutoff_a) {
@@ -956,7 +962,7 @@ static int launch_forces(og_engine* e, uint32_t flags, double cutoff_a, double s
     // radii after it, or, on short work lists (a block per work item,
     // pair_wide.hip), with the force pass, which forms the radii itself.
     const bool lean = !energy && !sur && !e->prof;
-    const bool wide = lean && forces && e->n_tile_pairs <= OG_WIDE_FORCE_MAX;
+    const bool wide = !energy && forces && wide_force(e, sur);
     const bool wide_d = wide && e->n_work <= OG_WIDE_DESCREEN_MAX;
     // energies only, the same way
     const bool wide_e = energy && !forces && !sur && !e->prof &&
@@ -1610,9 +1616,25 @@ extern "C" int og_autotune(og_engine* e, uint32_t flags, int32_t* choice, double
         return OG_OK;
     };
     const bool mode_a = flags & OG_MODE_A;
-    // the force pass's tile shape (j tiles per strip; the pass runs one wave
-    // per work item), then the descreening pass's launch width; each
-    // candidate timed twice, the faster kept
+    // the force pass's tile shape (j tiles per strip) on the kernel that
+    // evaluations will launch, then the descreening pass's launch width (a
+    // single candidate on lists short enough for the block-per-item form);
+    // each candidate timed twice, the faster kept
+    const bool wide = wide_force(e, flags & OG_SURROGATE);
+    if (wide) {
+        // that kernel forms the Born radii itself, from the integrals
+        og_launch_zero_acc(e->facc, e->iacc, e->n_atoms, e->stream);
+        og_launch_pair_descreen(pair_args(e, 10.0), mode_a, e->stream);
+    }
+    auto force_pass = [&](const og_pair_args& a) {
+        if (!wide) {
+            og_launch_pair_force(a, mode_a, e->stream);
+            return;
+        }
+        og_radii_args r{};                          // no atoms: the pair blocks alone
+        r.rho = e->rho;
+        og_launch_wide_force(a, r, og_bonded_args{}, mode_a, e->stream);
+    };
     int best_grid = 0, best_strip = e->strip_j;
     float best_force = 1e30f, best_desc = 1e30f;
     for (int sj : {2, 4, 8}) {
@@ -1620,7 +1642,7 @@ extern "C" int og_autotune(og_engine* e, uint32_t flags, int32_t* choice, double
         og_pair_args a = pair_args(e, 10.0);
         for (int rep = 0; rep < 2; ++rep) {
             float ms = 0.0f;
-            if (int rc = timed([&] { og_launch_pair_force(a, mode_a, e->stream); }, ms)) return rc;
+            if (int rc = timed([&] { force_pass(a); }, ms)) return rc;
             if (ms < best_force) { best_force = ms; best_strip = sj; }
         }
     }
@@ -1638,7 +1660,7 @@ extern "C" int og_autotune(og_engine* e, uint32_t flags, int32_t* choice, double
     }
     const float best_pair = best_force + best_desc;
     e->pair_grid = best_grid;
-    int best_sasa = og_sasa_max_blocks(&e->sasa);
+    int best_sasa = 0;                              // not timed: og_set_launch keeps the width
     float best_s = 0.0f;
     if ((flags & OG_SASA) && e->n_sasa_work > 0) {
         og_sasa_set_passes(&e->sasa, 0);

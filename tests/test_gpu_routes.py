@@ -1,5 +1,7 @@
 """What a call leaves and answers whichever kernels it takes: state after a
 minimisation, launch choices, host copies, network inputs, pair-kernel forms."""
+import time
+
 import numpy as np
 import pytest
 
@@ -67,3 +69,36 @@ def test_descriptors_of_tiles_that_reach_far(E, chains, apart):
     mass = np.concatenate([s.mass for s in systems])
     rho = np.concatenate([s.gb_rho for s in systems])
     assert np.array_equal(got.astype(np.float64), SO.descriptors(x, mass, rho, eng.offsets))
+
+
+def test_autotune_without_sasa_leaves_the_sasa_width(E):
+    """A width that was not timed is not chosen: choice 0, which og_set_launch keeps."""
+    systems = [S.seeded_chain(3, 10)] * 4
+    eng = E.Engine(systems)
+    ch = eng.autotune()
+    assert ch["sasa_blocks"] == 0 and ch["pair_blocks"] > 0
+    eng.set_launch(pair_blocks=ch["pair_blocks"], sasa_blocks=ch["sasa_blocks"])
+    x = _jittered(systems, 4)
+    assert np.array_equal(eng.total_force(x, include_sasa=True), E.Engine(systems).total_force(x, include_sasa=True))
+    assert eng.autotune(include_sasa=True)["sasa_blocks"] > 0
+
+
+def test_autotune_times_the_force_pass_that_runs(E):
+    """The strip length it keeps is the fastest of the three, within a few per
+    cent, in the steps that follow (64 chains of 20 residues, whose force pass
+    takes a block per item: 8 j tiles are a tenth faster than 2 or 4)."""
+    systems = [S.seeded_chain(4, 20)] * 64
+    eng = E.Engine(systems)
+    eng.set_positions(_jittered(systems, 2))
+    eng.set_velocities(np.zeros((eng.n_atoms, 3)))
+    kept = eng.autotune()["strip_tiles"]
+    eng.dynamics_setup([300.0] * 64, dt_fs=1e-3, seed=1)
+    best = {n: np.inf for n in (2, 4, 8)}
+    for _ in range(8):
+        for n in best:
+            eng.strip_tiles(n)
+            eng.run(5)
+            t = time.perf_counter()
+            eng.run(40)
+            best[n] = min(best[n], time.perf_counter() - t)
+    assert best[kept] <= 1.05 * min(best.values()), (kept, best)
