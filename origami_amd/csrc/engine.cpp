@@ -25,7 +25,17 @@
 // og_run's default: captured steps below this many atoms
 #define OG_SPLIT_MAX_TILES 4           // systems up to 256 atoms: off-diagonal tile pairs in halves
 #define OG_STRIP_DEFAULT 4             // j tiles per force strip until the autotuner picks
-#define OG_STAGE_MAX_ATOMS 8192        // host copies of up to so many atoms go through pinned staging
+// Pinned staging.  An evaluation reads its coordinates from it and leaves its
+// forces there up to OG_STAGE_MAX_ATOMS atoms (us per force call, staged
+// against copies: 39.7 and 68.0 at 340 atoms, 91 and 125 at 4 915, 136 and 158
+// at 7 830; still 132 and 151 at 9 830 and 1 216 and 1 244 at 157 280, so the
+// line is where the memory pinned for every engine's life ends, 192 KB, not a
+// crossing).  A copy alone goes through it up to OG_STAGE_COPY_BYTES: the
+// runtime's own copy of pageable memory takes 15-21 us in and 23-28 out up to
+// 16 KB, against 15 both ways staged; above, 10.7 at 17 KB and 15 at 118 KB,
+// against 15 and 18 staged (17 for the first thousand copies of a process).
+#define OG_STAGE_MAX_ATOMS 8192
+#define OG_STAGE_COPY_BYTES 16384
 #define OG_SR_DOTS 960                 // Shrake-Rupley dots per atom (SHRAKE_RUPLEY_DOTS, sasa.rs:27)
 #define OG_PERSIST_MAX_TILES 8         // persistent replica steps: systems of up to 512 atoms
 #define OG_PERSIST_CHUNK 512           // steps per persistent launch
@@ -816,10 +826,14 @@ static void publish_add(og_publish_args& p, int q, const void* src, void* dst, s
     p.n[q] = (int)(bytes / 4);
 }
 
-// Device words to the caller's buffer, through the staging buffer where they
-// fit; returns with the stream idle.
+// Copies that go through the staging buffer.
+static bool staged_copy(const og_engine* e, size_t bytes) {
+    return bytes <= OG_STAGE_COPY_BYTES && bytes <= e->stage_bytes;
+}
+
+// Device words to the caller's buffer; returns with the stream idle.
 static int fetch(og_engine* e, void* host, const void* dev, size_t bytes) {
-    if (bytes > e->stage_bytes) {
+    if (!staged_copy(e, bytes)) {
         HIPCHK(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, e->stream));
         HIPCHK(hipStreamSynchronize(e->stream));
         return OG_OK;
@@ -839,7 +853,7 @@ static int copy_state(og_engine* e, double* dev, const double* host, bool to_dev
     if (!to_dev) return fetch(e, (void*)host, dev, bytes);
     const size_t bad = first_nonfinite(host, n);
     if (bad < n) return fail(OG_ERR_ARG, "non-finite input at %zu", bad);
-    if (bytes <= e->stage_bytes) {
+    if (staged_copy(e, bytes)) {
         std::memcpy(e->stage_x, host, bytes);
         og_publish_args p{};
         publish_add(p, 0, e->stage_x, dev, bytes);

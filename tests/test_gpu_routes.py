@@ -5,6 +5,7 @@ import time
 import numpy as np
 import pytest
 
+from oracle import oracle as O
 from origami_amd import system as S
 
 pytestmark = pytest.mark.gpu
@@ -102,3 +103,38 @@ def test_autotune_times_the_force_pass_that_runs(E):
             eng.run(40)
             best[n] = min(best[n], time.perf_counter() - t)
     assert best[kept] <= 1.05 * min(best.values()), (kept, best)
+
+
+@pytest.mark.parametrize("residues", [1, 42, 43, 44, 300, 520])
+def test_state_copies_of_every_size(E, residues):
+    """Positions and velocities come back as they were set and forces as the
+    call returned them, on both sides of the sizes where copies change route
+    (16 KB: 682 atoms; 8 192 atoms)."""
+    s = S.seeded_chain(5, residues)
+    eng = E.Engine([s])
+    rng = np.random.default_rng(residues)
+    x, v = s.pos + rng.normal(scale=0.02, size=s.pos.shape), rng.normal(size=s.pos.shape)
+    eng.set_velocities(v)
+    eng.set_positions(x)
+    assert np.array_equal(eng.positions(), x) and np.array_equal(eng.velocities(), v)
+    f = eng.total_force()
+    assert np.array_equal(eng.forces(), f)
+    assert np.array_equal(E.Engine([s]).total_force(x), f)
+    x[-1, 2] = np.nan
+    with pytest.raises(E.EngineError, match="non-finite input at %d" % (x.size - 1)):
+        eng.set_positions(x)
+
+
+@pytest.mark.parametrize("steps", [3, 1024, 1025])
+def test_kinetic_energies_of_every_length(E, steps):
+    """Recorded kinetic energies on both sides of the copy's route, against those of the call without allocation."""
+    s = S.seeded_chain(3, 2)
+    out = []
+    for noalloc in (False, True):
+        eng = E.Engine([s, s])
+        eng.set_velocities(np.random.default_rng(1).normal(scale=0.002, size=(eng.n_atoms, 3)))
+        eng.dynamics_setup([300.0, 310.0], dt_fs=0.1, friction_ps_inv=1.0, seed=3)
+        out.append(eng.run(steps, record_ke=True, noalloc=noalloc))
+    assert np.all(out[0] > 0.0) and np.array_equal(*out)
+    ref = O.Oracle(s).kinetic_energy(eng.split(eng.velocities())[1])
+    assert abs(out[0][-1][1] - ref) <= s.n_atoms * 2.0 ** -33 + 1e-14 * s.n_atoms * ref
