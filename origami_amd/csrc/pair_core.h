@@ -1,7 +1,10 @@
 // Per-pair arithmetic and tile loads of the all-pairs kernels, shared by the
 // wave-per-item kernels (pair_kernels.hip) and the block-per-item kernels for
 // small work lists (pair_wide.hip).  Both forms evaluate a pair with the same
-// products in the same order, so their results agree bit for bit.
+// products in the same order, so their results agree bit for bit.  Which
+// product is fused into which sum is written out and contraction is off in the
+// functions below that form pair terms: left to the compiler it depends on the
+// loop they are inlined into.
 //
 //   descreening   energy/src/gb.rs:271-283 (pair), :347-369 (h)
 //   LJ + Coulomb  energy/src/forces_nonbonded.rs:196-232
@@ -60,6 +63,7 @@ __device__ __forceinline__ float swap32(float v) { return __shfl_xor(v, 32, 64);
 // 1/U^2 - 1/L^2 = -(1/L - 1/U)(U+L)/(LU),  ln(L/U) = ln(L^2/(LU)), with
 // L = max(r - S, rho~) covering both the overlapping and the separate case.
 __device__ __forceinline__ float descreen_h(float r2, float inv_r, float rt, float S, float S2) {
+#pragma clang fp contract(off)
     // r = r2 * inv_r is not rounded on its own (left to the compiler, some
     // loops did and some did not)
     const float U = fmaf(r2, inv_r, S);
@@ -95,6 +99,7 @@ template <bool MODEA, int PART>
 __device__ __forceinline__ void descreen_tile_far(const og_pair_args& a, const LaneData& di,
                                                   const float4* P, const float4* Q, int lane,
                                                   float& acc_i, float& acc_j) {
+#pragma clang fp contract(off)
     float gj = 0.0f;
     const float Si2 = di.gb.y * di.gb.y;
     const float ci3 = (-1.0f / 3.0f) * Si2 * di.gb.y;
@@ -105,15 +110,15 @@ __device__ __forceinline__ void descreen_tile_far(const og_pair_args& a, const L
         const float inv_r = __builtin_amdgcn_rsqf(r2);
         const float inv_r2 = inv_r * inv_r;
         const float inv_r4 = inv_r2 * inv_r2;
-        const float hij = (qj.z * inv_r4) * series(qj.y * inv_r2);
-        const float hji = (ci3 * inv_r4) * series(Si2 * inv_r2);
+        const float ki = qj.z * inv_r4, si = series(qj.y * inv_r2);
+        const float kj = ci3 * inv_r4, sj = series(Si2 * inv_r2);
         if (MODEA) {
             const bool ok = r2 <= a.rc2_ds;
-            acc_i += ok ? hij : 0.0f;
-            gj += ok ? hji : 0.0f;
+            acc_i += ok ? ki * si : 0.0f;
+            gj += ok ? kj * sj : 0.0f;
         } else {
-            acc_i += hij;
-            gj += hji;
+            acc_i = fmaf(ki, si, acc_i);
+            gj = fmaf(kj, sj, gj);
         }
         gj = rot(gj);                  // after step 63 this is the way home
     };
@@ -178,6 +183,7 @@ template <bool MODEA, bool MASKED>
 __device__ __forceinline__ float tile_coef(const og_pair_args& a, const LaneData& di, float qki, float qj, float sej,
                                            float rmj, float se14j, float rm14j, float Rj, float iRj, bool excl,
                                            bool one4, float dx, float dy, float dz) {
+#pragma clang fp contract(off)
     const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
     const float inv_r = __builtin_amdgcn_rsqf(r2);
     const float inv_r2 = inv_r * inv_r;
@@ -191,12 +197,11 @@ __device__ __forceinline__ float tile_coef(const og_pair_args& a, const LaneData
     }
     const float t2 = rmin * rmin * inv_r2;
     const float t6 = t2 * t2 * t2;
-    const float lj = eij * inv_r2 * (t6 - t6 * t6);
     const float qq = di.q * qj;
     float coul;
-    if (MODEA) coul = -qq * (inv_r2 * inv_r - a.inv_rc3);
+    if (MODEA) coul = -qq * fmaf(inv_r2, inv_r, -a.inv_rc3);
     else coul = -qq * inv_r2 * inv_r;
-    float cnb = lj + coul;
+    float cnb = fmaf(eij * inv_r2, fmaf(-t6, t6, t6), coul);
     if (MODEA) cnb = (r2 <= a.rc2_nb) ? cnb : 0.0f;
     if (MASKED) cnb = excl ? 0.0f : cnb;
     // GB pair (frozen radii): f^2 = r^2 + R_i R_j exp(-r^2 / (4 R_i R_j))
@@ -205,9 +210,8 @@ __device__ __forceinline__ float tile_coef(const og_pair_args& a, const LaneData
     const float f2 = fmaf(Rp, e, r2);
     const float inv_f = __builtin_amdgcn_rsqf(f2);
     const float qgb = qki * qj;
-    float gbc = qgb * fmaf(-0.25f, e, 1.0f) * (inv_f * inv_f * inv_f);
-    if (MODEA) gbc = (r2 <= a.rc2_gb) ? gbc : 0.0f;
-    const float c = cnb + gbc;
+    const float k = qgb * fmaf(-0.25f, e, 1.0f), f3 = inv_f * inv_f * inv_f;
+    const float c = MODEA ? cnb + (r2 <= a.rc2_gb ? k * f3 : 0.0f) : fmaf(k, f3, cnb);
     return r2 >= 1e-18f ? c : 0.0f;
 }
 
@@ -237,6 +241,7 @@ __device__ __forceinline__ StripAtom strip_atom(const LaneData& d) {
 template <bool MODEA, bool FAR = false>
 __device__ __forceinline__ float strip_coef(const og_pair_args& a, const StripAtom& I, float4 pj, float4 qj,
                                             float dx, float dy, float dz) {
+#pragma clang fp contract(off)
     const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
     const float inv_r = __builtin_amdgcn_rsqf(r2);
     const float inv_r2 = inv_r * inv_r;
@@ -245,22 +250,24 @@ __device__ __forceinline__ float strip_coef(const og_pair_args& a, const StripAt
     const float t6 = t2 * t2 * t2;
     const float lj = (I.se * qj.x) * inv_r2 * fmaf(-t6, t6, t6);
     const float qq = I.q * pj.w;
-    float gb;
+    float k, f3;
     if (FAR) {
-        gb = kGbK * (inv_r * inv_r * inv_r);
+        k = kGbK;
+        f3 = inv_r * inv_r * inv_r;
     } else {
         const float e = __builtin_amdgcn_exp2f(-r2 * (I.gw * qj.w));
         const float f2 = fmaf(I.R * qj.z, e, r2);
         const float inv_f = __builtin_amdgcn_rsqf(f2);
-        gb = fmaf(-0.25f * kGbK, e, kGbK) * (inv_f * inv_f * inv_f);
+        k = fmaf(-0.25f * kGbK, e, kGbK);
+        f3 = inv_f * inv_f * inv_f;
     }
     if (MODEA) {
-        float cnb = fmaf(-qq, inv_r2 * inv_r - a.inv_rc3, lj);
+        float cnb = fmaf(-qq, fmaf(inv_r2, inv_r, -a.inv_rc3), lj);
         cnb = (r2 <= a.rc2_nb) ? cnb : 0.0f;
-        const float gbc = (r2 <= a.rc2_gb) ? qq * gb : 0.0f;
+        const float gbc = (r2 <= a.rc2_gb) ? qq * (k * f3) : 0.0f;
         return cnb + gbc;
     }
-    return fmaf(qq, gb - inv_r2 * inv_r, lj);
+    return fmaf(qq, fmaf(k, f3, -(inv_r2 * inv_r)), lj);
 }
 
 // Bounds of a strip's two i tiles about the origin (the first one's first
