@@ -138,3 +138,35 @@ def test_kinetic_energies_of_every_length(E, steps):
     assert np.all(out[0] > 0.0) and np.array_equal(*out)
     ref = O.Oracle(s).kinetic_energy(eng.split(eng.velocities())[1])
     assert abs(out[0][-1][1] - ref) <= s.n_atoms * 2.0 ** -33 + 1e-14 * s.n_atoms * ref
+
+
+# (systems, strip length): one chain of 4 915 atoms, whose strips are too many
+# to be split over their i and j sides (two coefficient buffers, one barrier a
+# j tile; with 5 and 8 j tiles a second group of them), and lists of more work
+# items than the block-per-item descreening takes with a force pass of that
+# form (systems of 3 to 5, 8 or 9, and 20 to 22 tiles)
+@pytest.mark.parametrize("mode_a", [False, True])
+@pytest.mark.parametrize("chains, strip", [([(5, 300)], 1), ([(5, 300)], 4), ([(5, 300)], 5), ([(5, 300)], 8),
+                                           ([(40 + k, 14) for k in range(70)], 4),
+                                           ([(40 + k, 30) for k in range(16)], 8),
+                                           ([(40 + k, 80) for k in range(9)], 8)])
+def test_pair_forms_of_long_lists_agree(E, chains, strip, mode_a):
+    """Block-per-item and one-wave pair kernels (the profiled path runs the
+    latter) leave the same bits where strips are evaluated whole and where only
+    the force pass has the block form."""
+    systems = [S.seeded_chain(*c) for c in chains]
+    x = _jittered(systems, 6)
+    out = []
+    for profiled in (False, True):
+        eng = E.Engine(systems)
+        assert eng.info()["tile_pairs"] <= 4864
+        eng.strip_tiles(strip)
+        eng.profile(profiled)
+        f = eng.total_force(x, mode_a=mode_a)
+        r, h = eng.born_radii()
+        eng.set_velocities(np.zeros_like(x))
+        eng.dynamics_setup([300.0] * len(systems), dt_fs=0.01, seed=9, mode_a=mode_a)
+        eng.run(3)
+        out.append((f, r, h, eng.positions(), eng.velocities(), eng.status()["clamped"]))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
