@@ -158,18 +158,24 @@ OG_HD int intersect_count_fast(const Cap& c1, const Cap& c2) {
 #define SA_COV_SLACK 2e-5
 #define SA_COV_FULL 100.0f
 
+// The device's reciprocal and square root are off by up to a unit in the last
+// place; host builds may set relative errors in their place.
+#ifndef OG_COVER_RCP_ERR
+#define OG_COVER_RCP_ERR 0.0f
+#define OG_COVER_SQRT_ERR 0.0f
+#endif
 OG_HD inline float cover_rcp(float x) {
 #ifdef __HIP_DEVICE_COMPILE__
     return __builtin_amdgcn_rcpf(x);
 #else
-    return 1.0f / x;
+    return 1.0f / x * (1.0f + OG_COVER_RCP_ERR);
 #endif
 }
 OG_HD inline float cover_sqrt(float x) {
 #ifdef __HIP_DEVICE_COMPILE__
     return __builtin_amdgcn_sqrtf(x);
 #else
-    return sqrtf(x);
+    return sqrtf(x) * (1.0f + OG_COVER_SQRT_ERR);
 #endif
 }
 // arc cosine, Abramowitz and Stegun 4.4.46 (2e-8 before rounding)
