@@ -306,7 +306,7 @@ def main():
                     help="short workload for hardware-counter runs: a 512 MiB device copy (the "
                          "calibration kernel) and three force evaluations of the 64-chain batch")
     ap.add_argument("--step-mode", choices=["auto", "graph", "direct", "persistent"], default="auto",
-                    help="how og_run issues a step: by batch size (auto), captured graphs, direct "
+                    help="how og_run issues a step: the engine's choice (auto), captured graphs, direct "
                          "launches, or the persistent replica-step kernel")
     ap.add_argument("--no-fixtures", action="store_true",
                     help="skip the timing of the reference's own PDB systems (1UAO, 1L2Y, 2F4K)")
@@ -341,8 +341,8 @@ def main():
         systems, temps = build_config3(n_rep=args.replicas)
         include_sasa = False
         workload = ("REMD batch: %d replicas of a seeded 10-residue chain, 280-395 K geometric "
-                    "ladder; all-pairs GB + LJ + Coulomb; BAOAB dt 2 fs + SHAKE; one captured "
-                    "graph per step for all replicas" % args.replicas)
+                    "ladder; all-pairs GB + LJ + Coulomb; BAOAB dt 2 fs + SHAKE; one set of "
+                    "launches per step for all replicas" % args.replicas)
     log("built %d systems in %.1f s" % (len(systems), time.time() - t0))
     eng = E.Engine(systems)
     info = eng.info()
@@ -364,7 +364,7 @@ def main():
     log("autotune:", tune)
     eng.use_graphs({"auto": None, "graph": True, "direct": False, "persistent": "persistent"}[args.step_mode])
     eng.run(args.warmup)
-    # timed run: no per-kernel events (captured graphs below 20 000 atoms)
+    # timed run: no per-kernel events (direct launches unless --step-mode asks otherwise)
     t0 = time.perf_counter()
     eng.run(args.steps)
     wall = time.perf_counter() - t0

@@ -243,12 +243,13 @@ int og_frames_read(og_engine* e, double* xyz, uint32_t* steps, int32_t max_frame
 
 /* How og_run issues a step (no counterpart in origami; its step loop is
  * langevin.rs:195-367, run per replica by remd.rs:286):
- *   0 direct launches (five per step on small batches);
+ *   0 direct launches (four per step on small batches);
  *   1 one captured hipGraph per BAOAB step (all systems, every launch of the
  *     step), replayed, when profiling is off and no per-step kinetic energy
  *     is requested;
  *   2 the engine's choice (the default): direct launches, measured fastest
- *     on the REMD batch and the 64-chain batch;
+ *     without SASA; with SASA captured steps are up to 5 % faster on small
+ *     batches and even on the 64-chain batch;
  *   3 persistent replica steps: one launch per run of steps, one block of
  *     512 threads per system, for batches of systems of up to 512 atoms
  *     without SASA or the surrogate (else direct launches).
@@ -298,7 +299,10 @@ int og_swap_pairs(og_engine* e, const int32_t* pairs, int32_t n);
 int og_get_status(og_engine* e, int32_t* diverged, int32_t* shake_failures, int32_t* clamped);
 
 /* Kernel timing: when enabled, every launch is bracketed by HIP events on
- * the engine's stream.  og_profile_read returns, per kernel class
+ * the engine's stream.  So that each class has launches of its own, passes run
+ * one after another in their wave-per-item form; without profiling short lists
+ * take shared launches and the block-per-item form (the same bits, other
+ * times), and SASA runs beside the pair kernels.  og_profile_read returns, per kernel class
  * (OG_K_*), total milliseconds and launch counts since the last reset. */
 enum og_kernel_class {
     OG_K_CLUSTER = 0, OG_K_BONDED, OG_K_DESCREEN, OG_K_RADII, OG_K_FORCE, OG_K_SASA, OG_K_BACK,

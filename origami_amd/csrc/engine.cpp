@@ -22,7 +22,6 @@
 #include "og_sasa.h"
 #include "og_sur.h"
 
-// og_run's default: captured steps below this many atoms
 #define OG_SPLIT_MAX_TILES 4           // systems up to 256 atoms: off-diagonal tile pairs in halves
 #define OG_STRIP_DEFAULT 4             // j tiles per force strip until the autotuner picks
 // Pinned staging.  An evaluation reads its coordinates from it and leaves its
@@ -1358,11 +1357,11 @@ static int run_steps(og_engine* e, int32_t n_steps, long long* ke_dev, bool allo
     og_sur* sur = (p.flags & OG_SURROGATE) ? e->sur : nullptr;
     // Persistent replica steps (og_use_graphs 3): one launch runs many whole
     // steps, a block per system (batches of small systems without SASA or the
-    // surrogate), chunked at frame boundaries.  Measured on the REMD batch (8
-    // and 64 replicas of 171 atoms): 56 us per step against 36.5 us with
-    // direct launches and 39.4 us with captured steps: one CU's four SIMDs
-    // take a replica's 18 tile-pair items in turn, where the launches spread
-    // them over the chip.
+    // surrogate), chunked at frame boundaries.  us per step of 8 and 64
+    // replicas of 171 atoms: 51 and 51, against 25.3 and 35.3 with direct
+    // launches and 26.7 and 39.0 with captured steps: one CU's four SIMDs take
+    // a replica's tile-pair items in turn, where the launches spread them over
+    // the chip.
     const bool persist_ok = !(p.flags & (OG_SASA | OG_SURROGATE)) && !e->prof &&
                             e->max_sys_tiles <= OG_PERSIST_MAX_TILES && e->n_clusters_small == e->n_clusters &&
                             n_steps > 0;
@@ -1412,9 +1411,11 @@ static int run_steps(og_engine* e, int32_t n_steps, long long* ke_dev, bool allo
     // Captured steps (og_use_graphs 1): every launch of one BAOAB step
     // (cluster B-A-SHAKE-O-A, forces, final kick) is recorded once into a
     // hipGraph and replayed; the step counter lives in device memory so one
-    // graph serves every step.  Direct launches measured faster on both the
-    // REMD batch (36.5 against 39.4 us per step) and the 64-chain batch, so
-    // they are the engine's choice.
+    // graph serves every step.  Direct launches are the engine's choice: 25.3
+    // against 26.7 us per step on 8 replicas of 171 atoms, 30.2 against 34.4 on
+    // a chain of 1 425, 569 against 571 on 64 chains (160 000 atoms).  With
+    // SASA captured steps take 110.8 against 114.8 on the replicas and 106.7
+    // against 111.5 on the chain, and the same on the 64 chains (1 706 and 1 705).
     const bool want = e->graph_mode == 1;
     const bool graphs = allow_graphs && want && !e->prof && !ke_dev && n_steps >= 2;
     if (graphs) {
@@ -1590,13 +1591,6 @@ extern "C" int og_use_graphs(og_engine* e, int32_t on) {
     return OG_OK;
 }
 
-// Autotuner: times the candidate launch widths of the all-pairs kernels and
-// of the SASA arrangement kernel on the engine's current positions and keeps
-// the fastest.  Candidates: pair kernels 2..32 blocks of 256 threads per CU;
-// SASA 2..8 blocks of 2 waves per CU.  With SASA the widths are timed on the
-// whole force evaluation, SASA on its stream beside the pair chain, since the
-// best split of the CUs between the two depends on both: first the SASA width
-// with the pair width that is fastest alone, then the pair width again.
 extern "C" int og_set_launch(og_engine* e, int32_t pair_blocks, int32_t sasa_blocks, int32_t sasa_passes) {
     if (!e) return fail(OG_ERR_ARG, "engine is NULL");
     if (sasa_passes < 0 || sasa_passes > 2) return fail(OG_ERR_ARG, "sasa_passes must be 0, 1 or 2");
@@ -1607,6 +1601,14 @@ extern "C" int og_set_launch(og_engine* e, int32_t pair_blocks, int32_t sasa_blo
     return OG_OK;
 }
 
+// Autotuner: times the force pass's strip lengths, the candidate launch widths
+// of the descreening pass and those of the SASA arrangement kernel on the
+// engine's current positions and keeps the fastest.  Candidates: strips of 2, 4
+// and 8 j tiles; descreening 2..32 blocks of 256 threads per CU; SASA 2..8
+// blocks of 2 waves per CU.  With SASA the widths are timed on the
+// whole force evaluation, SASA on its stream beside the pair chain, since the
+// best split of the CUs between the two depends on both: first the SASA width
+// with the pair width that is fastest alone, then the pair width again.
 extern "C" int og_autotune(og_engine* e, uint32_t flags, int32_t* choice, double* best_ms) {
     if (!e) return fail(OG_ERR_ARG, "engine is NULL");
     if ((flags & OG_SURROGATE) && !(e->sur && e->sur->enabled))

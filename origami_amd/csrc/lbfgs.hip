@@ -442,7 +442,10 @@ void og_launch_lbfgs(int phase, const og_lbfgs_args& a, int step, hipStream_t s)
         hipLaunchKernelGGL(og_k_lb_init, dim3(1), dim3(kThreads), 0, s, a);
         break;
     case OG_LB_K_BEGIN:
-        // in registers up to 20 values per thread (1 706 atoms)
+        // in registers up to 20 values per thread (1 706 atoms); us per
+        // iteration with 8 values, 20 and in chunks: 94, 113 and 121 at 83
+        // atoms, 116, 132 and 140 at 659; 20 and chunks: 134 and 149 at 959,
+        // 154 and 195 at 1 641
         if (a.max_n3 <= 8 * kThreads) hipLaunchKernelGGL(og_k_lb_begin<8>, dim3(a.n_sys), dim3(kThreads), 0, s, a, step);
         else if (a.max_n3 <= 20 * kThreads)
             hipLaunchKernelGGL(og_k_lb_begin<20>, dim3(a.n_sys), dim3(kThreads), 0, s, a, step);

@@ -202,7 +202,13 @@ void og_launch_bonded_terms(const og_bonded_args& a, hipStream_t s);
 // per item -> a block per item):
 //   force, up to 19 tile pairs per CU: 33 -> 25 at 6 tile pairs, 82 -> 54 at
 //   210, 83 -> 55 at 861, 100 -> 91 at 4 274; 103 -> 108 at 6 007, where the
-//   one-wave items fill the chip and the block form's LDS traffic costs more
+//   one-wave items fill the chip and the block form's LDS traffic costs more.
+//   Under cutoffs, which leave both forms most items to skip, it gains more
+//   (67 -> 48 at 1 711, 98 -> 73 at 4 851).  Beside the SASA arrangement the
+//   form fits no CU that holds three of its blocks (75 808 + 3 x 31 040 bytes
+//   of LDS), so it gains nothing there: steps within 3 % either way from 1 to
+//   4 851 tile pairs (207 -> 216 at worst, 1 chain of 6 230 atoms), force
+//   calls 186 -> 203 at worst (1 chain of 4 915 atoms)
 //   descreening, up to 2 items per CU: 69 -> 63 at 21 items, 82 -> 78 at 210,
 //   83 -> 81 at 496; 83 -> 86 at 861
 //   strips split into their i sides and j sides (pairs evaluated twice), up

@@ -441,9 +441,8 @@ __device__ __forceinline__ void wide_force_strip(WideForce& L, const og_pair_arg
 
 }  // namespace
 
-// blocks [0, n_work): descreening items; the rest: bonded terms
-// (four waves per SIMD, so that two blocks share a CU: left to itself the
-// compiler spends 149-164 registers on the bonded and noise code)
+// blocks [0, n_work): descreening items; the rest: bonded terms, whose
+// registers (164, with energies 182) leave one block a CU
 template <bool MODEA, bool ENERGY>
 __global__ void __launch_bounds__(OG_WIDE_THREADS) og_k_wide_descreen(og_pair_args a, og_bonded_args b) {
     __shared__ WideDescreen L;
@@ -458,6 +457,8 @@ __global__ void __launch_bounds__(OG_WIDE_THREADS) og_k_wide_descreen(og_pair_ar
 
 // blocks: strips (ns blocks each), force items, then nr blocks of radii, the
 // rest the gather
+// (four waves per SIMD, so that two blocks share a CU: left to itself the
+// compiler spends up to 149 registers, with the noise code)
 template <bool MODEA, bool NOISE>
 __global__ void __launch_bounds__(OG_WIDE_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 og_k_wide_force(og_pair_args a, og_radii_args r, og_bonded_args b, int ns, int nr) {

@@ -719,7 +719,6 @@ int refresh_copies(og_sur* s) {
     return hipGetLastError() == hipSuccess ? 0 : fail("kernel launch failed");
 }
 
-// forward + backward + weight gradients on the batch already in Xb/XbT/tb
 // forward, backward and weight gradients of B rows of (X, t); the gradient
 // goes to grad, or (null) one Adam step is taken
 int batch_gradient(og_sur* s, const unsigned short* X, const float* t, long long n_rows, unsigned long long seed,
